@@ -574,20 +574,53 @@ void gs7(const Dim &d, const T *ac, const T *cc, const T *fc, T *x,
 // is pair m-1's second point (the previous lane, or lane 63 of the previous
 // segment for lane 0); its east neighbour is pair m+1's first point.
 constexpr int ROWS_MAXN = 128 * 4 + 1;
-// A point's operands for its update (gsd.cc:160-211), as loaded: the
-// couplings and neighbour values of its own plane (all but the two in-row
-// neighbours), of the plane above (u) and of the plane below (d).
+// Two or four consecutive elements by one load each (two for four doubles),
+// aligned to the element only.
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));
+__device__ __forceinline__ void ldn(const float *p, float (&v)[2]) {
+  const f32x2u t = *(const f32x2u *)p;
+  v[0] = t.x, v[1] = t.y;
+}
+__device__ __forceinline__ void ldn(const double *p, double (&v)[2]) {
+  const f64x2u t = *(const f64x2u *)p;
+  v[0] = t.x, v[1] = t.y;
+}
+__device__ __forceinline__ void ldn(const float *p, float (&v)[4]) {
+  const f32x4u t = *(const f32x4u *)p;
+  v[0] = t.x, v[1] = t.y, v[2] = t.z, v[3] = t.w;
+}
+__device__ __forceinline__ void ldn(const double *p, double (&v)[4]) {
+  const f64x2u t = *(const f64x2u *)p, u = *(const f64x2u *)(p + 2);
+  v[0] = t.x, v[1] = t.y, v[2] = u.x, v[3] = u.y;
+}
+// Element di of a row whose first element is base, for the lane `off` bytes
+// into the row: the base is the same for the whole wavefront (a scalar
+// address) and the lane part stays one 32-bit offset for every array.
+template <class T>
+__device__ __forceinline__ const T *lane_at(const T *base, int di,
+                                            unsigned off) {
+  return (const T *)((const char *)(base + di) + off);
+}
+
+// The operands of a pair of i-adjacent points (i0, i0 + 1) for their updates
+// (gsd.cc:160-211), as loaded.  Every coupling comes for both points with
+// one two-element load and every neighbouring row of x with one four-element
+// load (i0 - 1 .. i0 + 2): 37 loads of a pair against 106 scalar ones.
 template <class T>
 struct G27Raw {
-  T cN[2], xN[2];  // oN(p) x(p+sy), oN(p-sy) x(p-sy)
-  T cE, cW;        // oE(p), oE(p-1): the in-row couplings
-  T c[4], xv[4];   // the other four in-plane terms
-  T cu[9], xu[9], cd[9], xd[9];
-  T f, oC, cc;
+  T cN[2], cS[2];      // oN(p), oN(p - sy)
+  T cE[2], cW;         // oE(p) of both points, oE(p - 1) of the first
+  T c[4][2];           // oNE(p), oNW(p), oNW(p + 1 - sy), oNE(p - 1 - sy)
+  T cu[9][2], cd[9][2];
+  T xN[4], xS[4];      // x of rows j + 1, j - 1 in the own plane
+  T xu[3][4], xd[3][4];  // rows j, j + 1, j - 1 of the planes above, below
+  T f[2], oC[2], cc[2];
 };
 
-// The terms that do not involve the two in-row neighbours, summed in the
-// reference's order as far as they go.
+// The terms of one point that do not involve the two in-row neighbours,
+// summed in the reference's order as far as they go.
 template <class T>
 struct G27Part {
   T a;             // oN(p) x(p+sy) + oN(p-sy) x(p-sy): the first two terms
@@ -600,18 +633,20 @@ struct G27Part {
 // The neighbour rows come from four arrays by their offset (dy, dz) from
 // this row: xO (dy, dz even: the row itself), xN (dy odd, dz = 0), xU
 // (dy = 0, dz odd), xNU (dy and dz odd); the new values go to xW.  A
-// sweep kept in one array passes it for all five.
+// sweep kept in one array passes it for all five.  The loads of the last
+// pair of the grid's last row reach one element past the end of x, whose
+// value no sum uses: every x array has that element (allocations are
+// padded).
 template <class T, int ADJ, int PPL>
 __device__ __forceinline__ void gs27_row(
     int nx, int ny, int nz, const T *__restrict__ ac, const T *__restrict__ cc,
     const T *__restrict__ fc, int pz, int py, int j, int k, int zmask,
     const T *xO, const T *xN, const T *xU, const T *xNU, T *xW) {
   const int lane = threadIdx.x & 63;
-  const size_t n = (size_t)nx * ny * nz, sy = nx, sz = (size_t)nx * ny;
-  const T *oE = ac + n, *oN = ac + 2 * n, *uC = ac + 3 * n, *oNE = ac + 4 * n,
-          *oNW = ac + 5 * n, *uE = ac + 6 * n, *uW = ac + 7 * n,
-          *uN = ac + 8 * n, *uS = ac + 9 * n, *uNE = ac + 10 * n,
-          *uNW = ac + 11 * n, *uSE = ac + 12 * n, *uSW = ac + 13 * n;
+  j = __builtin_amdgcn_readfirstlane(j);
+  k = __builtin_amdgcn_readfirstlane(k);
+  const size_t n = (size_t)nx * ny * nz;
+  const long long sy = nx, sz = (long long)nx * ny;
   // neighbour row classes: (dy, dz) -> zero?
   auto zr = [&](int dy, int dz) -> bool {
     const int cls = 2 * (pz ^ (dz != 0)) + (py ^ (dy != 0));
@@ -620,71 +655,83 @@ __device__ __forceinline__ void gs27_row(
   const bool zN = zr(1, 0), zU = zr(0, 1), zNU = zr(1, 1);  // classes
   const bool zown = (zmask >> (2 * pz + py)) & 1;
   const size_t rb = ix(nx, ny, 1, j, k);  // row base (i = 1)
+  const T *A = ac + rb;                   // plane q of the row: A + q n
   // The loads are unconditional: rows that are still zero in a zero-start
-  // sweep are loaded and replaced by 0 afterwards, and points past the row
-  // end read the last interior point's operands and are not stored.
+  // sweep are loaded and replaced by 0 afterwards, and pairs past the row
+  // end read the last interior point's and are not stored.
   auto load = [&](int i) -> G27Raw<T> {
-    const size_t p = rb + min(i, nx - 1) - 1;
+    const unsigned off = (unsigned)(min(i, nx - 1) - 1) * (unsigned)sizeof(T);
+    auto at = [&](int pl, long long d) {
+      return lane_at(A + (long long)pl * (long long)n + d, 0, off);
+    };
     G27Raw<T> r;
-    r.cN[0] = oN[p], r.xN[0] = xN[p + sy];
-    r.cN[1] = oN[p - sy], r.xN[1] = xN[p - sy];
-    r.cE = oE[p];
-    r.cW = oE[p - 1];
-    r.c[0] = oNE[p], r.xv[0] = xN[p + 1 + sy];
-    r.c[1] = oNW[p], r.xv[1] = xN[p - 1 + sy];
-    r.c[2] = oNW[p + 1 - sy], r.xv[2] = xN[p + 1 - sy];
-    r.c[3] = oNE[p - 1 - sy], r.xv[3] = xN[p - 1 - sy];
-    const T *cu[9] = {uC, uN, uS, uE, uW, uNE, uNW, uSE, uSW};
-    const long long du[9] = {0,
-                             (long long)sy,
-                             -(long long)sy,
-                             1,
-                             -1,
-                             1 + (long long)sy,
-                             -1 + (long long)sy,
-                             1 - (long long)sy,
-                             -1 - (long long)sy};
+    ldn(at(2, 0), r.cN);
+    ldn(at(2, -sy), r.cS);
+    ldn(at(1, 0), r.cE);
+    r.cW = *at(1, -1);
+    ldn(at(4, 0), r.c[0]);
+    ldn(at(5, 0), r.c[1]);
+    ldn(at(5, 1 - sy), r.c[2]);
+    ldn(at(4, -1 - sy), r.c[3]);
+    // planes uC, uN, uS, uE, uW, uNE, uNW, uSE, uSW of the plane above
+    constexpr int pu[9] = {3, 8, 9, 6, 7, 10, 11, 12, 13};
     // the plane below couples through the mirrored plane of the neighbour
-    const T *cd[9] = {uC, uS, uN, uW, uE, uSW, uSE, uNW, uNE};
-    // terms 0, 3, 4 stay in the row's column of planes (dy = 0)
-    const bool dy0[9] = {true, false, false, true, true,
-                         false, false, false, false};
+    constexpr int pd[9] = {3, 9, 8, 7, 6, 13, 12, 11, 10};
+    const long long du[9] = {0, sy, -sy, 1, -1, 1 + sy, -1 + sy, 1 - sy,
+                             -1 - sy};
 #pragma unroll
     for (int m = 0; m < 9; m++) {
-      const T *xz = dy0[m] ? xU : xNU;
-      r.cu[m] = cu[m][p];
-      r.xu[m] = xz[p + du[m] + sz];
-      r.cd[m] = cd[m][p + du[m] - sz];
-      r.xd[m] = xz[p + du[m] - sz];
+      ldn(at(pu[m], 0), r.cu[m]);
+      ldn(at(pd[m], du[m] - sz), r.cd[m]);
     }
-    r.f = fc[p];
-    r.oC = ac[p];
-    r.cc = cc[p];
+    auto row = [&](const T *x, long long d, T(&v)[4]) {
+      ldn(lane_at(x + rb + d, -1, off), v);
+    };
+    row(xN, sy, r.xN);
+    row(xN, -sy, r.xS);
+    row(xU, sz, r.xu[0]);
+    row(xNU, sy + sz, r.xu[1]);
+    row(xNU, -sy + sz, r.xu[2]);
+    row(xU, -sz, r.xd[0]);
+    row(xNU, sy - sz, r.xd[1]);
+    row(xNU, -sy - sz, r.xd[2]);
+    ldn(lane_at(fc + rb, 0, off), r.f);
+    ldn(at(0, 0), r.oC);
+    ldn(lane_at(cc + rb, 0, off), r.cc);
     return r;
   };
-  auto part = [&](const G27Raw<T> &r) -> G27Part<T> {
+  // point s (0, 1) of the pair
+  auto part = [&](const G27Raw<T> &r, auto sc) -> G27Part<T> {
+    constexpr int s = decltype(sc)::value;
     auto Z = [](T v, bool z) -> T { return z ? (T)0 : v; };
     G27Part<T> g;
-    g.a = r.cN[0] * Z(r.xN[0], zN) + r.cN[1] * Z(r.xN[1], zN);
-    g.cE = r.cE;
-    g.cW = r.cW;
+    g.a = r.cN[s] * Z(r.xN[s + 1], zN) + r.cS[s] * Z(r.xS[s + 1], zN);
+    g.cE = r.cE[s];
+    g.cW = s ? r.cE[0] : r.cW;
+    const T xv[4] = {r.xN[s + 2], r.xN[s], r.xS[s + 2], r.xS[s]};
 #pragma unroll
-    for (int m = 0; m < 4; m++) g.c[m] = r.c[m], g.xv[m] = Z(r.xv[m], zN);
-    // u: uC with the plane above's own column, the others diagonal (zNU)
-    // except uE, uW (same row, zU)
-    const bool zu[9] = {zU, zNU, zNU, zU, zU, zNU, zNU, zNU, zNU};
-    T u = r.cu[0] * Z(r.xu[0], zu[0]);
+    for (int m = 0; m < 4; m++) g.c[m] = r.c[m][s], g.xv[m] = Z(xv[m], zN);
+    // terms C, N, S, E, W, NE, NW, SE, SW: the row of the plane (0 the own
+    // column of planes, zU; 1, 2 the rows j + 1, j - 1, zNU) and the place
+    // in it
+    constexpr int tr[9] = {0, 1, 2, 0, 0, 1, 1, 2, 2};
+    constexpr int te[9] = {1, 1, 1, 2, 0, 2, 0, 2, 0};
+    T u = r.cu[0][s] * Z(r.xu[0][s + 1], zU);
 #pragma unroll
-    for (int m = 1; m < 9; m++) u += r.cu[m] * Z(r.xu[m], zu[m]);
-    T dd = r.cd[0] * Z(r.xd[0], zu[0]);
+    for (int m = 1; m < 9; m++)
+      u += r.cu[m][s] * Z(r.xu[tr[m]][s + te[m]], tr[m] ? zNU : zU);
+    T dd = r.cd[0][s] * Z(r.xd[0][s + 1], zU);
 #pragma unroll
-    for (int m = 1; m < 9; m++) dd += r.cd[m] * Z(r.xd[m], zu[m]);
+    for (int m = 1; m < 9; m++)
+      dd += r.cd[m][s] * Z(r.xd[tr[m]][s + te[m]], tr[m] ? zNU : zU);
     g.u = u;
     g.dd = dd;
-    g.f = r.f;
-    g.dg = r.oC + r.cc;
+    g.f = r.f[s];
+    g.dg = r.oC[s] + r.cc[s];
     return g;
   };
+  using P0 = std::integral_constant<int, 0>;
+  using P1 = std::integral_constant<int, 1>;
   // the update from the part and the in-row neighbours xw (i-1), xe (i+1)
   auto fin = [&](const G27Part<T> &g, T xw, T xe) -> T {
     const T o = g.a + g.cE * xe + g.cW * xw + g.c[0] * g.xv[0] +
@@ -701,49 +748,19 @@ __device__ __forceinline__ void gs27_row(
     v0[q] = i0[q] <= nx - 1;
     v1[q] = i1[q] <= nx - 1;
     // current values of the own row, boundary included (i <= nx)
-    const T r0 = xO[rb + min(i0[q], nx) - 1], r1 = xO[rb + min(i1[q], nx) - 1];
+    T r[2];
+    ldn(lane_at(xO + rb, 0,
+                (unsigned)(min(i0[q], nx - 1) - 1) * (unsigned)sizeof(T)),
+        r);
+    // (a pair starting at i = nx, all of it past the interior, has its
+    // first value in the second place of the last pair)
+    const T r0 = v0[q] ? r[0] : r[1], r1 = r[1];
     a0[q] = (i0[q] <= nx) ? (zown && v0[q] ? (T)0 : r0) : (T)0;
     a1[q] = (i1[q] <= nx) ? (zown && v1[q] ? (T)0 : r1) : (T)0;
     n0[q] = a0[q];
     n1[q] = a1[q];
   }
   const T xb1 = xO[rb];  // i = 1 boundary
-  // One lane pair per lane (rows up to 129 points), and two in FP32 (rows
-  // up to 257 points, 4 x 53 values): every load of the lane's points is
-  // issued before any arithmetic, so the row waits for memory once; only
-  // the in-row terms wait for the first colour.  FP64 rows of up to 257
-  // points load each colour's two points together (two round trips instead
-  // of four); longer rows load each point's operands just before its
-  // update.  Same arithmetic in every case.
-  G27Part<T> g0[PPL], g1[PPL];
-  constexpr bool PRE = PPL == 1 || (PPL == 2 && sizeof(T) == 4);
-  if constexpr (PPL == 1) {
-    const G27Raw<T> r0 = load(i0[0]), r1 = load(i1[0]);
-    __builtin_amdgcn_sched_barrier(0);
-    g0[0] = part(r0);
-    g1[0] = part(r1);
-  } else if constexpr (PRE) {
-    const G27Raw<T> r00 = load(i0[0]), r10 = load(i1[0]), r01 = load(i0[1]),
-                    r11 = load(i1[1]);
-    __builtin_amdgcn_sched_barrier(0);
-    g0[0] = part(r00);
-    g1[0] = part(r10);
-    g0[1] = part(r01);
-    g1[1] = part(r11);
-  }
-  constexpr bool PRE1 = !PRE && PPL == 2;
-  auto part0 = [&](int q) -> G27Part<T> {
-    return PRE ? g0[q] : part(load(i0[q]));
-  };
-  auto part1 = [&](int q) -> G27Part<T> {
-    return PRE ? g1[q] : part(load(i1[q]));
-  };
-  auto batch = [&](const int *ii, G27Part<T> *g) {
-    const G27Raw<T> ra = load(ii[0]), rb = load(ii[1]);
-    __builtin_amdgcn_sched_barrier(0);
-    g[0] = part(ra);
-    g[1] = part(rb);
-  };
   // value of the previous pair's second point / next pair's first point
   // (every lane takes part in the shuffles)
   auto west = [&](const T *s, int q) -> T {
@@ -757,36 +774,53 @@ __device__ __forceinline__ void gs27_row(
                                 : e;  // beyond the last interior point
     return lane == 63 ? first : e;
   };
-  if (ADJ == 0) {
-    // colour i%2 = 0 (points i0) from the old odd values, then i%2 = 1
-    if constexpr (PRE1) batch(i0, g0);
-#pragma unroll
-    for (int q = 0; q < PPL; q++) {
+  // The first colour of the row (points i0, or i1 with ADJ) reads old values
+  // only, so pair by pair: load everything the pair needs (one memory round
+  // trip), update its first colour, and keep the terms of the second.  Rows
+  // of up to 257 points in FP32 load both pairs before any arithmetic.
+  constexpr bool BOTH = PPL == 2 && sizeof(T) == 4;
+  G27Part<T> g[PPL];  // the second colour's terms
+  auto first = [&](const G27Raw<T> &r, int q) {
+    if (ADJ == 0) {
       const T w = west(a1, q);
-      const G27Part<T> g = PRE1 ? g0[q] : part0(q);
-      if (v0[q]) n0[q] = fin(g, w, a1[q]);
-    }
-    if constexpr (PRE1) batch(i1, g1);
-#pragma unroll
-    for (int q = 0; q < PPL; q++) {
-      const T e = east(n0, q);
-      const G27Part<T> g = PRE1 ? g1[q] : part1(q);
-      if (v1[q]) n1[q] = fin(g, n0[q], e);
-    }
-  } else {
-    if constexpr (PRE1) batch(i1, g1);
-#pragma unroll
-    for (int q = 0; q < PPL; q++) {
+      const T v = fin(part(r, P0{}), w, a1[q]);
+      n0[q] = v0[q] ? v : n0[q];
+      g[q] = part(r, P1{});
+    } else {
       const T e = east(a0, q);
-      const G27Part<T> g = PRE1 ? g1[q] : part1(q);
-      if (v1[q]) n1[q] = fin(g, a0[q], e);
+      const T v = fin(part(r, P1{}), a0[q], e);
+      n1[q] = v1[q] ? v : n1[q];
+      g[q] = part(r, P0{});
     }
-    if constexpr (PRE1) batch(i0, g0);
+  };
+  if constexpr (BOTH) {
+    const G27Raw<T> ra = load(i0[0]), rc = load(i0[1]);
+    __builtin_amdgcn_sched_barrier(0);
+    first(ra, 0);
+    first(rc, 1);
+  } else {
 #pragma unroll
     for (int q = 0; q < PPL; q++) {
+      const G27Raw<T> ra = load(i0[q]);
+      __builtin_amdgcn_sched_barrier(0);
+      first(ra, q);
+      if (PPL > 1) {  // finish this pair's sums before the next pair's loads
+        asm volatile("" : "+v"(g[q].a), "+v"(g[q].u), "+v"(g[q].dd),
+                          "+v"(g[q].dg), "+v"(n0[q]), "+v"(n1[q]));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < PPL; q++) {
+    if (ADJ == 0) {
+      const T e = east(n0, q);
+      const T v = fin(g[q], n0[q], e);
+      n1[q] = v1[q] ? v : n1[q];
+    } else {
       const T w = west(n1, q);
-      const G27Part<T> g = PRE1 ? g0[q] : part0(q);
-      if (v0[q]) n0[q] = fin(g, w, n1[q]);
+      const T v = fin(g[q], w, n1[q]);
+      n0[q] = v0[q] ? v : n0[q];
     }
   }
 #pragma unroll
