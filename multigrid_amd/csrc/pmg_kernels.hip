@@ -213,9 +213,13 @@ __device__ inline T sum7(const T *__restrict__ ac, size_t n, size_t sy,
          uC[p - sz] * (T)x[p - sz] + uC[p] * (T)x[p + sz];
 }
 
+static unsigned p27_partials(const Dim &d);
 size_t max_partials(const Dim &d) {
-  // bound for any k chunk (kchunk() may pick one plane per block)
-  return (size_t)cdiv(d.nx, BX) * cdiv(d.ny, BY) * d.nz + 64;
+  // bound for any k chunk (kchunk() may pick one plane per block) of the
+  // (BX, BY) blocks, and for the pair kernels of 27-point levels
+  const size_t blocks =
+      (size_t)cdiv(d.nx, BX) * cdiv(d.ny, BY) * d.nz + 64;
+  return std::max(blocks, (size_t)p27_partials(d));
 }
 
 // Planes per block for the residual and matvec kernels: KCH on large
@@ -595,6 +599,17 @@ __device__ __forceinline__ void ldn(const double *p, double (&v)[4]) {
   const f64x2u t = *(const f64x2u *)p, u = *(const f64x2u *)(p + 2);
   v[0] = t.x, v[1] = t.y, v[2] = u.x, v[3] = u.y;
 }
+__device__ __forceinline__ void stn(float *p, const float (&v)[4]) {
+  f32x4u t;
+  t.x = v[0], t.y = v[1], t.z = v[2], t.w = v[3];
+  *(f32x4u *)p = t;
+}
+__device__ __forceinline__ void stn(double *p, const double (&v)[4]) {
+  f64x2u t, u;
+  t.x = v[0], t.y = v[1], u.x = v[2], u.y = v[3];
+  *(f64x2u *)p = t;
+  *(f64x2u *)(p + 2) = u;
+}
 // Element di of a row whose first element is base, for the lane `off` bytes
 // into the row: the base is the same for the whole wavefront (a scalar
 // address) and the lane part stays one 32-bit offset for every array.
@@ -604,20 +619,93 @@ __device__ __forceinline__ const T *lane_at(const T *base, int di,
   return (const T *)((const char *)(base + di) + off);
 }
 
-// The operands of a pair of i-adjacent points (i0, i0 + 1) for their updates
-// (gsd.cc:160-211), as loaded.  Every coupling comes for both points with
-// one two-element load and every neighbouring row of x with one four-element
-// load (i0 - 1 .. i0 + 2): 37 loads of a pair against 106 scalar ones.
+// The operands of a pair of i-adjacent points (i0, i0 + 1) of a 27-point
+// level (gsd.cc:160-211, matvecd.cc:137-170), as loaded.  Every coupling
+// comes for both points with one two-element load and every neighbouring row
+// of x with one four-element load (i0 - 1 .. i0 + 2): 37 loads of a pair
+// against 106 scalar ones.  The kernels on 27-point levels were bound by the
+// rate at which a compute unit takes vector memory instructions, not by
+// bytes (MI355X, the sweeps per paired launch, scalar loads -> these: 145^3
+// FP32 56 -> 44 us, 81^3 FP32 11.2 -> 8.4, FP64 16.5 -> 12.2, 33^3 and 17^3
+// FP64 8.2 -> 5.8 us; the same sums in the same order).  The four-element
+// loads of the last pair of the grid's last row reach one element past the
+// end of x, whose value no sum uses: every x array has that element
+// (allocations are padded).
 template <class T>
-struct G27Raw {
+struct G27C {          // couplings, the right-hand side, the diagonal's parts
   T cN[2], cS[2];      // oN(p), oN(p - sy)
   T cE[2], cW;         // oE(p) of both points, oE(p - 1) of the first
   T c[4][2];           // oNE(p), oNW(p), oNW(p + 1 - sy), oNE(p - 1 - sy)
   T cu[9][2], cd[9][2];
-  T xN[4], xS[4];      // x of rows j + 1, j - 1 in the own plane
-  T xu[3][4], xd[3][4];  // rows j, j + 1, j - 1 of the planes above, below
-  T f[2], oC[2], cc[2];
+  T oC[2], cc[2];
 };
+template <class T>
+struct G27X {
+  T xN[4], xS[4];        // x of rows j + 1, j - 1 in the own plane
+  T xu[3][4], xd[3][4];  // rows j, j + 1, j - 1 of the planes above, below
+};
+// A = ac + base, cc: the arrays at an index `base` that is the same for the
+// whole wavefront (a row or a plane); the pair's first point lies off bytes
+// further.  PL: the planes above and below are wanted (else they count as
+// zero and are not loaded).
+template <bool PL, class T>
+__device__ __forceinline__ void g27_couplings(const T *__restrict__ A,
+                                              const T *__restrict__ cc,
+                                              size_t n, long long sy,
+                                              long long sz, unsigned off,
+                                              G27C<T> &r) {
+  auto at = [&](int pl, long long d) {
+    return lane_at(A + (long long)pl * (long long)n + d, 0, off);
+  };
+  ldn(at(2, 0), r.cN);
+  ldn(at(2, -sy), r.cS);
+  ldn(at(1, 0), r.cE);
+  r.cW = *at(1, -1);
+  ldn(at(4, 0), r.c[0]);
+  ldn(at(5, 0), r.c[1]);
+  ldn(at(5, 1 - sy), r.c[2]);
+  ldn(at(4, -1 - sy), r.c[3]);
+  // planes uC, uN, uS, uE, uW, uNE, uNW, uSE, uSW of the plane above
+  constexpr int pu[9] = {3, 8, 9, 6, 7, 10, 11, 12, 13};
+  // the plane below couples through the mirrored plane of the neighbour
+  constexpr int pd[9] = {3, 9, 8, 7, 6, 13, 12, 11, 10};
+  const long long du[9] = {0,       sy,      -sy,    1,      -1,
+                           1 + sy, -1 + sy, 1 - sy, -1 - sy};
+  if constexpr (PL) {
+#pragma unroll
+    for (int m = 0; m < 9; m++) {
+      ldn(at(pu[m], 0), r.cu[m]);
+      ldn(at(pd[m], du[m] - sz), r.cd[m]);
+    }
+  } else {
+#pragma unroll
+    for (int m = 0; m < 9; m++)
+      r.cu[m][0] = r.cu[m][1] = r.cd[m][0] = r.cd[m][1] = (T)0;
+  }
+  ldn(at(0, 0), r.oC);
+  ldn(lane_at(cc, 0, off), r.cc);
+}
+// The neighbour rows from three arrays by their offset (dy, dz): xN (dy odd,
+// dz = 0), xU (dy = 0, dz odd), xNU (dy and dz odd), each at the base.
+template <bool PL, class T>
+__device__ __forceinline__ void g27_rows(const T *xN, const T *xU,
+                                         const T *xNU, long long sy,
+                                         long long sz, unsigned off,
+                                         G27X<T> &r) {
+  ldn(lane_at(xN + sy, -1, off), r.xN);
+  ldn(lane_at(xN - sy, -1, off), r.xS);
+  if constexpr (PL) {
+    ldn(lane_at(xU + sz, -1, off), r.xu[0]);
+    ldn(lane_at(xNU + sy + sz, -1, off), r.xu[1]);
+    ldn(lane_at(xNU - sy + sz, -1, off), r.xu[2]);
+    ldn(lane_at(xU - sz, -1, off), r.xd[0]);
+    ldn(lane_at(xNU + sy - sz, -1, off), r.xd[1]);
+    ldn(lane_at(xNU - sy - sz, -1, off), r.xd[2]);
+  } else {
+#pragma unroll
+    for (int m = 0; m < 12; m++) r.xu[m / 4][m % 4] = r.xd[m / 4][m % 4] = (T)0;
+  }
+}
 
 // The terms of one point that do not involve the two in-row neighbours,
 // summed in the reference's order as far as they go.
@@ -626,19 +714,51 @@ struct G27Part {
   T a;             // oN(p) x(p+sy) + oN(p-sy) x(p-sy): the first two terms
   T cE, cW;
   T c[4], xv[4];   // the four in-plane terms after the in-row ones
-  T u, dd, f, dg;  // upper and lower plane sums, fc, oC + cc
+  T u, dd, dg;     // upper and lower plane sums, oC + cc
 };
+// Point s (0, 1) of the pair; zN: the rows j +- 1 of the own plane count as
+// zero.
+template <class T, int s>
+__device__ __forceinline__ G27Part<T> g27_part(const G27C<T> &r,
+                                               const G27X<T> &x, bool zN) {
+  auto Z = [](T v, bool z) -> T { return z ? (T)0 : v; };
+  G27Part<T> g;
+  g.a = r.cN[s] * Z(x.xN[s + 1], zN) + r.cS[s] * Z(x.xS[s + 1], zN);
+  g.cE = r.cE[s];
+  g.cW = s ? r.cE[0] : r.cW;
+  const T xv[4] = {x.xN[s + 2], x.xN[s], x.xS[s + 2], x.xS[s]};
+#pragma unroll
+  for (int m = 0; m < 4; m++) g.c[m] = r.c[m][s], g.xv[m] = Z(xv[m], zN);
+  // terms C, N, S, E, W, NE, NW, SE, SW: the row of the plane and the place
+  // in it
+  constexpr int tr[9] = {0, 1, 2, 0, 0, 1, 1, 2, 2};
+  constexpr int te[9] = {1, 1, 1, 2, 0, 2, 0, 2, 0};
+  T u = r.cu[0][s] * x.xu[0][s + 1];
+#pragma unroll
+  for (int m = 1; m < 9; m++) u += r.cu[m][s] * x.xu[tr[m]][s + te[m]];
+  T dd = r.cd[0][s] * x.xd[0][s + 1];
+#pragma unroll
+  for (int m = 1; m < 9; m++) dd += r.cd[m][s] * x.xd[tr[m]][s + te[m]];
+  g.u = u;
+  g.dd = dd;
+  g.dg = r.oC[s] + r.cc[s];
+  return g;
+}
+// The in-plane sum from the part and the in-row neighbours xw, xe.
+template <class T>
+__device__ __forceinline__ T g27_plane(const G27Part<T> &g, T xw, T xe) {
+  return g.a + g.cE * xe + g.cW * xw + g.c[0] * g.xv[0] + g.c[1] * g.xv[1] +
+         g.c[2] * g.xv[2] + g.c[3] * g.xv[3];
+}
 
 // One row (j, k) of class (pz, py) of a 27-point sweep, by one wavefront.
 // The neighbour rows come from four arrays by their offset (dy, dz) from
 // this row: xO (dy, dz even: the row itself), xN (dy odd, dz = 0), xU
 // (dy = 0, dz odd), xNU (dy and dz odd); the new values go to xW.  A
-// sweep kept in one array passes it for all five.  The loads of the last
-// pair of the grid's last row reach one element past the end of x, whose
-// value no sum uses: every x array has that element (allocations are
-// padded).
-template <class T, int ADJ, int PPL>
-__device__ __forceinline__ void gs27_row(
+// sweep kept in one array passes it for all five.  zmask as k_gs27_rows; PL
+// false: the two classes of the other planes are still zero (see gs27_row).
+template <class T, int ADJ, int PPL, bool PL>
+__device__ __forceinline__ void gs27_row_(
     int nx, int ny, int nz, const T *__restrict__ ac, const T *__restrict__ cc,
     const T *__restrict__ fc, int pz, int py, int j, int k, int zmask,
     const T *xO, const T *xN, const T *xU, const T *xNU, T *xW) {
@@ -647,96 +767,29 @@ __device__ __forceinline__ void gs27_row(
   k = __builtin_amdgcn_readfirstlane(k);
   const size_t n = (size_t)nx * ny * nz;
   const long long sy = nx, sz = (long long)nx * ny;
-  // neighbour row classes: (dy, dz) -> zero?
-  auto zr = [&](int dy, int dz) -> bool {
-    const int cls = 2 * (pz ^ (dz != 0)) + (py ^ (dy != 0));
-    return (zmask >> cls) & 1;
-  };
-  const bool zN = zr(1, 0), zU = zr(0, 1), zNU = zr(1, 1);  // classes
+  const bool zN = (zmask >> (2 * pz + 1 - py)) & 1;
   const bool zown = (zmask >> (2 * pz + py)) & 1;
   const size_t rb = ix(nx, ny, 1, j, k);  // row base (i = 1)
-  const T *A = ac + rb;                   // plane q of the row: A + q n
-  // The loads are unconditional: rows that are still zero in a zero-start
-  // sweep are loaded and replaced by 0 afterwards, and pairs past the row
-  // end read the last interior point's and are not stored.
-  auto load = [&](int i) -> G27Raw<T> {
+  struct Raw {
+    G27C<T> c;
+    G27X<T> x;
+    T f[2];
+  };
+  // The loads are unconditional over the lanes: rows of the own plane that
+  // are still zero in a zero-start sweep are loaded and replaced by 0
+  // afterwards, and pairs past the row end read the last interior point's
+  // and are not stored.
+  auto load = [&](int i) -> Raw {
     const unsigned off = (unsigned)(min(i, nx - 1) - 1) * (unsigned)sizeof(T);
-    auto at = [&](int pl, long long d) {
-      return lane_at(A + (long long)pl * (long long)n + d, 0, off);
-    };
-    G27Raw<T> r;
-    ldn(at(2, 0), r.cN);
-    ldn(at(2, -sy), r.cS);
-    ldn(at(1, 0), r.cE);
-    r.cW = *at(1, -1);
-    ldn(at(4, 0), r.c[0]);
-    ldn(at(5, 0), r.c[1]);
-    ldn(at(5, 1 - sy), r.c[2]);
-    ldn(at(4, -1 - sy), r.c[3]);
-    // planes uC, uN, uS, uE, uW, uNE, uNW, uSE, uSW of the plane above
-    constexpr int pu[9] = {3, 8, 9, 6, 7, 10, 11, 12, 13};
-    // the plane below couples through the mirrored plane of the neighbour
-    constexpr int pd[9] = {3, 9, 8, 7, 6, 13, 12, 11, 10};
-    const long long du[9] = {0, sy, -sy, 1, -1, 1 + sy, -1 + sy, 1 - sy,
-                             -1 - sy};
-#pragma unroll
-    for (int m = 0; m < 9; m++) {
-      ldn(at(pu[m], 0), r.cu[m]);
-      ldn(at(pd[m], du[m] - sz), r.cd[m]);
-    }
-    auto row = [&](const T *x, long long d, T(&v)[4]) {
-      ldn(lane_at(x + rb + d, -1, off), v);
-    };
-    row(xN, sy, r.xN);
-    row(xN, -sy, r.xS);
-    row(xU, sz, r.xu[0]);
-    row(xNU, sy + sz, r.xu[1]);
-    row(xNU, -sy + sz, r.xu[2]);
-    row(xU, -sz, r.xd[0]);
-    row(xNU, sy - sz, r.xd[1]);
-    row(xNU, -sy - sz, r.xd[2]);
+    Raw r;
+    g27_couplings<PL>(ac + rb, cc + rb, n, sy, sz, off, r.c);
+    g27_rows<PL>(xN + rb, xU + rb, xNU + rb, sy, sz, off, r.x);
     ldn(lane_at(fc + rb, 0, off), r.f);
-    ldn(at(0, 0), r.oC);
-    ldn(lane_at(cc + rb, 0, off), r.cc);
     return r;
   };
-  // point s (0, 1) of the pair
-  auto part = [&](const G27Raw<T> &r, auto sc) -> G27Part<T> {
-    constexpr int s = decltype(sc)::value;
-    auto Z = [](T v, bool z) -> T { return z ? (T)0 : v; };
-    G27Part<T> g;
-    g.a = r.cN[s] * Z(r.xN[s + 1], zN) + r.cS[s] * Z(r.xS[s + 1], zN);
-    g.cE = r.cE[s];
-    g.cW = s ? r.cE[0] : r.cW;
-    const T xv[4] = {r.xN[s + 2], r.xN[s], r.xS[s + 2], r.xS[s]};
-#pragma unroll
-    for (int m = 0; m < 4; m++) g.c[m] = r.c[m][s], g.xv[m] = Z(xv[m], zN);
-    // terms C, N, S, E, W, NE, NW, SE, SW: the row of the plane (0 the own
-    // column of planes, zU; 1, 2 the rows j + 1, j - 1, zNU) and the place
-    // in it
-    constexpr int tr[9] = {0, 1, 2, 0, 0, 1, 1, 2, 2};
-    constexpr int te[9] = {1, 1, 1, 2, 0, 2, 0, 2, 0};
-    T u = r.cu[0][s] * Z(r.xu[0][s + 1], zU);
-#pragma unroll
-    for (int m = 1; m < 9; m++)
-      u += r.cu[m][s] * Z(r.xu[tr[m]][s + te[m]], tr[m] ? zNU : zU);
-    T dd = r.cd[0][s] * Z(r.xd[0][s + 1], zU);
-#pragma unroll
-    for (int m = 1; m < 9; m++)
-      dd += r.cd[m][s] * Z(r.xd[tr[m]][s + te[m]], tr[m] ? zNU : zU);
-    g.u = u;
-    g.dd = dd;
-    g.f = r.f[s];
-    g.dg = r.oC[s] + r.cc[s];
-    return g;
-  };
-  using P0 = std::integral_constant<int, 0>;
-  using P1 = std::integral_constant<int, 1>;
   // the update from the part and the in-row neighbours xw (i-1), xe (i+1)
-  auto fin = [&](const G27Part<T> &g, T xw, T xe) -> T {
-    const T o = g.a + g.cE * xe + g.cW * xw + g.c[0] * g.xv[0] +
-                g.c[1] * g.xv[1] + g.c[2] * g.xv[2] + g.c[3] * g.xv[3];
-    return (g.f + ((o + g.u) + g.dd)) / g.dg;
+  auto fin = [&](const G27Part<T> &g, T f, T xw, T xe) -> T {
+    return (f + ((g27_plane(g, xw, xe) + g.u) + g.dd)) / g.dg;
   };
   int i0[PPL], i1[PPL];
   bool v0[PPL], v1[PPL];
@@ -780,28 +833,31 @@ __device__ __forceinline__ void gs27_row(
   // of up to 257 points in FP32 load both pairs before any arithmetic.
   constexpr bool BOTH = PPL == 2 && sizeof(T) == 4;
   G27Part<T> g[PPL];  // the second colour's terms
-  auto first = [&](const G27Raw<T> &r, int q) {
+  T f2[PPL];
+  auto first = [&](const Raw &r, int q) {
     if (ADJ == 0) {
       const T w = west(a1, q);
-      const T v = fin(part(r, P0{}), w, a1[q]);
+      const T v = fin(g27_part<T, 0>(r.c, r.x, zN), r.f[0], w, a1[q]);
       n0[q] = v0[q] ? v : n0[q];
-      g[q] = part(r, P1{});
+      g[q] = g27_part<T, 1>(r.c, r.x, zN);
+      f2[q] = r.f[1];
     } else {
       const T e = east(a0, q);
-      const T v = fin(part(r, P1{}), a0[q], e);
+      const T v = fin(g27_part<T, 1>(r.c, r.x, zN), r.f[1], a0[q], e);
       n1[q] = v1[q] ? v : n1[q];
-      g[q] = part(r, P0{});
+      g[q] = g27_part<T, 0>(r.c, r.x, zN);
+      f2[q] = r.f[0];
     }
   };
   if constexpr (BOTH) {
-    const G27Raw<T> ra = load(i0[0]), rc = load(i0[1]);
+    const Raw ra = load(i0[0]), rc = load(i0[1]);
     __builtin_amdgcn_sched_barrier(0);
     first(ra, 0);
     first(rc, 1);
   } else {
 #pragma unroll
     for (int q = 0; q < PPL; q++) {
-      const G27Raw<T> ra = load(i0[q]);
+      const Raw ra = load(i0[q]);
       __builtin_amdgcn_sched_barrier(0);
       first(ra, q);
       if (PPL > 1) {  // finish this pair's sums before the next pair's loads
@@ -815,11 +871,11 @@ __device__ __forceinline__ void gs27_row(
   for (int q = 0; q < PPL; q++) {
     if (ADJ == 0) {
       const T e = east(n0, q);
-      const T v = fin(g[q], n0[q], e);
+      const T v = fin(g[q], f2[q], n0[q], e);
       n1[q] = v1[q] ? v : n1[q];
     } else {
       const T w = west(n1, q);
-      const T v = fin(g[q], w, n1[q]);
+      const T v = fin(g[q], f2[q], w, n1[q]);
       n0[q] = v0[q] ? v : n0[q];
     }
   }
@@ -828,6 +884,23 @@ __device__ __forceinline__ void gs27_row(
     if (v0[q]) xW[rb + i0[q] - 1] = n0[q];
     if (v1[q]) xW[rb + i1[q] - 1] = n1[q];
   }
+}
+
+// The sweeps take the classes plane parity by plane parity, so in a
+// zero-start sweep both classes of the other planes are still zero during
+// the first half: their couplings and values are then not loaded (11 of 37
+// loads are left).
+template <class T, int ADJ, int PPL>
+__device__ __forceinline__ void gs27_row(
+    int nx, int ny, int nz, const T *__restrict__ ac, const T *__restrict__ cc,
+    const T *__restrict__ fc, int pz, int py, int j, int k, int zmask,
+    const T *xO, const T *xN, const T *xU, const T *xNU, T *xW) {
+  if ((zmask >> (2 * (1 - pz))) & 3)
+    gs27_row_<T, ADJ, PPL, false>(nx, ny, nz, ac, cc, fc, pz, py, j, k, zmask,
+                                  xO, xN, xU, xNU, xW);
+  else
+    gs27_row_<T, ADJ, PPL, true>(nx, ny, nz, ac, cc, fc, pz, py, j, k, zmask,
+                                 xO, xN, xU, xNU, xW);
 }
 
 template <class T, int ADJ, int PPL>
@@ -1007,11 +1080,11 @@ void gs27(const Dim &d, const T *ac, const T *cc, const T *fc, T *x,
 }
 
 // ---------------------------------------------------------------------------
-// Residual (Vmresid7_1s / Vmresid27_1s) with optional L1 partial sums: one
-// thread per (i, j) column of a chunk of kc planes (7-point levels with the
-// precomputed diagonal take the march k_resid7m below instead)
+// Residual (Vmresid7_1s / Vmresid27_1s) with optional L1 partial sums.
+// 7-point levels: one thread per (i, j) column of a chunk of kc planes (the
+// march k_resid7m below where it fits).
 // ---------------------------------------------------------------------------
-template <class T, class TO, int ND>
+template <class T, class TO>
 __device__ __forceinline__ void resid_body(
     int nx, int ny, int nz, const T *__restrict__ ac,
     const T *__restrict__ cc, const T *__restrict__ fc,
@@ -1025,20 +1098,20 @@ __device__ __forceinline__ void resid_body(
   const int j = 2 + by * BY + threadIdx.y;
   const int k0 = 2 + bz * kc;
   double acc = 0.0;
-  if (ND == 7 && kc == KCH && tok && i <= nx - 1 && j <= ny - 1) {
+  const T *oE = ac + n, *oN = ac + 2 * n, *uC = ac + 3 * n;
+  auto value = [&](size_t p) -> T {
+    const T dgp = ac[p] + cc[p];
+    return fc[p] + oN[p] * x[p + sy] + oN[p - sy] * x[p - sy] +
+           oE[p] * x[p + 1] + oE[p - 1] * x[p - 1] + uC[p - sz] * x[p - sz] +
+           uC[p] * x[p + sz] - dgp * x[p];
+  };
+  if (kc == KCH && tok && i <= nx - 1 && j <= ny - 1) {
     // the chunk's planes with a fixed trip count and clamped (always valid)
     // loads, so every plane's loads can be issued before the first result
     T vv[KCH];
 #pragma unroll
-    for (int kk = 0; kk < KCH; kk++) {
-      const int k = min(k0 + kk, nz - 1);
-      const size_t p = ix(nx, ny, i, j, k);
-      const T *oE = ac + n, *oN = ac + 2 * n, *uC = ac + 3 * n;
-      const T dgp = ac[p] + cc[p];
-      vv[kk] = fc[p] + oN[p] * x[p + sy] + oN[p - sy] * x[p - sy] +
-               oE[p] * x[p + 1] + oE[p - 1] * x[p - 1] +
-               uC[p - sz] * x[p - sz] + uC[p] * x[p + sz] - dgp * x[p];
-    }
+    for (int kk = 0; kk < KCH; kk++)
+      vv[kk] = value(ix(nx, ny, i, j, min(k0 + kk, nz - 1)));
 #pragma unroll
     for (int kk = 0; kk < KCH; kk++) {
       if (k0 + kk > nz - 1) break;
@@ -1050,19 +1123,7 @@ __device__ __forceinline__ void resid_body(
       const int k = k0 + kk;
       if (k > nz - 1) break;
       const size_t p = ix(nx, ny, i, j, k);
-      T v;
-      if (ND == 7) {
-        const T *oE = ac + n, *oN = ac + 2 * n, *uC = ac + 3 * n;
-        const T dgp = ac[p] + cc[p];
-        v = fc[p] + oN[p] * x[p + sy] + oN[p - sy] * x[p - sy] +
-            oE[p] * x[p + 1] + oE[p - 1] * x[p - 1] +
-            uC[p - sz] * x[p - sz] + uC[p] * x[p + sz] - dgp * x[p];
-      } else {
-        double sO, sU, sD;
-        sum27<T, T>(ac, n, sy, sz, p, x, sO, sU, sD);
-        v = (T)((T)((T)(fc[p] + (T)sO) + (T)sU) + (T)sD) -
-            (ac[p] + cc[p]) * x[p];
-      }
+      const T v = value(p);
       if (r) r[p] = (TO)v;
       acc += fabs((double)v);
     }
@@ -1073,14 +1134,126 @@ __device__ __forceinline__ void resid_body(
   }
 }
 
-template <class T, class TO, int ND>
+template <class T, class TO>
 __global__ __launch_bounds__(256) void k_resid(
     int nx, int ny, int nz, const T *__restrict__ ac,
     const T *__restrict__ cc, const T *__restrict__ fc,
     const T *__restrict__ x, TO *__restrict__ r, Red rd, int do_red, int kc,
     XG xg) {
-  resid_body<T, TO, ND>(nx, ny, nz, ac, cc, fc, x, r, rd, do_red, kc, xg,
-                        blockIdx.x);
+  resid_body<T, TO>(nx, ny, nz, ac, cc, fc, x, r, rd, do_red, kc, xg,
+                    blockIdx.x);
+}
+
+// Residual and operator product on 27-point levels: a thread takes pairs of
+// i-adjacent points (G27C), a workgroup consecutive pairs of a plane (i
+// fastest across row ends, so short rows leave no lanes idle) over a chunk of
+// planes.  The plane's base address is the same for the whole workgroup, so
+// every load is a scalar base plus one lane offset.  Small levels, bound by
+// latency, take one-wavefront workgroups over single planes, so that a
+// compute unit issues the 39 loads of few wavefronts; levels of more than
+// NARROW_TILES such workgroups (65^3 up) take workgroups of four, and from
+// 100 planes on chunks of four planes, whose shared couplings then come from
+// the L1 (145^3 FP32 product 42 us; single planes in the order of the
+// workgroups 47 us).  Fewer workgroups also mean fewer partial sums for the
+// prolongation after a product (2840 of 73^3: 21 us against 13).
+constexpr int NARROW_TILES = 1024;
+struct P27 {
+  int np, gx, gz, kc;  // pairs per row, tiles per plane, chunks, planes each
+  int rows;            // wavefronts per workgroup
+  unsigned nblk;
+};
+static P27 p27_shape(const Dim &d) {
+  P27 s;
+  s.np = (d.nx - 1) / 2;
+  const int pairs = s.np * (d.ny - 2);
+  s.rows = cdiv(pairs, BX) * (d.nz - 2) > NARROW_TILES ? BY : 1;
+  s.kc = d.nz >= 100 ? KCH : 1;
+  s.gx = cdiv(pairs, BX * s.rows);
+  s.gz = cdiv(d.nz - 2, s.kc);
+  s.nblk = 8u * (unsigned)cdiv(s.gx * s.gz, 8);
+  return s;
+}
+static unsigned p27_partials(const Dim &d) {
+  return d.nx < 3 || d.ny < 3 || d.nz < 3 ? 0 : p27_shape(d).nblk;
+}
+// Calls f(base, off, both) for every pair of the workgroup's tile: base the
+// index of the plane's first element, off the pair's bytes into the plane,
+// both whether its second point is interior.
+template <class T, class F>
+__device__ __forceinline__ void p27_each(int nx, int ny, int nz, const P27 &s,
+                                         unsigned bid, F f) {
+  const int nt = s.gx * s.gz, per = (nt + 7) / 8;
+  const int t = (int)(bid % 8u) * per + (int)(bid / 8u);
+  if (t >= nt) return;
+  const int q = (t % s.gx) * (BX * s.rows) + threadIdx.y * BX + threadIdx.x;
+  const int j = 2 + q / s.np, i = 2 + 2 * (q % s.np);
+  if (j > ny - 1) return;
+  const unsigned off =
+      (unsigned)((j - 1) * nx + i - 1) * (unsigned)sizeof(T);
+  const int k0 = 2 + (t / s.gx) * s.kc, k1 = min(k0 + s.kc, nz);
+#pragma unroll 1
+  for (int k = k0; k < k1; k++) {
+    int ko = k;  // addresses from this plane's base, not 50 running pointers
+    asm volatile("" : "+s"(ko));
+    f(ix(nx, ny, 1, 1, ko), off, i + 1 <= nx - 1);
+  }
+}
+// Sums over the workgroup's wavefronts (valid in every thread).
+__device__ __forceinline__ void p27_sum(const P27 &s, double &a, double &b,
+                                        double *red) {
+  a = wave_sum(a), b = wave_sum(b);
+  if (s.rows == 1) return;
+  if (threadIdx.x == 0) red[2 * threadIdx.y] = a, red[2 * threadIdx.y + 1] = b;
+  __syncthreads();
+  a = (red[0] + red[2]) + (red[4] + red[6]);
+  b = (red[1] + red[3]) + (red[5] + red[7]);
+}
+
+template <class T, class TO>
+__device__ __forceinline__ void resid27_body(
+    int nx, int ny, int nz, const T *__restrict__ ac,
+    const T *__restrict__ cc, const T *__restrict__ fc,
+    const T *__restrict__ x, TO *__restrict__ r, Red rd, int do_red, P27 s,
+    unsigned bid) {
+  __shared__ double red[2 * BY];
+  const size_t n = (size_t)nx * ny * nz;
+  const long long sy = nx, sz = (long long)nx * ny;
+  double acc = 0.0;
+  p27_each<T>(nx, ny, nz, s, bid, [&](size_t base, unsigned off, bool both) {
+    G27C<T> c;
+    G27X<T> v;
+    T xo[4], f[2];
+    g27_couplings<true>(ac + base, cc + base, n, sy, sz, off, c);
+    g27_rows<true>(x + base, x + base, x + base, sy, sz, off, v);
+    ldn(lane_at(x + base, -1, off), xo);
+    ldn(lane_at(fc + base, 0, off), f);
+    __builtin_amdgcn_sched_barrier(0);  // every load before any arithmetic
+    const G27Part<T> g0 = g27_part<T, 0>(c, v, false),
+                     g1 = g27_part<T, 1>(c, v, false);
+    const T r0 = (((f[0] + g27_plane(g0, xo[0], xo[2])) + g0.u) + g0.dd) -
+                 g0.dg * xo[1];
+    const T r1 = (((f[1] + g27_plane(g1, xo[1], xo[3])) + g1.u) + g1.dd) -
+                 g1.dg * xo[2];
+    if (r) {
+      TO *o = (TO *)((char *)(r + base) + off / sizeof(T) * sizeof(TO));
+      o[0] = (TO)r0;
+      if (both) o[1] = (TO)r1;
+    }
+    acc += fabs((double)r0);
+    if (both) acc += fabs((double)r1);
+  });
+  if (do_red) {
+    double none = 0.0;
+    p27_sum(s, acc, none, red);
+    red_store_at<1>(rd, bid, acc, 0.0);
+  }
+}
+template <class T, class TO>
+__global__ __launch_bounds__(256) void k_resid27(
+    int nx, int ny, int nz, const T *__restrict__ ac,
+    const T *__restrict__ cc, const T *__restrict__ fc,
+    const T *__restrict__ x, TO *__restrict__ r, Red rd, int do_red, P27 s) {
+  resid27_body<T, TO>(nx, ny, nz, ac, cc, fc, x, r, rd, do_red, s, blockIdx.x);
 }
 
 // The 7-point residual with the precomputed diagonal as a march in k (the
@@ -1248,16 +1421,20 @@ void resid(const Dim &d, int numdia, const T *ac, const T *cc, const T *fc,
     check_launch("resid");
     return;
   }
+  const Red rd = red ? *red : Red{};
+  const dim3 b(BX, BY);
+  if (numdia == 27) {
+    const P27 sh = p27_shape(d);
+    k_resid27<T, TO><<<sh.nblk, dim3(BX, sh.rows), 0, s>>>(d.nx, d.ny, d.nz, ac, cc, fc, x, r,
+                                           rd, red ? 1 : 0, sh);
+    if (red) red_final<1, 0>(rd, dim3(sh.nblk), s);
+    check_launch("resid");
+    return;
+  }
   const int kc = kchunk(d, red ? 40 : 80);
   dim3 g(cdiv(d.nx - 2, BX), cdiv(d.ny - 2, BY), cdiv(d.nz - 2, kc));
-  dim3 b(BX, BY);
-  const Red rd = red ? *red : Red{};
-  if (numdia == 7)
-    k_resid<T, TO, 7><<<xcd_blocks(g), b, 0, s>>>(
-        d.nx, d.ny, d.nz, ac, cc, fc, x, r, rd, red ? 1 : 0, kc, xg_of(g));
-  else
-    k_resid<T, TO, 27><<<xcd_blocks(g), b, 0, s>>>(
-        d.nx, d.ny, d.nz, ac, cc, fc, x, r, rd, red ? 1 : 0, kc, xg_of(g));
+  k_resid<T, TO><<<xcd_blocks(g), b, 0, s>>>(d.nx, d.ny, d.nz, ac, cc, fc, x,
+                                             r, rd, red ? 1 : 0, kc, xg_of(g));
   if (red) red_final<1, 0>(rd, dim3(xcd_blocks(g)), s);
   check_launch("resid");
 }
@@ -1382,7 +1559,7 @@ void nmresid(const Dim &d, int numdia, const double *ac, const double *cc,
 // y = A x with partial sums of x.w0 and x.y (Vmatvec + 2 Vxdot, Vxdot
 // being x . y; the reference's squares x)
 // ---------------------------------------------------------------------------
-template <class T, int ND>
+template <class T>
 __device__ __forceinline__ void matvec_dots_body(
     int nx, int ny, int nz, const T *__restrict__ ac,
     const T *__restrict__ cc, const T *__restrict__ x,
@@ -1397,21 +1574,15 @@ __device__ __forceinline__ void matvec_dots_body(
   const int k0 = 2 + bz * kc;
   double a0 = 0.0, a1 = 0.0;
   if (tok && i <= nx - 1 && j <= ny - 1) {
+    const T *oE = ac + n, *oN = ac + 2 * n, *uC = ac + 3 * n;
     for (int kk = 0; kk < kc; kk++) {
       const int k = k0 + kk;
       if (k > nz - 1) break;
       const size_t p = ix(nx, ny, i, j, k);
-      T v;
-      if (ND == 7) {
-        const T *oE = ac + n, *oN = ac + 2 * n, *uC = ac + 3 * n;
-        v = -oN[p] * x[p + sy] - oN[p - sy] * x[p - sy] - oE[p] * x[p + 1] -
-            oE[p - 1] * x[p - 1] - uC[p - sz] * x[p - sz] -
-            uC[p] * x[p + sz] + (ac[p] + cc[p]) * x[p];
-      } else {
-        double sO, sU, sD;
-        sum27<T, T>(ac, n, sy, sz, p, x, sO, sU, sD);
-        v = (T)((T)(-(T)sO + -(T)sU) + -(T)sD) + (ac[p] + cc[p]) * x[p];
-      }
+      const T v = -oN[p] * x[p + sy] - oN[p - sy] * x[p - sy] -
+                  oE[p] * x[p + 1] - oE[p - 1] * x[p - 1] -
+                  uC[p - sz] * x[p - sz] - uC[p] * x[p + sz] +
+                  (ac[p] + cc[p]) * x[p];
       if (y) y[p] = v;
       if (w0) a0 += (double)x[p] * (double)w0[p];
       a1 += (double)x[p] * (double)v;
@@ -1424,190 +1595,270 @@ __device__ __forceinline__ void matvec_dots_body(
   }
 }
 
-template <class T, int ND>
+template <class T>
 __global__ __launch_bounds__(256) void k_matvec_dots(
     int nx, int ny, int nz, const T *__restrict__ ac,
     const T *__restrict__ cc, const T *__restrict__ x,
     const T *__restrict__ w0, T *__restrict__ y, Red rd, int do_red, int kc,
     XG xg) {
-  matvec_dots_body<T, ND>(nx, ny, nz, ac, cc, x, w0, y, rd, do_red, kc, xg,
-                          blockIdx.x);
+  matvec_dots_body<T>(nx, ny, nz, ac, cc, x, w0, y, rd, do_red, kc, xg,
+                      blockIdx.x);
+}
+
+// 27-point levels: pairs, as resid27_body.
+template <class T>
+__device__ __forceinline__ void matvec27_body(
+    int nx, int ny, int nz, const T *__restrict__ ac,
+    const T *__restrict__ cc, const T *__restrict__ x,
+    const T *__restrict__ w0, T *__restrict__ y, Red rd, int do_red, P27 s,
+    unsigned bid) {
+  __shared__ double red[2 * BY];
+  const size_t n = (size_t)nx * ny * nz;
+  const long long sy = nx, sz = (long long)nx * ny;
+  double a0 = 0.0, a1 = 0.0;
+  p27_each<T>(nx, ny, nz, s, bid, [&](size_t base, unsigned off, bool both) {
+    G27C<T> c;
+    G27X<T> v;
+    T xo[4], w[2] = {(T)0, (T)0};
+    g27_couplings<true>(ac + base, cc + base, n, sy, sz, off, c);
+    g27_rows<true>(x + base, x + base, x + base, sy, sz, off, v);
+    ldn(lane_at(x + base, -1, off), xo);
+    if (w0) ldn(lane_at(w0 + base, 0, off), w);
+    __builtin_amdgcn_sched_barrier(0);
+    const G27Part<T> g0 = g27_part<T, 0>(c, v, false),
+                     g1 = g27_part<T, 1>(c, v, false);
+    const T y0 = ((-g27_plane(g0, xo[0], xo[2]) + -g0.u) + -g0.dd) +
+                 g0.dg * xo[1];
+    const T y1 = ((-g27_plane(g1, xo[1], xo[3]) + -g1.u) + -g1.dd) +
+                 g1.dg * xo[2];
+    if (y) {
+      T *o = (T *)((char *)(y + base) + off);
+      o[0] = y0;
+      if (both) o[1] = y1;
+    }
+    a0 += (double)xo[1] * (double)w[0];
+    a1 += (double)xo[1] * (double)y0;
+    if (both) {
+      a0 += (double)xo[2] * (double)w[1];
+      a1 += (double)xo[2] * (double)y1;
+    }
+  });
+  if (do_red) {
+    p27_sum(s, a0, a1, red);
+    red_store_at<2>(rd, bid, a0, a1);
+  }
+}
+template <class T>
+__global__ __launch_bounds__(256) void k_matvec27(
+    int nx, int ny, int nz, const T *__restrict__ ac,
+    const T *__restrict__ cc, const T *__restrict__ x,
+    const T *__restrict__ w0, T *__restrict__ y, Red rd, int do_red, P27 s) {
+  matvec27_body<T>(nx, ny, nz, ac, cc, x, w0, y, rd, do_red, s, blockIdx.x);
+}
+
+// Launches the product of a level; returns its workgroups (and partials).
+template <class T>
+static unsigned matvec_launch(const Dim &d, int numdia, const T *ac,
+                              const T *cc, const T *x, const T *w0, T *y,
+                              const Red *red, hipStream_t s) {
+  const Red rd = red ? *red : Red{};
+  const dim3 b(BX, BY);
+  unsigned nb;
+  if (numdia == 7) {
+    const int kc = kchunk(d);
+    const dim3 g(cdiv(d.nx - 2, BX), cdiv(d.ny - 2, BY), cdiv(d.nz - 2, kc));
+    nb = xcd_blocks(g);
+    k_matvec_dots<T><<<nb, b, 0, s>>>(d.nx, d.ny, d.nz, ac, cc, x, w0, y, rd,
+                                      red ? 1 : 0, kc, xg_of(g));
+  } else {
+    const P27 sh = p27_shape(d);
+    nb = sh.nblk;
+    k_matvec27<T><<<nb, dim3(BX, sh.rows), 0, s>>>(d.nx, d.ny, d.nz, ac, cc, x, w0, y, rd,
+                                   red ? 1 : 0, sh);
+  }
+  check_launch("matvec_dots");
+  return nb;
 }
 
 template <class T>
 void matvec_dots(const Dim &d, int numdia, const T *ac, const T *cc,
                  const T *x, const T *w0, T *y, const Red *red,
                  hipStream_t s) {
-  const int kc = kchunk(d);
-  dim3 g(cdiv(d.nx - 2, BX), cdiv(d.ny - 2, BY), cdiv(d.nz - 2, kc));
-  dim3 b(BX, BY);
-  const Red rd = red ? *red : Red{};
-  if (numdia == 7)
-    k_matvec_dots<T, 7><<<xcd_blocks(g), b, 0, s>>>(d.nx, d.ny, d.nz, ac, cc, x, w0, y,
-                                        rd, red ? 1 : 0, kc, xg_of(g));
-  else
-    k_matvec_dots<T, 27><<<xcd_blocks(g), b, 0, s>>>(d.nx, d.ny, d.nz, ac, cc, x, w0, y,
-                                         rd, red ? 1 : 0, kc, xg_of(g));
-  if (red) red_final<2, 1>(rd, dim3(xcd_blocks(g)), s);
-  check_launch("matvec_dots");
+  const unsigned nb = matvec_launch<T>(d, numdia, ac, cc, x, w0, y, red, s);
+  if (red) red_final<2, 1>(*red, dim3(nb), s);
 }
 
 template <class T>
 unsigned matvec_dots_part(const Dim &d, int numdia, const T *ac, const T *cc,
                           const T *x, const T *w0, T *y, double *part,
                           hipStream_t s) {
-  const int kc = kchunk(d);
-  dim3 g(cdiv(d.nx - 2, BX), cdiv(d.ny - 2, BY), cdiv(d.nz - 2, kc));
-  dim3 b(BX, BY);
   Red rd;
   rd.part = part;
-  if (numdia == 7)
-    k_matvec_dots<T, 7><<<xcd_blocks(g), b, 0, s>>>(d.nx, d.ny, d.nz, ac, cc, x, w0, y,
-                                        rd, 1, kc, xg_of(g));
-  else
-    k_matvec_dots<T, 27><<<xcd_blocks(g), b, 0, s>>>(d.nx, d.ny, d.nz, ac, cc, x, w0, y,
-                                         rd, 1, kc, xg_of(g));
-  check_launch("matvec_dots");
-  return xcd_blocks(g);
+  return matvec_launch<T>(d, numdia, ac, cc, x, w0, y, &rd, s);
 }
 
 // ---------------------------------------------------------------------------
 // Grid transfer: Vrestrc2 (matvecd.cc:755-795), VinterpPMG2 (:878-960)
 // ---------------------------------------------------------------------------
-template <class T>
+// A thread restricts to two i-adjacent coarse points: every P plane comes for
+// both with one two-element load, a fine row's five values with a four-element
+// and a scalar load (45 loads for two points against 108).  A workgroup
+// takes consecutive pairs of a coarse plane, i fastest across row ends; one
+// wavefront of them on small levels, four on large ones (as P27).
+struct PR {
+  int np, gx, nt;  // pairs per row, tiles per plane, tiles
+  int rows;        // wavefronts per workgroup
+  unsigned nblk;
+};
+// rows x planes of pairs; npt: points (or cells) per row
+static PR pr_shape(int npt, int rows, int planes) {
+  PR s;
+  s.np = (npt + 1) / 2;
+  s.rows = cdiv(s.np * rows, BX) * planes > NARROW_TILES ? BY : 1;
+  s.gx = cdiv(s.np * rows, BX * s.rows);
+  s.nt = s.gx * planes;
+  s.nblk = 8u * (unsigned)cdiv(s.nt, 8);
+  return s;
+}
+// The pair of this thread in the XCD-contiguous tiles: place in the row, row
+// and plane (from 0); false past the last tile or row.
+__device__ __forceinline__ bool pr_pair(const PR &s, unsigned bid, int rows,
+                                        int &m, int &row, int &plane) {
+  const int per = (s.nt + 7) / 8;
+  const int t = (int)(bid % 8u) * per + (int)(bid / 8u);
+  if ((int)(bid / 8u) >= per || t >= s.nt) return false;
+  plane = t / s.gx;
+  const int q = (t % s.gx) * (BX * s.rows) + threadIdx.y * BX + threadIdx.x;
+  m = q % s.np, row = q / s.np;
+  return row < rows;
+}
+
+// NS sources restricted in one pass (the setup's cc and fc; Newton's
+// right-hand side and Jacobian term): every P plane is loaded once for all of
+// them; each sum keeps its term order, so the results do not depend on NS.
+template <class T, int NS>
+struct RSrc {
+  const T *in[NS];
+  T *out[NS];
+  float *out32[NS];
+};
+template <class T, int NS>
 __device__ __forceinline__ void restrict_body(int nxf, int nyf, int nxc,
                                               int nyc, int nzc,
-                                              const T *__restrict__ xin,
-                                              T *__restrict__ xout,
-                                              const T *__restrict__ pc, XG xg,
-                                              float *__restrict__ out32,
+                                              const RSrc<T, NS> &io,
+                                              const T *__restrict__ pc, PR s,
                                               unsigned bid) {
   // no multiply-add contraction: the setup restricts cc and fc with this
   // kernel, and a source of both signs cancels in those sums, so the
   // coarse cc and fc are the oracle's to the bit only with the same
   // roundings (same term order, separate multiply and add)
 #pragma clang fp contract(off)
-  int bx, by, bz;
-  if (!xcd_tile_at(xg, bid, bx, by, bz)) return;
-  const int ii = 2 + bx * BX + threadIdx.x;
-  const int jj = 2 + by * BY + threadIdx.y;
-  const int kk = 2 + bz;
-  if (ii > nxc - 1 || jj > nyc - 1) return;
-  const size_t nc = (size_t)nxc * nyc * nzc, pC = ix(nxc, nyc, ii, jj, kk);
-  const size_t sy = nxf, sz = (size_t)nxf * nyf;
-  const size_t f = ix(nxf, nyf, 2 * ii - 1, 2 * jj - 1, 2 * kk - 1);
-  // in-plane offsets in P plane order C,N,S,E,W,NE,NW,SE,SW
-  const long long off[9] = {0,
-                            (long long)sy,
-                            -(long long)sy,
-                            1,
-                            -1,
-                            1 + (long long)sy,
-                            -1 + (long long)sy,
-                            1 - (long long)sy,
-                            -1 - (long long)sy};
-  const long long zo[3] = {0, (long long)sz, -(long long)sz};
-  T t[3];
+  int m, row, plane;
+  if (!pr_pair(s, bid, nyc - 2, m, row, plane)) return;
+  const int ii = 2 + 2 * m, jj = 2 + row, kk = 2 + plane;
+  const bool both = ii + 1 <= nxc - 1;
+  const size_t nc = (size_t)nxc * nyc * nzc;
+  const long long sy = nxf, sz = (long long)nxf * nyf;
+  // plane bases (the same for the workgroup) and the pair's bytes into them
+  const size_t pb = ix(nxc, nyc, 1, 1, kk);
+  const unsigned po = (unsigned)((jj - 1) * nxc + ii - 1) * (unsigned)sizeof(T);
+  const size_t fb = ix(nxf, nyf, 1, 1, 2 * kk - 1);
+  const unsigned fo =
+      (unsigned)((2 * jj - 2) * nxf + 2 * ii - 2) * (unsigned)sizeof(T);
+  // P planes C,N,S,E,W,NE,NW,SE,SW of each z: the row and the place in it
+  constexpr int tr[9] = {0, 1, 2, 0, 0, 1, 1, 2, 2};
+  constexpr int te[9] = {1, 1, 1, 2, 0, 2, 0, 2, 0};
+  const long long ro[3] = {0, sy, -sy}, zo[3] = {0, sz, -sz};
+  T w[3][9][2], f[NS][3][3][5], t[NS][2][3];
+  // ZG planes of P and of the sources are loaded before their sums: all
+  // three, or one after the other for two sources (within 256 registers)
+  constexpr int ZG = NS == 1 ? 3 : 1;
 #pragma unroll
-  for (int b = 0; b < 3; b++) {
-    T acc = pc[(size_t)(9 * b) * nc + pC] * xin[f + zo[b]];
+  for (int z0 = 0; z0 < 3; z0 += ZG) {
 #pragma unroll
-    for (int q = 1; q < 9; q++)
-      acc += pc[(size_t)(9 * b + q) * nc + pC] * xin[f + zo[b] + off[q]];
-    t[b] = acc;
+    for (int z = z0; z < z0 + ZG; z++) {
+#pragma unroll
+      for (int q = 0; q < 9; q++)
+        ldn(lane_at(pc + (size_t)(9 * z + q) * nc + pb, 0, po), w[z][q]);
+#pragma unroll
+      for (int v = 0; v < NS; v++)
+#pragma unroll
+        for (int r = 0; r < 3; r++) {  // f - 1 .. f + 3 of rows j, j+1, j-1
+          const T *g = lane_at(io.in[v] + fb + ro[r] + zo[z], -1, fo);
+          T h[4];
+          ldn(g, h);
+          f[v][z][r][0] = h[0], f[v][z][r][1] = h[1];
+          f[v][z][r][2] = h[2], f[v][z][r][3] = h[3];
+          f[v][z][r][4] = g[4];
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int z = z0; z < z0 + ZG; z++)
+#pragma unroll
+      for (int v = 0; v < NS; v++)
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+          T acc = w[z][0][e] * f[v][z][0][1 + 2 * e];
+#pragma unroll
+          for (int q = 1; q < 9; q++)
+            acc += w[z][q][e] * f[v][z][tr[q]][te[q] + 2 * e];
+          t[v][e][z] = acc;
+        }
+    if (NS > 1) {
+#pragma unroll
+      for (int v = 0; v < NS; v++)
+        asm volatile("" : "+v"(t[v][0][z0]), "+v"(t[v][1][z0]));
+      __builtin_amdgcn_sched_barrier(0);
+    }
   }
-  const T v = t[0] + t[1] + t[2];
-  xout[pC] = v;
-  if (out32) out32[pC] = (float)v;
+  const size_t pC = pb + (size_t)(jj - 1) * nxc + (ii - 1);
+#pragma unroll
+  for (int v = 0; v < NS; v++)
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+      if (e && !both) break;
+      const T r = t[v][e][0] + t[v][e][1] + t[v][e][2];
+      io.out[v][pC + e] = r;
+      if (io.out32[v]) io.out32[v][pC + e] = (float)r;
+    }
 }
 
-template <class T>
+template <class T, int NS>
 __global__ __launch_bounds__(256) void k_restrict(int nxf, int nyf, int nxc,
                                                   int nyc, int nzc,
-                                                  const T *__restrict__ xin,
-                                                  T *__restrict__ xout,
-                                                  const T *__restrict__ pc, XG xg,
-                                                  float *__restrict__ out32) {
-  restrict_body<T>(nxf, nyf, nxc, nyc, nzc, xin, xout, pc, xg, out32,
-                   blockIdx.x);
+                                                  RSrc<T, NS> io,
+                                                  const T *__restrict__ pc,
+                                                  PR s) {
+  restrict_body<T, NS>(nxf, nyf, nxc, nyc, nzc, io, pc, s, blockIdx.x);
+}
+
+template <class T, int NS>
+static void restrict_launch(const Dim &f, const Dim &c,
+                            const RSrc<T, NS> &io, const T *pc,
+                            hipStream_t s) {
+  if (c.nx < 3 || c.ny < 3 || c.nz < 3) return;
+  if (f.nx != 2 * c.nx - 1 || f.ny != 2 * c.ny - 1 || f.nz != 2 * c.nz - 1) {
+    fprintf(stderr, "pmg: restrict shape mismatch\n");
+    return;
+  }
+  const PR sh = pr_shape(c.nx - 2, c.ny - 2, c.nz - 2);
+  k_restrict<T, NS><<<sh.nblk, dim3(BX, sh.rows), 0, s>>>(f.nx, f.ny, c.nx, c.ny,
+                                                     c.nz, io, pc, sh);
+  check_launch("restrict");
 }
 
 template <class T>
 void restrict_(const Dim &f, const Dim &c, const T *xin, T *xout, const T *pc,
                hipStream_t s, float *out32) {
-  if (c.nx < 3 || c.ny < 3 || c.nz < 3) return;
-  if (f.nx != 2 * c.nx - 1 || f.ny != 2 * c.ny - 1 || f.nz != 2 * c.nz - 1) {
-    fprintf(stderr, "pmg: restrict shape mismatch\n");
-    return;
-  }
-  dim3 g(cdiv(c.nx - 2, BX), cdiv(c.ny - 2, BY), c.nz - 2);
-  k_restrict<T><<<xcd_blocks(g), dim3(BX, BY), 0, s>>>(f.nx, f.ny, c.nx, c.ny, c.nz, xin,
-                                           xout, pc, xg_of(g), out32);
-  check_launch("restrict");
-}
-
-// Two sources restricted in one pass (the setup's cc and fc): every P plane
-// is loaded once for both sums, each of which keeps restrict_body's term
-// order, so the results are those of two k_restrict launches to the bit.
-__global__ __launch_bounds__(256) void k_restrict2(
-    int nxf, int nyf, int nxc, int nyc, int nzc, const double *__restrict__ a,
-    const double *__restrict__ b, double *__restrict__ ao,
-    double *__restrict__ bo, const double *__restrict__ pc, XG xg,
-    float *__restrict__ ao32, float *__restrict__ bo32) {
-#pragma clang fp contract(off)
-  int bx, by, bz;
-  if (!xcd_tile(xg, bx, by, bz)) return;
-  const int ii = 2 + bx * BX + threadIdx.x;
-  const int jj = 2 + by * BY + threadIdx.y;
-  const int kk = 2 + bz;
-  if (ii > nxc - 1 || jj > nyc - 1) return;
-  const size_t nc = (size_t)nxc * nyc * nzc, pC = ix(nxc, nyc, ii, jj, kk);
-  const size_t sy = nxf, sz = (size_t)nxf * nyf;
-  const size_t f = ix(nxf, nyf, 2 * ii - 1, 2 * jj - 1, 2 * kk - 1);
-  const long long off[9] = {0,
-                            (long long)sy,
-                            -(long long)sy,
-                            1,
-                            -1,
-                            1 + (long long)sy,
-                            -1 + (long long)sy,
-                            1 - (long long)sy,
-                            -1 - (long long)sy};
-  const long long zo[3] = {0, (long long)sz, -(long long)sz};
-  double ta[3], tb[3];
-#pragma unroll
-  for (int z = 0; z < 3; z++) {
-    const double w0 = pc[(size_t)(9 * z) * nc + pC];
-    double sa = w0 * a[f + zo[z]], sb = w0 * b[f + zo[z]];
-#pragma unroll
-    for (int q = 1; q < 9; q++) {
-      const double w = pc[(size_t)(9 * z + q) * nc + pC];
-      sa += w * a[f + zo[z] + off[q]];
-      sb += w * b[f + zo[z] + off[q]];
-    }
-    ta[z] = sa;
-    tb[z] = sb;
-  }
-  const double va = ta[0] + ta[1] + ta[2];
-  ao[pC] = va;
-  if (ao32) ao32[pC] = (float)va;
-  const double vb = tb[0] + tb[1] + tb[2];
-  bo[pC] = vb;
-  if (bo32) bo32[pC] = (float)vb;
+  restrict_launch<T, 1>(f, c, RSrc<T, 1>{{xin}, {xout}, {out32}}, pc, s);
 }
 
 void restrict2(const Dim &f, const Dim &c, const double *a, const double *b,
                double *ao, double *bo, const double *pc, hipStream_t s,
                float *ao32, float *bo32) {
-  if (c.nx < 3 || c.ny < 3 || c.nz < 3) return;
-  if (f.nx != 2 * c.nx - 1 || f.ny != 2 * c.ny - 1 || f.nz != 2 * c.nz - 1) {
-    fprintf(stderr, "pmg: restrict shape mismatch\n");
-    return;
-  }
-  dim3 g(cdiv(c.nx - 2, BX), cdiv(c.ny - 2, BY), c.nz - 2);
-  k_restrict2<<<xcd_blocks(g), dim3(BX, BY), 0, s>>>(
-      f.nx, f.ny, c.nx, c.ny, c.nz, a, b, ao, bo, pc, xg_of(g), ao32, bo32);
-  check_launch("restrict2");
+  restrict_launch<double, 2>(
+      f, c, RSrc<double, 2>{{a, b}, {ao, bo}, {ao32, bo32}}, pc, s);
 }
 
 enum : int {
@@ -1616,10 +1867,16 @@ enum : int {
   dPC, dPN, dPS, dPE, dPW, dPNE, dPNW, dPSE, dPSW
 };
 
-// One thread per coarse cell (ii, jj, kk) in 1..nc-1: the 8 fine points of
-// the cell, as VinterpPMG2.  ADD: xf += xdamp * value on fine interior
-// points (Vxaxpy over the interior); otherwise xf = value (the fine
-// boundary is zeroed separately).
+// The 8 fine points of coarse cell (ii, jj, kk) in 1..nc-1, as VinterpPMG2.
+// ADD: xf += xdamp * value on fine interior points (Vxaxpy over the
+// interior); otherwise xf = value (the fine boundary is zeroed separately).
+// A thread takes two i-adjacent cells: each P plane and coarse value comes
+// for both with one load, the four fine points of a row are read and written
+// with one each (39 memory instructions for two cells against 102).
+// xdamp: the device scalar, or the sum of the nblk (x.w0, x.y) partials of
+// the coarse matvec (mgcsd.cc:429-452), which every wavefront adds up by
+// itself (one-wavefront workgroups: no barrier between launch and result) or
+// every workgroup of four adds up together, in a fixed order.
 template <class T, bool ADD>
 __device__ __forceinline__ void interp_body(int nxc, int nyc, int nzc,
                                             int nxf, int nyf, int nzf,
@@ -1628,69 +1885,101 @@ __device__ __forceinline__ void interp_body(int nxc, int nyc, int nzc,
                                             T *__restrict__ xf,
                                             const double *xdamp,
                                             const double *part,
-                                            unsigned nblk, XG xg,
+                                            unsigned nblk, PR s,
                                             unsigned bid) {
-  int bx, by, bz;
-  const bool tok = xcd_tile_at(xg, bid, bx, by, bz);
-  const int ii = 1 + bx * BX + threadIdx.x;
-  const int jj = 1 + by * BY + threadIdx.y;
-  const int kk = 1 + bz;
-  // xdamp from the (x.w0, x.y) partials of the coarse matvec, summed by
-  // every block in the same fixed order (mgcsd.cc:429-452)
-  __shared__ double red[8];
-  __shared__ double dsh;
-  if (ADD && part) {
-    const int tid = threadIdx.x + threadIdx.y * BX;
-    double a = 0.0, c = 0.0;
-    for (unsigned q = tid; q < nblk; q += BX * BY) {
-      a += part[2 * (size_t)q];
-      c += part[2 * (size_t)q + 1];
-    }
-    a = block_sum<BX * BY>(a, red);
-    c = block_sum<BX * BY>(c, red);
-    if (tid == 0) dsh = c != 0.0 ? a / c : 0.0;
-    __syncthreads();
-  }
-  if (!tok || ii > nxc - 1 || jj > nyc - 1) return;
+  int m, row, plane;
+  __shared__ double red[2 * BY];
+  const bool live = pr_pair(s, bid, nyc - 1, m, row, plane);
+  if (!live) m = row = plane = 0;
+  const int ii = 1 + 2 * m, jj = 1 + row, kk = 1 + plane;
+  const bool both = ii + 1 <= nxc - 1;
   const size_t nc = (size_t)nxc * nyc * nzc;
   const size_t c0 = ix(nxc, nyc, ii, jj, kk);
   const size_t cx = 1, cy = nxc, cz = (size_t)nxc * nyc;
-#define PW(pl, o) pc[(size_t)(pl)*nc + c0 + (o)]
-#define XC(o) xc[c0 + (o)]
-  const T x000 = XC(0), x100 = XC(cx), x010 = XC(cy), x110 = XC(cx + cy),
-          x001 = XC(cz), x101 = XC(cx + cz), x011 = XC(cy + cz),
-          x111 = XC(cx + cy + cz);
-  T v[8];
-  v[0] = x000;
-  v[1] = PW(oPE, 0) * x000 + PW(oPW, cx) * x100;
-  v[2] = PW(oPN, 0) * x000 + PW(oPS, cy) * x010;
-  v[4] = PW(uPC, 0) * x000 + PW(dPC, cz) * x001;
-  v[3] = PW(oPNE, 0) * x000 + PW(oPNW, cx) * x100 + PW(oPSE, cy) * x010 +
-         PW(oPSW, cx + cy) * x110;
-  v[5] = PW(uPE, 0) * x000 + PW(uPW, cx) * x100 + PW(dPE, cz) * x001 +
-         PW(dPW, cx + cz) * x101;
-  v[6] = PW(uPN, 0) * x000 + PW(uPS, cy) * x010 + PW(dPN, cz) * x001 +
-         PW(dPS, cy + cz) * x011;
-  v[7] = +PW(uPNE, 0) * x000 + PW(uPNW, cx) * x100 + PW(uPSE, cy) * x010 +
-         PW(uPSW, cx + cy) * x110 + PW(dPNE, cz) * x001 +
-         PW(dPNW, cx + cz) * x101 + PW(dPSE, cy + cz) * x011 +
-         PW(dPSW, cx + cy + cz) * x111;
+  T x[4][4];  // coarse values of the rows (0, 0), (cy), (cz), (cy + cz)
+  ldn(xc + c0, x[0]);
+  ldn(xc + c0 + cy, x[1]);
+  ldn(xc + c0 + cz, x[2]);
+  ldn(xc + c0 + cy + cz, x[3]);
+  const size_t f0 = ix(nxf, nyf, 2 * ii - 1, 2 * jj - 1, 2 * kk - 1);
+  const size_t fy = nxf, fz = (size_t)nxf * nyf;
+  T old[4][4];  // fine rows (0, 0), (fy), (fz), (fy + fz)
+  if (ADD) {
+    ldn(xf + f0, old[0]);
+    ldn(xf + f0 + fy, old[1]);
+    ldn(xf + f0 + fz, old[2]);
+    ldn(xf + f0 + fy + fz, old[3]);
+  }
+  T w[27][2];
+#define PW(pl, o) ldn(pc + (size_t)(pl)*nc + c0 + (o), w[pl])
+  PW(oPE, 0), PW(oPW, cx);
+  PW(oPN, 0), PW(oPS, cy);
+  PW(uPC, 0), PW(dPC, cz);
+  PW(oPNE, 0), PW(oPNW, cx), PW(oPSE, cy), PW(oPSW, cx + cy);
+  PW(uPE, 0), PW(uPW, cx), PW(dPE, cz), PW(dPW, cx + cz);
+  PW(uPN, 0), PW(uPS, cy), PW(dPN, cz), PW(dPS, cy + cz);
+  PW(uPNE, 0), PW(uPNW, cx), PW(uPSE, cy), PW(uPSW, cx + cy);
+  PW(dPNE, cz), PW(dPNW, cx + cz), PW(dPSE, cy + cz), PW(dPSW, cx + cy + cz);
 #undef PW
-#undef XC
-  const int i = 2 * ii - 1, j = 2 * jj - 1, k = 2 * kk - 1;
   T damp = (T)0;
-  if (ADD) damp = (T)(part ? dsh : *xdamp);
-#pragma unroll
-  for (int q = 0; q < 8; q++) {
-    const int fi = i + (q & 1), fj = j + ((q >> 1) & 1), fk = k + (q >> 2);
-    const size_t p = ix(nxf, nyf, fi, fj, fk);
-    if (ADD) {
-      if (fi >= 2 && fi <= nxf - 1 && fj >= 2 && fj <= nyf - 1 && fk >= 2 &&
-          fk <= nzf - 1)
-        xf[p] += damp * v[q];
+  if (ADD) {
+    if (part) {
+      double a = 0.0, c = 0.0;
+      for (unsigned q = threadIdx.y * BX + threadIdx.x; q < nblk;
+           q += BX * s.rows) {
+        double v[2];
+        ldn(part + 2 * (size_t)q, v);
+        a += v[0], c += v[1];
+      }
+      a = wave_sum(a), c = wave_sum(c);
+      if (s.rows > 1) {
+        if (threadIdx.x == 0)
+          red[2 * threadIdx.y] = a, red[2 * threadIdx.y + 1] = c;
+        __syncthreads();
+        a = (red[0] + red[2]) + (red[4] + red[6]);
+        c = (red[1] + red[3]) + (red[5] + red[7]);
+      }
+      damp = (T)(c != 0.0 ? a / c : 0.0);
     } else {
-      xf[p] = v[q];
+      damp = (T)*xdamp;
     }
+  }
+  T v[4][4];  // fine rows as above; the cell e gives the points 2 e, 2 e + 1
+#pragma unroll
+  for (int e = 0; e < 2; e++) {
+    const T x000 = x[0][e], x100 = x[0][e + 1], x010 = x[1][e],
+            x110 = x[1][e + 1], x001 = x[2][e], x101 = x[2][e + 1],
+            x011 = x[3][e], x111 = x[3][e + 1];
+    v[0][2 * e] = x000;
+    v[0][2 * e + 1] = w[oPE][e] * x000 + w[oPW][e] * x100;
+    v[1][2 * e] = w[oPN][e] * x000 + w[oPS][e] * x010;
+    v[2][2 * e] = w[uPC][e] * x000 + w[dPC][e] * x001;
+    v[1][2 * e + 1] = w[oPNE][e] * x000 + w[oPNW][e] * x100 +
+                      w[oPSE][e] * x010 + w[oPSW][e] * x110;
+    v[2][2 * e + 1] = w[uPE][e] * x000 + w[uPW][e] * x100 + w[dPE][e] * x001 +
+                      w[dPW][e] * x101;
+    v[3][2 * e] = w[uPN][e] * x000 + w[uPS][e] * x010 + w[dPN][e] * x001 +
+                  w[dPS][e] * x011;
+    v[3][2 * e + 1] = +w[uPNE][e] * x000 + w[uPNW][e] * x100 +
+                      w[uPSE][e] * x010 + w[uPSW][e] * x110 +
+                      w[dPNE][e] * x001 + w[dPNW][e] * x101 +
+                      w[dPSE][e] * x011 + w[dPSW][e] * x111;
+  }
+  if (!live) return;
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    // rows on the fine boundary (j = 1 or k = 1) are left alone, and so is
+    // the point i = 1, which gets its own value back
+    if (ADD && ((!(r & 1) && jj == 1) || (!(r & 2) && kk == 1))) continue;
+    T o[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) o[q] = ADD ? old[r][q] + damp * v[r][q] : v[r][q];
+    if (ADD && ii == 1) o[0] = old[r][0];
+    T *g = xf + f0 + ((r & 1) ? fy : 0) + ((r & 2) ? fz : 0);
+    if (both)
+      stn(g, o);
+    else
+      g[0] = o[0], g[1] = o[1];
   }
 }
 
@@ -1702,44 +1991,39 @@ __global__ __launch_bounds__(256) void k_interp(int nxc, int nyc, int nzc,
                                                 T *__restrict__ xf,
                                                 const double *xdamp,
                                                 const double *part,
-                                                unsigned nblk, XG xg) {
+                                                unsigned nblk, PR s) {
   interp_body<T, ADD>(nxc, nyc, nzc, nxf, nyf, nzf, xc, pc, xf, xdamp, part,
-                      nblk, xg, blockIdx.x);
+                      nblk, s, blockIdx.x);
+}
+
+template <class T, bool ADD>
+static void interp_launch(const Dim &c, const Dim &f, const T *xc, const T *pc,
+                          T *xf, const double *xdamp, const double *part,
+                          unsigned nblk, hipStream_t s) {
+  if (f.nx != 2 * c.nx - 1 || f.ny != 2 * c.ny - 1 || f.nz != 2 * c.nz - 1) {
+    fprintf(stderr, "pmg: interp shape mismatch\n");
+    return;
+  }
+  const PR sh = pr_shape(c.nx - 1, c.ny - 1, c.nz - 1);
+  k_interp<T, ADD><<<sh.nblk, dim3(BX, sh.rows), 0, s>>>(
+      c.nx, c.ny, c.nz, f.nx, f.ny, f.nz, xc, pc, xf, xdamp, part, nblk, sh);
+  if constexpr (!ADD && sizeof(T) == 8) fbound00(f, (double *)xf, s);
+  check_launch("interp");
 }
 
 template <class T>
 void interp(const Dim &c, const Dim &f, const T *xc, const T *pc, T *xf,
             const double *xdamp, hipStream_t s) {
-  if (f.nx != 2 * c.nx - 1 || f.ny != 2 * c.ny - 1 || f.nz != 2 * c.nz - 1) {
-    fprintf(stderr, "pmg: interp shape mismatch\n");
-    return;
-  }
-  dim3 g(cdiv(c.nx - 1, BX), cdiv(c.ny - 1, BY), c.nz - 1);
-  if (xdamp) {
-    k_interp<T, true><<<xcd_blocks(g), dim3(BX, BY), 0, s>>>(c.nx, c.ny, c.nz, f.nx, f.ny,
-                                                 f.nz, xc, pc, xf, xdamp,
-                                                 nullptr, 0u, xg_of(g));
-  } else {
-    k_interp<T, false><<<xcd_blocks(g), dim3(BX, BY), 0, s>>>(c.nx, c.ny, c.nz, f.nx,
-                                                  f.ny, f.nz, xc, pc, xf,
-                                                  nullptr, nullptr, 0u, xg_of(g));
-    if constexpr (sizeof(T) == 8) fbound00(f, (double *)xf, s);
-  }
-  check_launch("interp");
+  if (xdamp)
+    interp_launch<T, true>(c, f, xc, pc, xf, xdamp, nullptr, 0u, s);
+  else
+    interp_launch<T, false>(c, f, xc, pc, xf, nullptr, nullptr, 0u, s);
 }
 
 template <class T>
 void interp_damped(const Dim &c, const Dim &f, const T *xc, const T *pc,
                    T *xf, const double *part, unsigned nblk, hipStream_t s) {
-  if (f.nx != 2 * c.nx - 1 || f.ny != 2 * c.ny - 1 || f.nz != 2 * c.nz - 1) {
-    fprintf(stderr, "pmg: interp shape mismatch\n");
-    return;
-  }
-  dim3 g(cdiv(c.nx - 1, BX), cdiv(c.ny - 1, BY), c.nz - 1);
-  k_interp<T, true><<<xcd_blocks(g), dim3(BX, BY), 0, s>>>(c.nx, c.ny, c.nz, f.nx, f.ny,
-                                               f.nz, xc, pc, xf, nullptr, part,
-                                               nblk, xg_of(g));
-  check_launch("interp_damped");
+  interp_launch<T, true>(c, f, xc, pc, xf, nullptr, part, nblk, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1827,19 +2111,8 @@ void stop_diff(const Dim &d, int kind, double *tru, const double *u,
 template <class T>
 void dot_energy(const Dim &d, int numdia, const T *ac, const T *cc,
                 const T *w, T *y, const Red &red, hipStream_t s) {
-  const int kc = kchunk(d);
-  dim3 g(cdiv(d.nx - 2, BX), cdiv(d.ny - 2, BY), cdiv(d.nz - 2, kc));
-  dim3 b(BX, BY);
-  if (numdia == 7)
-    k_matvec_dots<T, 7><<<xcd_blocks(g), b, 0, s>>>(d.nx, d.ny, d.nz, ac, cc,
-                                                    w, w, y, red, 1, kc,
-                                                    xg_of(g));
-  else
-    k_matvec_dots<T, 27><<<xcd_blocks(g), b, 0, s>>>(d.nx, d.ny, d.nz, ac, cc,
-                                                     w, w, y, red, 1, kc,
-                                                     xg_of(g));
-  red_final<2, 2>(red, dim3(xcd_blocks(g)), s);
-  check_launch("dot_energy");
+  const unsigned nb = matvec_launch<T>(d, numdia, ac, cc, w, w, y, &red, s);
+  red_final<2, 2>(red, dim3(nb), s);
 }
 
 // Vextrac (matvecd.cc:997-1008): coarse interior by injection.
@@ -3210,13 +3483,21 @@ struct A_res {
   XG xg;
   unsigned nblk;
   const T *dg;
+  P27 s27;
 };
-template <class T, class TO, int ND>
+template <class T, class TO>
 __global__ __launch_bounds__(256) void kb_resid(const GTab<A_res<T, TO>> t) {
   const A_res<T, TO> &a = t.a[blockIdx.y];
   if (blockIdx.x >= a.nblk) return;
-  resid_body<T, TO, ND>(a.nx, a.ny, a.nz, a.ac, a.cc, a.fc, a.x, a.r, a.rd,
-                        a.do_red, a.kc, a.xg, blockIdx.x);
+  resid_body<T, TO>(a.nx, a.ny, a.nz, a.ac, a.cc, a.fc, a.x, a.r, a.rd,
+                    a.do_red, a.kc, a.xg, blockIdx.x);
+}
+template <class T, class TO>
+__global__ __launch_bounds__(256) void kb_resid27(const GTab<A_res<T, TO>> t) {
+  const A_res<T, TO> &a = t.a[blockIdx.y];
+  if (blockIdx.x >= a.nblk) return;
+  resid27_body<T, TO>(a.nx, a.ny, a.nz, a.ac, a.cc, a.fc, a.x, a.r, a.rd,
+                      a.do_red, a.s27, blockIdx.x);
 }
 // 7-point levels with the precomputed diagonal: k_resid7m's march (xg holds
 // its tile counts)
@@ -3249,11 +3530,15 @@ void g_resid(const GResid<T, TO> *j, int n, hipStream_t s) {
     const Dim &d = j[q].d;
     const bool red = j[q].red != nullptr;
     const T *dg = j[q].numdia == 7 && resid7m_fits(d) ? j[q].dg : nullptr;
-    int kc;
-    XG xg;
+    int kc = 0;
+    XG xg{};
     unsigned nblk;
+    P27 s27{};
     if (dg) {
       nblk = resid7m_shape(d, kc, xg.gx, xg.gy, xg.gz);
+    } else if (j[q].numdia == 27) {
+      s27 = p27_shape(d);
+      nblk = s27.nblk;
     } else {
       kc = kchunk(d, red ? 40 : 80);
       const dim3 g(cdiv(d.nx - 2, BX), cdiv(d.ny - 2, BY),
@@ -3263,11 +3548,15 @@ void g_resid(const GResid<T, TO> *j, int n, hipStream_t s) {
     a[q] = A_res<T, TO>{d.nx,    d.ny,    d.nz,   j[q].ac,
                         j[q].cc, j[q].fc, j[q].x, j[q].r,
                         red ? *j[q].red : Red{}, red ? 1 : 0, kc,
-                        xg,      nblk,    dg};
+                        xg,      nblk,    dg,     s27};
   }
-  // variant key: 27 (27-point), 7 (7-point), 8 (7-point with dg)
+  // variant key: 7 (7-point), 8 (7-point with dg), 26 + wavefronts per
+  // workgroup (27-point)
   g_split<A_res<T, TO>>(
-      n, [&](int q) { return j[q].numdia == 7 && a[q].dg ? 8 : j[q].numdia; },
+      n,
+      [&](int q) {
+        return j[q].numdia == 7 ? (a[q].dg ? 8 : 7) : 26 + a[q].s27.rows;
+      },
       [&](int q) { return a[q]; },
       [&](const GTab<A_res<T, TO>> &t, int m, int key) {
         unsigned mx = 0;
@@ -3276,9 +3565,9 @@ void g_resid(const GResid<T, TO> *j, int n, hipStream_t s) {
         if (key == 8)
           kb_resid7m<T, TO><<<grid, dim3(RM_TX, RM_TY), 0, s>>>(t);
         else if (key == 7)
-          kb_resid<T, TO, 7><<<grid, b, 0, s>>>(t);
+          kb_resid<T, TO><<<grid, b, 0, s>>>(t);
         else
-          kb_resid<T, TO, 27><<<grid, b, 0, s>>>(t);
+          kb_resid27<T, TO><<<grid, dim3(BX, key - 26), 0, s>>>(t);
       });
   std::vector<int> rq;
   for (int q = 0; q < n; q++)
@@ -3298,18 +3587,16 @@ void g_resid(const GResid<T, TO> *j, int n, hipStream_t s) {
 template <class T>
 struct A_rs {
   int nxf, nyf, nxc, nyc, nzc;
-  const T *xin;
-  T *xout;
+  RSrc<T, 1> io;
   const T *pc;
-  XG xg;
-  unsigned nblk;
+  PR sh;
 };
 template <class T>
 __global__ __launch_bounds__(256) void kb_restrict(const GTab<A_rs<T>> t) {
   const A_rs<T> &a = t.a[blockIdx.y];
-  if (blockIdx.x >= a.nblk) return;
-  restrict_body<T>(a.nxf, a.nyf, a.nxc, a.nyc, a.nzc, a.xin, a.xout, a.pc,
-                   a.xg, nullptr, blockIdx.x);
+  if (blockIdx.x >= a.sh.nblk) return;
+  restrict_body<T, 1>(a.nxf, a.nyf, a.nxc, a.nyc, a.nzc, a.io, a.pc, a.sh,
+                      blockIdx.x);
 }
 
 template <class T>
@@ -3325,17 +3612,21 @@ void g_restrict(const GRestrict<T> *j, int n, hipStream_t s) {
     ok.push_back(q);
   }
   g_split<A_rs<T>>(
-      (int)ok.size(), [&](int) { return 0; },
+      (int)ok.size(),
+      [&](int q) {
+        const Dim &c = j[ok[q]].c;
+        return pr_shape(c.nx - 2, c.ny - 2, c.nz - 2).rows;
+      },
       [&](int q) {
         const GRestrict<T> &J = j[ok[q]];
-        const dim3 g(cdiv(J.c.nx - 2, BX), cdiv(J.c.ny - 2, BY), J.c.nz - 2);
-        return A_rs<T>{J.f.nx, J.f.ny, J.c.nx,   J.c.ny,   J.c.nz,
-                       J.xin,  J.xout, J.pc,     xg_of(g), xcd_blocks(g)};
+        return A_rs<T>{J.f.nx, J.f.ny, J.c.nx, J.c.ny, J.c.nz,
+                       RSrc<T, 1>{{J.xin}, {J.xout}, {nullptr}}, J.pc,
+                       pr_shape(J.c.nx - 2, J.c.ny - 2, J.c.nz - 2)};
       },
-      [&](const GTab<A_rs<T>> &t, int m, int) {
+      [&](const GTab<A_rs<T>> &t, int m, int rows) {
         unsigned mx = 0;
-        for (int q = 0; q < m; q++) mx = std::max(mx, t.a[q].nblk);
-        kb_restrict<T><<<dim3(mx, m), dim3(BX, BY), 0, s>>>(t);
+        for (int q = 0; q < m; q++) mx = std::max(mx, t.a[q].sh.nblk);
+        kb_restrict<T><<<dim3(mx, m), dim3(BX, rows), 0, s>>>(t);
       });
   check_launch("g_restrict");
 }
@@ -3346,42 +3637,43 @@ struct A_mv {
   const T *ac, *cc, *x, *w0;
   T *y;
   Red rd;
-  int kc;
-  XG xg;
-  unsigned nblk;
+  P27 s27;
 };
-template <class T, int ND>
-__global__ __launch_bounds__(256) void kb_matvec_dots(const GTab<A_mv<T>> t) {
+template <class T>
+__global__ __launch_bounds__(256) void kb_matvec27(const GTab<A_mv<T>> t) {
   const A_mv<T> &a = t.a[blockIdx.y];
-  if (blockIdx.x >= a.nblk) return;
-  matvec_dots_body<T, ND>(a.nx, a.ny, a.nz, a.ac, a.cc, a.x, a.w0, a.y, a.rd,
-                          1, a.kc, a.xg, blockIdx.x);
+  if (blockIdx.x >= a.s27.nblk) return;
+  matvec27_body<T>(a.nx, a.ny, a.nz, a.ac, a.cc, a.x, a.w0, a.y, a.rd, 1,
+                   a.s27, blockIdx.x);
 }
 
 template <class T>
 void g_matvec_dots_part(const GMatvec<T> *j, int n, unsigned *nb,
                         hipStream_t s) {
-  std::vector<A_mv<T>> a(n);
-  for (int q = 0; q < n; q++) {  // the launch shape of matvec_dots_part
-    const Dim &d = j[q].d;
-    const int kc = kchunk(d);
-    const dim3 g(cdiv(d.nx - 2, BX), cdiv(d.ny - 2, BY), cdiv(d.nz - 2, kc));
-    Red rd;
-    rd.part = j[q].part;
-    a[q] = A_mv<T>{d.nx,   d.ny,    d.nz, j[q].ac,  j[q].cc,      j[q].x,
-                   j[q].w0, j[q].y, rd,   kc,       xg_of(g),     xcd_blocks(g)};
-    nb[q] = a[q].nblk;
+  std::vector<int> ok;  // 27-point levels; others run alone
+  for (int q = 0; q < n; q++) {
+    if (j[q].numdia == 27) {
+      ok.push_back(q);
+      nb[q] = p27_shape(j[q].d).nblk;
+    } else {
+      nb[q] = matvec_dots_part<T>(j[q].d, j[q].numdia, j[q].ac, j[q].cc,
+                                  j[q].x, j[q].w0, j[q].y, j[q].part, s);
+    }
   }
   g_split<A_mv<T>>(
-      n, [&](int q) { return j[q].numdia; }, [&](int q) { return a[q]; },
-      [&](const GTab<A_mv<T>> &t, int m, int nd) {
+      (int)ok.size(),
+      [&](int q) { return p27_shape(j[ok[q]].d).rows; },
+      [&](int q) {
+        const GMatvec<T> &J = j[ok[q]];
+        Red rd;
+        rd.part = J.part;
+        return A_mv<T>{J.d.nx, J.d.ny, J.d.nz, J.ac, J.cc,
+                       J.x,    J.w0,   J.y,    rd,   p27_shape(J.d)};
+      },
+      [&](const GTab<A_mv<T>> &t, int m, int rows) {
         unsigned mx = 0;
-        for (int q = 0; q < m; q++) mx = std::max(mx, t.a[q].nblk);
-        const dim3 grid(mx, m), b(BX, BY);
-        if (nd == 7)
-          kb_matvec_dots<T, 7><<<grid, b, 0, s>>>(t);
-        else
-          kb_matvec_dots<T, 27><<<grid, b, 0, s>>>(t);
+        for (int q = 0; q < m; q++) mx = std::max(mx, t.a[q].s27.nblk);
+        kb_matvec27<T><<<dim3(mx, m), dim3(BX, rows), 0, s>>>(t);
       });
   check_launch("g_matvec_dots");
 }
@@ -3393,15 +3685,14 @@ struct A_ip {
   T *xf;
   const double *part;
   unsigned npart;
-  XG xg;
-  unsigned nblk;
+  PR sh;
 };
 template <class T>
 __global__ __launch_bounds__(256) void kb_interp_damped(const GTab<A_ip<T>> t) {
   const A_ip<T> &a = t.a[blockIdx.y];
-  if (blockIdx.x >= a.nblk) return;
+  if (blockIdx.x >= a.sh.nblk) return;
   interp_body<T, true>(a.nxc, a.nyc, a.nzc, a.nxf, a.nyf, a.nzf, a.xc, a.pc,
-                       a.xf, nullptr, a.part, a.npart, a.xg, blockIdx.x);
+                       a.xf, nullptr, a.part, a.npart, a.sh, blockIdx.x);
 }
 
 template <class T>
@@ -3416,18 +3707,21 @@ void g_interp_damped(const GInterp<T> *j, int n, hipStream_t s) {
     ok.push_back(q);
   }
   g_split<A_ip<T>>(
-      (int)ok.size(), [&](int) { return 0; },
+      (int)ok.size(),
+      [&](int q) {
+        const Dim &c = j[ok[q]].c;
+        return pr_shape(c.nx - 1, c.ny - 1, c.nz - 1).rows;
+      },
       [&](int q) {
         const GInterp<T> &J = j[ok[q]];
-        const dim3 g(cdiv(J.c.nx - 1, BX), cdiv(J.c.ny - 1, BY), J.c.nz - 1);
         return A_ip<T>{J.c.nx, J.c.ny, J.c.nz, J.f.nx, J.f.ny,
                        J.f.nz, J.xc,   J.pc,   J.xf,   J.part,
-                       J.nblk, xg_of(g), xcd_blocks(g)};
+                       J.nblk, pr_shape(J.c.nx - 1, J.c.ny - 1, J.c.nz - 1)};
       },
-      [&](const GTab<A_ip<T>> &t, int m, int) {
+      [&](const GTab<A_ip<T>> &t, int m, int rows) {
         unsigned mx = 0;
-        for (int q = 0; q < m; q++) mx = std::max(mx, t.a[q].nblk);
-        kb_interp_damped<T><<<dim3(mx, m), dim3(BX, BY), 0, s>>>(t);
+        for (int q = 0; q < m; q++) mx = std::max(mx, t.a[q].sh.nblk);
+        kb_interp_damped<T><<<dim3(mx, m), dim3(BX, rows), 0, s>>>(t);
       });
   check_launch("g_interp_damped");
 }
