@@ -135,10 +135,15 @@ void nrm1(const Dim &d, const T *x, const Red &red, hipStream_t s);
 
 // ---- coarsest-level CG (pmgc/cgd.cc:60-124), one workgroup, FP64 ----
 // Returns false if the level is too large for the single-workgroup kernel.
+// damp (may be null): receives the Hackbusch-Reusken factor (x.f) / (x.A x)
+// of the solution where the row-segment kernel serves (cg_rows_fits); the
+// single launcher returns whether it did.
 bool cg_fits(const Dim &d);
+bool cg_rows_fits(const Dim &d, int numdia);
 template <class T>
-void cg_single(const Dim &d, int numdia, const double *ac, const double *cc,
-               const T *f, T *x, int itmax, double errtol, hipStream_t s);
+bool cg_single(const Dim &d, int numdia, const double *ac, const double *cc,
+               const T *f, T *x, int itmax, double errtol, hipStream_t s,
+               double *damp = nullptr);
 
 // ---- the class-style solver (PBE_pmgc_class.h:1070-1133,
 // CG_Solver.h:45-242) ----
@@ -148,7 +153,8 @@ void cg_single(const Dim &d, int numdia, const double *ac, const double *cc,
 bool cg_class_fits(const Dim &d, int numdia);
 template <class T>
 void cg_class(const Dim &d, int numdia, const double *ac, const double *cc,
-              const T *f, T *x, int itmax, double thresh, hipStream_t s);
+              const T *f, T *x, int itmax, double thresh, hipStream_t s,
+              double *damp = nullptr);
 // red.out[0] = x.y over the interior (deterministic order)
 void dot_interior(const Dim &d, const double *x, const double *y,
                   const Red &red, hipStream_t s);
@@ -250,6 +256,29 @@ int pbe_assemble(int n, double h, double ionic, int natoms,
                  hipStream_t s, double eps_in = 2.0, double eps_out = 78.54,
                  double shell = 2.0);
 
+// ---- the two coarsest levels of a cycle (pmg_bottom.hip) ----
+// Where the coarsest level takes the row-segment CG and the level above it
+// is a 27-point level small enough for one compute unit's LDS, the cycle's
+// work between entering and leaving that level runs in three launches:
+// bottom_down (nu sweeps from zero, residual, its restriction), the CG (with
+// its damping factor), bottom_up (the damped prolongation, nu sweeps, the
+// damping factor of the next prolongation), each one workgroup per problem.
+template <class T>
+struct GBottom {
+  Dim d, dc;                  // the level and the coarsest one
+  const T *ac, *cc, *f, *pc;  // operator and right-hand side; P of dc
+  T *x, *fc;                  // the level's iterate; the coarsest rhs
+  const T *xc;                // the coarsest solution
+  double *damp;  // in: factor of xc; out: of x (device scalar)
+};
+template <class T>
+bool bottom_fits(const Dim &d, int numdia, const Dim &dc, int numdiac);
+template <class T>
+void bottom_down(const GBottom<T> *j, int n, int nu, hipStream_t s);
+template <class T>
+void bottom_up(const GBottom<T> *j, int n, int nu, int iadjoint,
+               hipStream_t s);
+
 // ---- grouped launches (the serving loop): the same step for up to GMAX
 // independent problems per launch, each problem running exactly the
 // workgroups and arithmetic of its own launch (bit-identical results).
@@ -302,11 +331,11 @@ template <class T>
 void g_matvec_dots_part(const GMatvec<T> *j, int n, unsigned *nb,
                         hipStream_t s);
 template <class T>
-struct GInterp {  // interp_damped()
+struct GInterp {  // interp_damped(); damp: xdamp itself, part then null
   Dim c, f;
   const T *xc, *pc;
   T *xf;
-  const double *part;
+  const double *damp, *part;
   unsigned nblk;
 };
 template <class T>
@@ -318,6 +347,7 @@ struct GCoarse {  // cg_single()
   const double *ac, *cc;
   const T *f;
   T *x;
+  double *damp;
 };
 template <class T>
 void g_cg(const GCoarse<T> *j, int n, int itmax, double errtol,

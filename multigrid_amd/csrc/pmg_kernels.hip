@@ -16,18 +16,12 @@
 #include <cmath>
 #include <cstdio>
 
+#include "pmg_device.h"
 #include "pmg_internal.h"
 
 namespace pmg {
 
 constexpr int BX = 64, BY = 4, KCH = 4;
-
-__host__ __device__ inline size_t ix(int nx, int ny, int i, int j, int k) {
-  return ((size_t)(k - 1) * (size_t)ny + (size_t)(j - 1)) * (size_t)nx +
-         (size_t)(i - 1);
-}
-
-inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 // XCD-aware tiling.  Workgroups are dispatched round-robin over the eight
 // XCDs (workgroup b runs on XCD b % 8), each with its own L2.  Stencil
@@ -69,34 +63,6 @@ static void check_launch(const char *what) {
 // ---------------------------------------------------------------------------
 // Wavefront and block reductions (deterministic for a fixed block shape)
 // ---------------------------------------------------------------------------
-// One DPP lane move of a double (both 32-bit halves with the same control);
-// lanes without a source, or in rows outside ROWMASK, read 0.
-template <int CTRL, int ROWMASK>
-__device__ inline double dpp_f64(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL,
-                                             ROWMASK, 0xF, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL,
-                                             ROWMASK, 0xF, true);
-  return __hiloint2double(hi, lo);
-}
-
-// Sum over the 64 lanes of a wavefront, returned in every lane.  Row
-// prefix sums by row_shr 1, 2, 4, 8 leave each 16-lane row's total in its
-// lane 15; row_bcast15 and row_bcast31 fold the four rows into lane 63,
-// which is then read out.  All moves stay in the VALU (no LDS round trips
-// as with lane shuffles), and the order of additions is fixed.
-__device__ inline double wave_sum(double v) {
-  v += dpp_f64<0x111, 0xF>(v);  // row_shr:1
-  v += dpp_f64<0x112, 0xF>(v);  // row_shr:2
-  v += dpp_f64<0x114, 0xF>(v);  // row_shr:4
-  v += dpp_f64<0x118, 0xF>(v);  // row_shr:8
-  v += dpp_f64<0x142, 0xA>(v);  // row_bcast:15 into rows 1, 3
-  v += dpp_f64<0x143, 0xC>(v);  // row_bcast:31 into rows 2, 3
-  const int lo = __builtin_amdgcn_readlane(__double2loint(v), 63);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), 63);
-  return __hiloint2double(hi, lo);
-}
-
 template <int NT>
 __device__ inline double block_sum(double v, double *red) {
   const int tid = threadIdx.x + threadIdx.y * blockDim.x;
@@ -578,179 +544,6 @@ void gs7(const Dim &d, const T *ac, const T *cc, const T *fc, T *x,
 // is pair m-1's second point (the previous lane, or lane 63 of the previous
 // segment for lane 0); its east neighbour is pair m+1's first point.
 constexpr int ROWS_MAXN = 128 * 4 + 1;
-// Two or four consecutive elements by one load each (two for four doubles),
-// aligned to the element only.
-typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
-typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));
-__device__ __forceinline__ void ldn(const float *p, float (&v)[2]) {
-  const f32x2u t = *(const f32x2u *)p;
-  v[0] = t.x, v[1] = t.y;
-}
-__device__ __forceinline__ void ldn(const double *p, double (&v)[2]) {
-  const f64x2u t = *(const f64x2u *)p;
-  v[0] = t.x, v[1] = t.y;
-}
-__device__ __forceinline__ void ldn(const float *p, float (&v)[4]) {
-  const f32x4u t = *(const f32x4u *)p;
-  v[0] = t.x, v[1] = t.y, v[2] = t.z, v[3] = t.w;
-}
-__device__ __forceinline__ void ldn(const double *p, double (&v)[4]) {
-  const f64x2u t = *(const f64x2u *)p, u = *(const f64x2u *)(p + 2);
-  v[0] = t.x, v[1] = t.y, v[2] = u.x, v[3] = u.y;
-}
-__device__ __forceinline__ void stn(float *p, const float (&v)[4]) {
-  f32x4u t;
-  t.x = v[0], t.y = v[1], t.z = v[2], t.w = v[3];
-  *(f32x4u *)p = t;
-}
-__device__ __forceinline__ void stn(double *p, const double (&v)[4]) {
-  f64x2u t, u;
-  t.x = v[0], t.y = v[1], u.x = v[2], u.y = v[3];
-  *(f64x2u *)p = t;
-  *(f64x2u *)(p + 2) = u;
-}
-// Element di of a row whose first element is base, for the lane `off` bytes
-// into the row: the base is the same for the whole wavefront (a scalar
-// address) and the lane part stays one 32-bit offset for every array.
-template <class T>
-__device__ __forceinline__ const T *lane_at(const T *base, int di,
-                                            unsigned off) {
-  return (const T *)((const char *)(base + di) + off);
-}
-
-// The operands of a pair of i-adjacent points (i0, i0 + 1) of a 27-point
-// level (gsd.cc:160-211, matvecd.cc:137-170), as loaded.  Every coupling
-// comes for both points with one two-element load and every neighbouring row
-// of x with one four-element load (i0 - 1 .. i0 + 2): 37 loads of a pair
-// against 106 scalar ones.  The kernels on 27-point levels were bound by the
-// rate at which a compute unit takes vector memory instructions, not by
-// bytes (MI355X, the sweeps per paired launch, scalar loads -> these: 145^3
-// FP32 56 -> 44 us, 81^3 FP32 11.2 -> 8.4, FP64 16.5 -> 12.2, 33^3 and 17^3
-// FP64 8.2 -> 5.8 us; the same sums in the same order).  The four-element
-// loads of the last pair of the grid's last row reach one element past the
-// end of x, whose value no sum uses: every x array has that element
-// (allocations are padded).
-template <class T>
-struct G27C {          // couplings, the right-hand side, the diagonal's parts
-  T cN[2], cS[2];      // oN(p), oN(p - sy)
-  T cE[2], cW;         // oE(p) of both points, oE(p - 1) of the first
-  T c[4][2];           // oNE(p), oNW(p), oNW(p + 1 - sy), oNE(p - 1 - sy)
-  T cu[9][2], cd[9][2];
-  T oC[2], cc[2];
-};
-template <class T>
-struct G27X {
-  T xN[4], xS[4];        // x of rows j + 1, j - 1 in the own plane
-  T xu[3][4], xd[3][4];  // rows j, j + 1, j - 1 of the planes above, below
-};
-// A = ac + base, cc: the arrays at an index `base` that is the same for the
-// whole wavefront (a row or a plane); the pair's first point lies off bytes
-// further.  PL: the planes above and below are wanted (else they count as
-// zero and are not loaded).
-template <bool PL, class T>
-__device__ __forceinline__ void g27_couplings(const T *__restrict__ A,
-                                              const T *__restrict__ cc,
-                                              size_t n, long long sy,
-                                              long long sz, unsigned off,
-                                              G27C<T> &r) {
-  auto at = [&](int pl, long long d) {
-    return lane_at(A + (long long)pl * (long long)n + d, 0, off);
-  };
-  ldn(at(2, 0), r.cN);
-  ldn(at(2, -sy), r.cS);
-  ldn(at(1, 0), r.cE);
-  r.cW = *at(1, -1);
-  ldn(at(4, 0), r.c[0]);
-  ldn(at(5, 0), r.c[1]);
-  ldn(at(5, 1 - sy), r.c[2]);
-  ldn(at(4, -1 - sy), r.c[3]);
-  // planes uC, uN, uS, uE, uW, uNE, uNW, uSE, uSW of the plane above
-  constexpr int pu[9] = {3, 8, 9, 6, 7, 10, 11, 12, 13};
-  // the plane below couples through the mirrored plane of the neighbour
-  constexpr int pd[9] = {3, 9, 8, 7, 6, 13, 12, 11, 10};
-  const long long du[9] = {0,       sy,      -sy,    1,      -1,
-                           1 + sy, -1 + sy, 1 - sy, -1 - sy};
-  if constexpr (PL) {
-#pragma unroll
-    for (int m = 0; m < 9; m++) {
-      ldn(at(pu[m], 0), r.cu[m]);
-      ldn(at(pd[m], du[m] - sz), r.cd[m]);
-    }
-  } else {
-#pragma unroll
-    for (int m = 0; m < 9; m++)
-      r.cu[m][0] = r.cu[m][1] = r.cd[m][0] = r.cd[m][1] = (T)0;
-  }
-  ldn(at(0, 0), r.oC);
-  ldn(lane_at(cc, 0, off), r.cc);
-}
-// The neighbour rows from three arrays by their offset (dy, dz): xN (dy odd,
-// dz = 0), xU (dy = 0, dz odd), xNU (dy and dz odd), each at the base.
-template <bool PL, class T>
-__device__ __forceinline__ void g27_rows(const T *xN, const T *xU,
-                                         const T *xNU, long long sy,
-                                         long long sz, unsigned off,
-                                         G27X<T> &r) {
-  ldn(lane_at(xN + sy, -1, off), r.xN);
-  ldn(lane_at(xN - sy, -1, off), r.xS);
-  if constexpr (PL) {
-    ldn(lane_at(xU + sz, -1, off), r.xu[0]);
-    ldn(lane_at(xNU + sy + sz, -1, off), r.xu[1]);
-    ldn(lane_at(xNU - sy + sz, -1, off), r.xu[2]);
-    ldn(lane_at(xU - sz, -1, off), r.xd[0]);
-    ldn(lane_at(xNU + sy - sz, -1, off), r.xd[1]);
-    ldn(lane_at(xNU - sy - sz, -1, off), r.xd[2]);
-  } else {
-#pragma unroll
-    for (int m = 0; m < 12; m++) r.xu[m / 4][m % 4] = r.xd[m / 4][m % 4] = (T)0;
-  }
-}
-
-// The terms of one point that do not involve the two in-row neighbours,
-// summed in the reference's order as far as they go.
-template <class T>
-struct G27Part {
-  T a;             // oN(p) x(p+sy) + oN(p-sy) x(p-sy): the first two terms
-  T cE, cW;
-  T c[4], xv[4];   // the four in-plane terms after the in-row ones
-  T u, dd, dg;     // upper and lower plane sums, oC + cc
-};
-// Point s (0, 1) of the pair; zN: the rows j +- 1 of the own plane count as
-// zero.
-template <class T, int s>
-__device__ __forceinline__ G27Part<T> g27_part(const G27C<T> &r,
-                                               const G27X<T> &x, bool zN) {
-  auto Z = [](T v, bool z) -> T { return z ? (T)0 : v; };
-  G27Part<T> g;
-  g.a = r.cN[s] * Z(x.xN[s + 1], zN) + r.cS[s] * Z(x.xS[s + 1], zN);
-  g.cE = r.cE[s];
-  g.cW = s ? r.cE[0] : r.cW;
-  const T xv[4] = {x.xN[s + 2], x.xN[s], x.xS[s + 2], x.xS[s]};
-#pragma unroll
-  for (int m = 0; m < 4; m++) g.c[m] = r.c[m][s], g.xv[m] = Z(xv[m], zN);
-  // terms C, N, S, E, W, NE, NW, SE, SW: the row of the plane and the place
-  // in it
-  constexpr int tr[9] = {0, 1, 2, 0, 0, 1, 1, 2, 2};
-  constexpr int te[9] = {1, 1, 1, 2, 0, 2, 0, 2, 0};
-  T u = r.cu[0][s] * x.xu[0][s + 1];
-#pragma unroll
-  for (int m = 1; m < 9; m++) u += r.cu[m][s] * x.xu[tr[m]][s + te[m]];
-  T dd = r.cd[0][s] * x.xd[0][s + 1];
-#pragma unroll
-  for (int m = 1; m < 9; m++) dd += r.cd[m][s] * x.xd[tr[m]][s + te[m]];
-  g.u = u;
-  g.dd = dd;
-  g.dg = r.oC[s] + r.cc[s];
-  return g;
-}
-// The in-plane sum from the part and the in-row neighbours xw, xe.
-template <class T>
-__device__ __forceinline__ T g27_plane(const G27Part<T> &g, T xw, T xe) {
-  return g.a + g.cE * xe + g.cW * xw + g.c[0] * g.xv[0] + g.c[1] * g.xv[1] +
-         g.c[2] * g.xv[2] + g.c[3] * g.xv[3];
-}
-
 // One row (j, k) of class (pz, py) of a 27-point sweep, by one wavefront.
 // The neighbour rows come from four arrays by their offset (dy, dz) from
 // this row: xO (dy, dz even: the row itself), xN (dy odd, dz = 0), xU
@@ -967,11 +760,6 @@ __global__ __launch_bounds__(64 * (RS2 + 1)) void k_gs27_pair(
     int bp, int nplanes, int nstrips, int zmask) {
   gs27_pair_body<T, ADJ, PPL, RS2>(nx, ny, nz, ac, cc, fc, cur, nxt, po, pz,
                                    bp, nplanes, nstrips, zmask, blockIdx.x);
-}
-
-static int count_parity(int n, int par) {  // #{v in [2, n-1] : v%2 == par}
-  const int first = 2 + par;
-  return first > n - 1 ? 0 : (n - 1 - first) / 2 + 1;
 }
 
 template <class T>
@@ -2342,7 +2130,7 @@ template <class T, bool WARM, bool ABS, bool ZT>
 __device__ __forceinline__ void cg_rows_body(
     int nx, int ny, int nz, const double *__restrict__ ac,
     const double *__restrict__ cc, const T *__restrict__ f,
-    T *__restrict__ xout, int itmax, double errtol) {
+    T *__restrict__ xout, int itmax, double errtol, double *damp) {
   constexpr int R = CG_R;
   double *P = cg_lds;
   __shared__ double rbuf[2][CG_RNT / 64];
@@ -2395,6 +2183,33 @@ __device__ __forceinline__ void cg_rows_body(
   // the loop's own stencil code (P = x0), then the CG proper starts.
   bool warm_pass = WARM;
   int b = 0;
+  double o[R], u[R], dd[R], pp[R];
+  auto stencil = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < R; r++) o[r] = u[r] = dd[r] = 0.0;
+#pragma unroll
+    for (int a = 0; a < 9; a++) {
+      const int dj = (a % 3) - 1, dk = (a / 3) - 1;
+      double w[R + 2];
+#pragma unroll
+      for (int c = 0; c < R + 2; c++) w[c] = P[rb[a] + c];
+      if (dj == 0 && dk == 0) {
+#pragma unroll
+        for (int r = 0; r < R; r++) pp[r] = w[r + 1];
+      }
+#pragma unroll
+      for (int q = 0; q < 26; q++) {
+        if (DJ[q] != dj || DK[q] != dk) continue;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+          const double t = cf[r][q] * w[r + 1 + DI[q]];
+          if (DK[q] == 0) o[r] += t;
+          else if (DK[q] > 0) u[r] += t;
+          else dd[r] += t;
+        }
+      }
+    }
+  };
   double rhok2 = 0.0, denom = 0.0;
   double s = 0.0;
   if constexpr (!WARM) {
@@ -2433,31 +2248,7 @@ __device__ __forceinline__ void cg_rows_body(
           if (val[r]) P[pidx[r]] = xr[r];
       }
       __syncthreads();
-      double o[R], u[R], dd[R], pp[R];
-#pragma unroll
-      for (int r = 0; r < R; r++) o[r] = u[r] = dd[r] = 0.0;
-#pragma unroll
-      for (int a = 0; a < 9; a++) {
-        const int dj = (a % 3) - 1, dk = (a / 3) - 1;
-        double w[R + 2];
-#pragma unroll
-        for (int c = 0; c < R + 2; c++) w[c] = P[rb[a] + c];
-        if (dj == 0 && dk == 0) {
-#pragma unroll
-          for (int r = 0; r < R; r++) pp[r] = w[r + 1];
-        }
-#pragma unroll
-        for (int q = 0; q < 26; q++) {
-          if (DJ[q] != dj || DK[q] != dk) continue;
-#pragma unroll
-          for (int r = 0; r < R; r++) {
-            const double t = cf[r][q] * w[r + 1 + DI[q]];
-            if (DK[q] == 0) o[r] += t;
-            else if (DK[q] > 0) u[r] += t;
-            else dd[r] += t;
-          }
-        }
-      }
+      stencil();
       s = 0.0;
       if (warm_pass) {  // r = f - A x0
 #pragma unroll
@@ -2506,20 +2297,44 @@ __device__ __forceinline__ void cg_rows_body(
 #pragma unroll
   for (int r = 0; r < R; r++)
     if (val[r]) xout[pidx[r]] = (T)xr[r];
+  // The Hackbusch-Reusken factor (x . f) / (x . A x) of the solution as
+  // stored (mgcsd.cc:429-452; 0 when the denominator is 0): one more
+  // application of the operator the threads hold, instead of a product
+  // kernel on a level of a few hundred points (4.8 us each).  Every read of
+  // P and of the other partial buffer lies before the last barrier.
+  if (damp) {
+    double s1 = 0.0;
+    s = 0.0;
+#pragma unroll
+    for (int r = 0; r < R; r++)
+      if (val[r]) P[pidx[r]] = (double)(T)xr[r];
+    __syncthreads();
+    stencil();
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      if (!val[r]) continue;
+      s += pp[r] * (double)f[pidx[r]];
+      s1 += pp[r] * (-o[r] + -u[r] + -dd[r] + dg[r] * pp[r]);
+    }
+    s = cg_allsum<CG_RNT / 64>(s, rbuf[b]);
+    s1 = cg_allsum<CG_RNT / 64>(s1, rbuf[b ^ 1]);
+    if (tid == 0) *damp = s1 != 0.0 ? s / s1 : 0.0;
+  }
 }
 
 template <class T, bool WARM, bool ABS, bool ZT>
 __global__ __launch_bounds__(CG_RNT) void k_cg_rows(
     int nx, int ny, int nz, const double *__restrict__ ac,
     const double *__restrict__ cc, const T *__restrict__ f,
-    T *__restrict__ xout, int itmax, double errtol) {
-  cg_rows_body<T, WARM, ABS, ZT>(nx, ny, nz, ac, cc, f, xout, itmax, errtol);
+    T *__restrict__ xout, int itmax, double errtol, double *damp) {
+  cg_rows_body<T, WARM, ABS, ZT>(nx, ny, nz, ac, cc, f, xout, itmax, errtol,
+                                 damp);
 }
 
 template <class T, int ND>
-static void cg_launch(const Dim &d, const double *ac, const double *cc,
+static bool cg_launch(const Dim &d, const double *ac, const double *cc,
                       const T *f, T *x, int itmax, double errtol,
-                      hipStream_t s) {
+                      hipStream_t s, double *damp) {
   const size_t lds = d.n() * sizeof(double);
   const size_t ni = d.interior();
   const int nrow = (int)((d.nx - 2 + CG_R - 1) / CG_R) * (d.ny - 2) * (d.nz - 2);
@@ -2528,12 +2343,12 @@ static void cg_launch(const Dim &d, const double *ac, const double *cc,
     if (errtol == 0.0)
       k_cg_rows<T, false, false, true>
           <<<1, nt, lds + (CG_R + 2) * sizeof(double), s>>>(
-              d.nx, d.ny, d.nz, ac, cc, f, x, itmax, errtol);
+              d.nx, d.ny, d.nz, ac, cc, f, x, itmax, errtol, damp);
     else
       k_cg_rows<T, false, false, false>
           <<<1, nt, lds + (CG_R + 2) * sizeof(double), s>>>(
-              d.nx, d.ny, d.nz, ac, cc, f, x, itmax, errtol);
-    return;
+              d.nx, d.ny, d.nz, ac, cc, f, x, itmax, errtol, damp);
+    return damp != nullptr;
   }
   // one interior point per thread when they fit: as few wavefronts as the
   // level needs (the loop is LDS- and barrier-bound, idle waves cost)
@@ -2545,20 +2360,22 @@ static void cg_launch(const Dim &d, const double *ac, const double *cc,
     k_cg_single<T, 2, ND><<<1, CG_NT, lds, s>>>(d.nx, d.ny, d.nz, ac, cc, f,
                                                 x, itmax, errtol);
   }
+  return false;
 }
 
 template <class T>
-void cg_single(const Dim &d, int numdia, const double *ac, const double *cc,
-               const T *f, T *x, int itmax, double errtol, hipStream_t s) {
+bool cg_single(const Dim &d, int numdia, const double *ac, const double *cc,
+               const T *f, T *x, int itmax, double errtol, hipStream_t s,
+               double *damp) {
   if (!cg_fits(d)) {
     fprintf(stderr, "pmg: coarsest level too large for cg_single\n");
-    return;
+    return false;
   }
-  if (numdia == 7)
-    cg_launch<T, 7>(d, ac, cc, f, x, itmax, errtol, s);
-  else
-    cg_launch<T, 27>(d, ac, cc, f, x, itmax, errtol, s);
+  const bool done =
+      numdia == 7 ? cg_launch<T, 7>(d, ac, cc, f, x, itmax, errtol, s, damp)
+                  : cg_launch<T, 27>(d, ac, cc, f, x, itmax, errtol, s, damp);
   check_launch("cg_single");
+  return done;
 }
 
 bool cg_class_fits(const Dim &d, int numdia) {
@@ -2569,7 +2386,8 @@ bool cg_class_fits(const Dim &d, int numdia) {
 
 template <class T>
 void cg_class(const Dim &d, int numdia, const double *ac, const double *cc,
-              const T *f, T *x, int itmax, double thresh, hipStream_t s) {
+              const T *f, T *x, int itmax, double thresh, hipStream_t s,
+              double *damp) {
   if (!cg_class_fits(d, numdia)) {
     fprintf(stderr, "pmg: coarsest level too large for cg_class\n");
     return;
@@ -2578,7 +2396,7 @@ void cg_class(const Dim &d, int numdia, const double *ac, const double *cc,
   const int nt = (nrow + 63) / 64 * 64;
   k_cg_rows<T, true, true, false>
       <<<1, nt, d.n() * sizeof(double) + (CG_R + 2) * sizeof(double), s>>>(
-          d.nx, d.ny, d.nz, ac, cc, f, x, itmax, thresh);
+          d.nx, d.ny, d.nz, ac, cc, f, x, itmax, thresh, damp);
   check_launch("cg_class");
 }
 
@@ -2955,13 +2773,6 @@ __device__ inline double coupling(const double *__restrict__ ac, size_t n,
   return ac[(size_t)pl * n + at];
 }
 
-__host__ __device__ constexpr int pplane(int dx, int dy, int dz) {
-  return 9 * (dz == 0 ? 0 : (dz == 1 ? 1 : 2)) +
-         (dy == -1 ? (dx == -1 ? 8 : (dx == 0 ? 2 : 7))
-                   : (dy == 0 ? (dx == -1 ? 4 : (dx == 0 ? 0 : 3))
-                              : (dx == -1 ? 6 : (dx == 0 ? 1 : 5))));
-}
-
 // Weights of the collapsed-operator rule: for F = C_f + d, axes with d_a = 0
 // are collapsed into the diagonal; neighbours towards C carry the known
 // weight of their own offset, neighbours away from C weight 0.
@@ -3265,34 +3076,6 @@ void buildG(const Dim &f, const Dim &c, int numdia, const double *pc,
 // solving it alone.  The launchers split the problems by kernel variant
 // and into launches of at most GMAX.
 // ---------------------------------------------------------------------------
-template <class A>
-struct GTab {
-  A a[GMAX];
-};
-
-// Launch f(tab, count) for each run of at most GMAX consecutive entries of
-// the problems whose key equals key (entries built by mk(q) into the tab).
-template <class A, class KeyF, class MkF, class LaunchF>
-static void g_split(int n, KeyF key, MkF mk, LaunchF launch) {
-  std::vector<char> done(n, 0);
-  for (int q0 = 0; q0 < n; q0++) {
-    if (done[q0]) continue;
-    const auto k0 = key(q0);
-    GTab<A> t{};
-    int m = 0;
-    for (int q = q0; q < n; q++) {
-      if (done[q] || !(key(q) == k0)) continue;
-      done[q] = 1;
-      t.a[m++] = mk(q);
-      if (m == GMAX) {
-        launch(t, m, k0);
-        m = 0;
-      }
-    }
-    if (m) launch(t, m, k0);
-  }
-}
-
 template <class T>
 struct A_gs7 {
   int nx, ny, nz;
@@ -3683,7 +3466,7 @@ struct A_ip {
   int nxc, nyc, nzc, nxf, nyf, nzf;
   const T *xc, *pc;
   T *xf;
-  const double *part;
+  const double *damp, *part;
   unsigned npart;
   PR sh;
 };
@@ -3692,7 +3475,7 @@ __global__ __launch_bounds__(256) void kb_interp_damped(const GTab<A_ip<T>> t) {
   const A_ip<T> &a = t.a[blockIdx.y];
   if (blockIdx.x >= a.sh.nblk) return;
   interp_body<T, true>(a.nxc, a.nyc, a.nzc, a.nxf, a.nyf, a.nzf, a.xc, a.pc,
-                       a.xf, nullptr, a.part, a.npart, a.sh, blockIdx.x);
+                       a.xf, a.damp, a.part, a.npart, a.sh, blockIdx.x);
 }
 
 template <class T>
@@ -3715,8 +3498,8 @@ void g_interp_damped(const GInterp<T> *j, int n, hipStream_t s) {
       [&](int q) {
         const GInterp<T> &J = j[ok[q]];
         return A_ip<T>{J.c.nx, J.c.ny, J.c.nz, J.f.nx, J.f.ny,
-                       J.f.nz, J.xc,   J.pc,   J.xf,   J.part,
-                       J.nblk, pr_shape(J.c.nx - 1, J.c.ny - 1, J.c.nz - 1)};
+                       J.f.nz, J.xc,   J.pc,   J.xf,   J.damp,
+                       J.part, J.nblk, pr_shape(J.c.nx - 1, J.c.ny - 1, J.c.nz - 1)};
       },
       [&](const GTab<A_ip<T>> &t, int m, int rows) {
         unsigned mx = 0;
@@ -3734,16 +3517,17 @@ struct A_cg {
   T *x;
   int itmax;
   double errtol;
+  double *damp;
 };
 template <class T, bool ZT>
 __global__ __launch_bounds__(CG_RNT) void kb_cg_rows(const GTab<A_cg<T>> t) {
   const A_cg<T> &a = t.a[blockIdx.y];
   cg_rows_body<T, false, false, ZT>(a.nx, a.ny, a.nz, a.ac, a.cc, a.f, a.x,
-                                    a.itmax, a.errtol);
+                                    a.itmax, a.errtol, a.damp);
 }
 
 // The 27-point coarsest levels k_cg_rows takes (cg_launch's first case).
-static bool g_cg_rows_ok(const Dim &d, int numdia) {
+bool cg_rows_fits(const Dim &d, int numdia) {
   const int nrow = (int)((d.nx - 2 + CG_R - 1) / CG_R) * (d.ny - 2) * (d.nz - 2);
   return numdia == 27 && nrow <= CG_RNT && cg_fits(d);
 }
@@ -3753,7 +3537,7 @@ void g_cg(const GCoarse<T> *j, int n, int itmax, double errtol,
           hipStream_t s) {
   std::vector<int> ok;
   for (int q = 0; q < n; q++) {
-    if (g_cg_rows_ok(j[q].d, j[q].numdia))
+    if (cg_rows_fits(j[q].d, j[q].numdia))
       ok.push_back(q);
     else
       cg_single<T>(j[q].d, j[q].numdia, j[q].ac, j[q].cc, j[q].f, j[q].x,
@@ -3769,7 +3553,7 @@ void g_cg(const GCoarse<T> *j, int n, int itmax, double errtol,
       [&](int q) {
         const GCoarse<T> &J = j[ok[q]];
         return A_cg<T>{J.d.nx, J.d.ny, J.d.nz, J.ac, J.cc, J.f, J.x, itmax,
-                       errtol};
+                       errtol, J.damp};
       },
       [&](const GTab<A_cg<T>> &t, int m, int) {
         int nt = 64;
@@ -3856,11 +3640,12 @@ template void dot_energy<double>(const Dim &, int, const double *,
                                         const T *, const T *, const T *, T *, \
                                         double *, hipStream_t);               \
   template void nrm1<T>(const Dim &, const T *, const Red &, hipStream_t);     \
-  template void cg_single<T>(const Dim &, int, const double *,                \
+  template bool cg_single<T>(const Dim &, int, const double *,                \
                              const double *, const T *, T *, int, double,     \
-                             hipStream_t);                                    \
+                             hipStream_t, double *);                          \
   template void cg_class<T>(const Dim &, int, const double *, const double *, \
-                            const T *, T *, int, double, hipStream_t);        \
+                            const T *, T *, int, double, hipStream_t,         \
+                            double *);                                        \
   template void fill<T>(T *, size_t, T, hipStream_t);                         \
   template void axpy_interior<T>(const Dim &, double, const T *, T *,         \
                                  hipStream_t);                                \

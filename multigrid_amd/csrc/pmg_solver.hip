@@ -183,14 +183,35 @@ bool smooth(pmg_ctx *c, const LV<T> &l, const T *f, T *x, int nu, int iadj,
 // ignores cc as the reference's band does).  FP64 inside either way.
 // errtol > 0: Vcghs's relative stopping test sqrt(r.r)/sqrt(r0.r0) <= errtol
 // with that tolerance instead of epsiln (at most 100 iterations).
+// damp (may be null): the device scalar for the Hackbusch-Reusken factor of
+// the solution; returns whether the solver wrote it.
 template <class T>
-void coarse_solve(pmg_ctx *c, int l, const double *ac64, const double *cc64,
-                  const T *f, T *x, double errtol = 0.0) {
+bool coarse_solve(pmg_ctx *c, int l, const double *ac64, const double *cc64,
+                  const T *f, T *x, double errtol = 0.0,
+                  double *damp = nullptr) {
   const Level &L = c->L[l];
-  if (c->p.mgsolv == 1)
+  if (c->p.mgsolv == 1) {
     band_solve<T>(L.d, L.numdia, c->band_rt, c->band_ct, f, x, c->s);
-  else
-    cg_single<T>(L.d, L.numdia, ac64, cc64, f, x, 100, errtol, c->s);
+    return false;
+  }
+  return cg_single<T>(L.d, L.numdia, ac64, cc64, f, x, 100, errtol, c->s,
+                      damp);
+}
+
+// Whether the last two levels of a cycle on L[0 .. nlev-1] run in the bottom
+// kernels: not with the banded coarsest solve, and not where the level above
+// the coarsest is the cycle's first.
+template <class T>
+bool bottom_ok(const Params &p, const LV<T> *L, int nlev) {
+  return p.mgsolv == 0 && nlev >= 3 &&
+         bottom_fits<T>(L[nlev - 2].d, L[nlev - 2].numdia, L[nlev - 1].d,
+                        L[nlev - 1].numdia);
+}
+template <class T>
+GBottom<T> bottom_of(pmg_ctx *c, const LV<T> *L, int nlev) {
+  const LV<T> &a = L[nlev - 2], &b = L[nlev - 1];
+  return GBottom<T>{a.d, b.d,  a.ac, a.cc, a.w0,
+                    b.pc, a.x, b.w0, b.x,  c->scal + S_XDAMP};
 }
 
 // Relative tolerance of the FP64 coarsest CG inside the FP32 V-cycle of the
@@ -233,24 +254,34 @@ bool vcycle(pmg_ctx *c, LV<T> *L, const T *frhs, const double *ac64c,
   smooth<T>(c, L[0], frhs, L[0].x, p.nu1, 0, true, fine_zero, fine_zero);
   resid<T, T>(L[0].d, L[0].numdia, L[0].ac, L[0].cc, frhs, L[0].x, L[0].r,
               nullptr, s, L[0].dg);
-  for (int l = 1; l < nlev; l++) {  // down (mgcsd.cc:325-360)
+  const bool bot = bottom_ok<T>(p, L, nlev);
+  const int last = bot ? nlev - 2 : nlev - 1;  // last level entered by itself
+  for (int l = 1; l <= last; l++) {  // down (mgcsd.cc:325-360)
     restrict_<T>(L[l - 1].d, L[l].d, L[l - 1].r, L[l].w0, L[l].pc, s);
-    if (l != nlev - 1) {
+    if (l != last) {
       // Vazeros + nu1 smoothings (zero start folded into the sweep)
       smooth<T>(c, L[l], L[l].w0, L[l].x, p.nu1, 0, false, true);
       resid<T, T>(L[l].d, L[l].numdia, L[l].ac, L[l].cc, L[l].w0, L[l].x,
                   L[l].r, nullptr, s);
     }
   }
-  coarse_solve<T>(c, c->nlev - 1, ac64c, cc64c, L[nlev - 1].w0,
-                  L[nlev - 1].x, coarse_tol);
-  for (int l = nlev - 2; l >= 0; l--) {  // up (mgcsd.cc:418-473)
+  const GBottom<T> gb = bottom_of<T>(c, L, std::max(nlev, 2));
+  if (bot) bottom_down<T>(&gb, 1, p.nu1, s);
+  bool damped = coarse_solve<T>(c, c->nlev - 1, ac64c, cc64c, L[nlev - 1].w0,
+                                L[nlev - 1].x, coarse_tol, gb.damp);
+  if (bot) bottom_up<T>(&gb, 1, p.nu2, 1, s);
+  for (int l = last - 1; l >= 0; l--) {  // up (mgcsd.cc:418-473)
     const int cl = l + 1;
-    const unsigned nb =
-        matvec_dots_part<T>(L[cl].d, L[cl].numdia, L[cl].ac, L[cl].cc,
-                            L[cl].x, L[cl].w0, L[cl].t, c->part, s);
-    interp_damped<T>(L[cl].d, L[l].d, L[cl].x, L[cl].pc, L[l].x, c->part, nb,
-                     s);
+    if (damped) {  // level cl's factor is there already
+      interp<T>(L[cl].d, L[l].d, L[cl].x, L[cl].pc, L[l].x, gb.damp, s);
+      damped = false;
+    } else {
+      const unsigned nb =
+          matvec_dots_part<T>(L[cl].d, L[cl].numdia, L[cl].ac, L[cl].cc,
+                              L[cl].x, L[cl].w0, L[cl].t, c->part, s);
+      interp_damped<T>(L[cl].d, L[l].d, L[cl].x, L[cl].pc, L[l].x, c->part,
+                       nb, s);
+    }
     if (l == 0)
       return smooth<T>(c, L[0], frhs, L[0].x, p.nu2, 1, true, false, false,
                        uadd);
@@ -951,15 +982,19 @@ void g_vcycle(pmg_ctx *const *c, int n, LV<T> *const *L,
     }
     g_resid<T, T>(j.data(), n, s);
   }
+  // the last level each context enters by itself (see vcycle)
+  std::vector<int> last(n);
+  for (int q = 0; q < n; q++)
+    last[q] = c[q]->nlev - (bottom_ok<T>(c[q]->p, L[q], c[q]->nlev) ? 2 : 1);
   for (int l = 1; l < lmax; l++) {  // down
     std::vector<GRestrict<T>> jr;
     std::vector<int> mid;
     std::vector<const T *> fm;
     for (int q = 0; q < n; q++) {
-      if (c[q]->nlev <= l) continue;
+      if (last[q] < l) continue;
       jr.push_back(GRestrict<T>{L[q][l - 1].d, L[q][l].d, L[q][l - 1].r,
                                 L[q][l].w0, L[q][l].pc});
-      if (l != c[q]->nlev - 1) {
+      if (l != last[q]) {
         mid.push_back(q);
         fm.push_back(L[q][l].w0);
       }
@@ -974,7 +1009,13 @@ void g_vcycle(pmg_ctx *const *c, int n, LV<T> *const *L,
     }
     g_resid<T, T>(j.data(), (int)j.size(), s);
   }
-  {  // coarsest levels
+  std::vector<char> damped(n, 0);
+  {  // bottom and coarsest levels
+    std::vector<GBottom<T>> jb;
+    for (int q = 0; q < n; q++)
+      if (last[q] == c[q]->nlev - 2)
+        jb.push_back(bottom_of<T>(c[q], L[q], c[q]->nlev));
+    bottom_down<T>(jb.data(), (int)jb.size(), nu1, s);
     std::vector<GCoarse<T>> jc;
     for (int q = 0; q < n; q++) {
       const int lc = c[q]->nlev - 1;
@@ -983,32 +1024,43 @@ void g_vcycle(pmg_ctx *const *c, int n, LV<T> *const *L,
         band_solve<T>(C.d, C.numdia, c[q]->band_rt, c[q]->band_ct,
                       L[q][lc].w0, L[q][lc].x, s);
       } else {
+        damped[q] = cg_rows_fits(C.d, C.numdia);
         jc.push_back(GCoarse<T>{C.d, C.numdia, C.ac, C.cc, L[q][lc].w0,
-                                L[q][lc].x});
+                                L[q][lc].x, c[q]->scal + S_XDAMP});
       }
     }
     g_cg<T>(jc.data(), (int)jc.size(), 100, coarse_tol, s);
+    bottom_up<T>(jb.data(), (int)jb.size(), nu2, 1, s);
   }
   for (int l = lmax - 2; l >= 0; l--) {  // up
-    std::vector<int> qs;
-    for (int q = 0; q < n; q++)
-      if (c[q]->nlev - 2 >= l) qs.push_back(q);
+    std::vector<int> qs, qm;  // contexts at this level; those with a product
+    for (int q = 0; q < n; q++) {
+      if (last[q] - 1 < l) continue;
+      qs.push_back(q);
+      if (!damped[q]) qm.push_back(q);
+    }
     if (qs.empty()) continue;
     const int cl = l + 1;
     std::vector<GMatvec<T>> jm;
-    for (int q : qs) {
+    for (int q : qm) {
       const LV<T> &v = L[q][cl];
       jm.push_back(GMatvec<T>{v.d, v.numdia, v.ac, v.cc, v.x, v.w0, v.t,
                               c[q]->part});
     }
-    std::vector<unsigned> nb(qs.size());
+    std::vector<unsigned> nb(qm.size());
     g_matvec_dots_part<T>(jm.data(), (int)jm.size(), nb.data(), s);
     std::vector<GInterp<T>> ji;
     std::vector<const T *> fu;
-    for (size_t k = 0; k < qs.size(); k++) {
-      const int q = qs[k];
+    size_t km = 0;
+    for (int q : qs) {
+      const bool have = damped[q];
       ji.push_back(GInterp<T>{L[q][cl].d, L[q][l].d, L[q][cl].x, L[q][cl].pc,
-                              L[q][l].x, c[q]->part, nb[k]});
+                              L[q][l].x,
+                              have ? c[q]->scal + S_XDAMP : nullptr,
+                              have ? nullptr : c[q]->part,
+                              have ? 0u : nb[km]});
+      if (!have) km++;
+      damped[q] = 0;
       fu.push_back(l == 0 ? frhs[q] : L[q][l].w0);
     }
     g_interp_damped<T>(ji.data(), (int)ji.size(), s);
@@ -1389,26 +1441,35 @@ template <class T>
 void class_vcycle(pmg_ctx *c, LV<T> *L, const T *frhs) {
   const int nlev = c->nlev;
   hipStream_t s = c->s;
-  for (int l = 0; l < nlev - 1; l++) {
+  const bool bot = bottom_ok<T>(c->p, L, nlev);
+  const int last = bot ? nlev - 2 : nlev - 1;  // as vcycle
+  for (int l = 0; l < last; l++) {
     const T *rhs = l == 0 ? frhs : L[l].w0;
     smooth<T>(c, L[l], rhs, L[l].x, 2, 0, false, true);
     resid<T, T>(L[l].d, L[l].numdia, L[l].ac, L[l].cc, rhs, L[l].x, L[l].r,
                 nullptr, s);
     restrict_<T>(L[l].d, L[l + 1].d, L[l].r, L[l + 1].w0, L[l + 1].pc, s);
   }
+  const GBottom<T> gb = bottom_of<T>(c, L, nlev);
+  if (bot) bottom_down<T>(&gb, 1, 2, s);
   {
     const Level &C = c->L[nlev - 1];
     const int ni = (int)C.d.interior();
     cg_class<T>(C.d, C.numdia, C.ac, C.cc, L[nlev - 1].w0, L[nlev - 1].x,
-                std::max(1000, 4 * ni), 1e-8, s);
+                std::max(1000, 4 * ni), 1e-8, s, gb.damp);
   }
-  for (int l = nlev - 2; l >= 0; l--) {
+  if (bot) bottom_up<T>(&gb, 1, 2, 0, s);
+  for (int l = last - 1; l >= 0; l--) {
     const int cl = l + 1;
-    const unsigned nb =
-        matvec_dots_part<T>(L[cl].d, L[cl].numdia, L[cl].ac, L[cl].cc,
-                            L[cl].x, L[cl].w0, L[cl].t, c->part, s);
-    interp_damped<T>(L[cl].d, L[l].d, L[cl].x, L[cl].pc, L[l].x, c->part, nb,
-                     s);
+    if (l == last - 1) {
+      interp<T>(L[cl].d, L[l].d, L[cl].x, L[cl].pc, L[l].x, gb.damp, s);
+    } else {
+      const unsigned nb =
+          matvec_dots_part<T>(L[cl].d, L[cl].numdia, L[cl].ac, L[cl].cc,
+                              L[cl].x, L[cl].w0, L[cl].t, c->part, s);
+      interp_damped<T>(L[cl].d, L[l].d, L[cl].x, L[cl].pc, L[l].x, c->part,
+                       nb, s);
+    }
     smooth<T>(c, L[l], l == 0 ? frhs : L[l].w0, L[l].x, 2, 0, false);
   }
 }
