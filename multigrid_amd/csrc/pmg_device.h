@@ -56,6 +56,40 @@ __device__ inline double wave_sum(double v) {
   return __hiloint2double(hi, lo);
 }
 
+// All lanes take part in the DPP moves below (no lane without a source).
+template <int CTRL>
+__device__ __forceinline__ double dpp_all(double v) {
+  return dpp_f64<CTRL, 0xF>(v);
+}
+// v plus the values of the lane 16 (32) away in its pair of rows (halves).
+__device__ __forceinline__ double add_rows16(double v) {
+  const auto lo = __builtin_amdgcn_permlane16_swap(
+      __double2loint(v), __double2loint(v), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(
+      __double2hiint(v), __double2hiint(v), false, false);
+  return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+__device__ __forceinline__ double add_rows32(double v) {
+  const auto lo = __builtin_amdgcn_permlane32_swap(
+      __double2loint(v), __double2loint(v), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(
+      __double2hiint(v), __double2hiint(v), false, false);
+  return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+// Sums of four values over the wavefront for little more than the price of
+// one: two exchanges hand each lane of a quad the quad's sum of one of the
+// values, and five additions then run on one register.  Lane l returns the
+// wavefront's sum of a[l % 4].
+__device__ __forceinline__ double wave_sum4(const double (&a)[4]) {
+  const bool odd = threadIdx.x & 1, two = threadIdx.x & 2;
+  const double b0 = (odd ? a[1] : a[0]) + dpp_all<0xB1>(odd ? a[0] : a[1]);
+  const double b1 = (odd ? a[3] : a[2]) + dpp_all<0xB1>(odd ? a[2] : a[3]);
+  double c = (two ? b1 : b0) + dpp_all<0x4E>(two ? b0 : b1);
+  c += dpp_all<0x124>(c);  // row_ror:4, row_ror:8: the row's four quads
+  c += dpp_all<0x128>(c);
+  return add_rows32(add_rows16(c));
+}
+
 // Two or four consecutive elements by one load each (two for four doubles),
 // aligned to the element only.
 typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));

@@ -2113,29 +2113,90 @@ __global__ __launch_bounds__(CG_NT) void k_cg_single(
     if (val[m]) xout[pidx[m]] = (T)xr[m];
 }
 
-// Row-segment variant for 27-point levels: each thread owns CG_R
+// Row-segment variant for 27-point levels: each thread owns R (2 or 3)
 // consecutive points of an i-row.  Per iteration it reads the R+2 values of
-// each of the 9 neighbouring rows once from LDS (15 reads per point instead
-// of 27) and keeps the 26 couplings of its points in registers; fewer
-// wavefronts make the per-iteration reductions and barriers cheaper.  Terms
+// each of the 9 neighbouring rows once from LDS (18 or 15 reads per point
+// instead of 27) and keeps the 26 couplings of its points in registers; fewer
+// wavefronts make the per-iteration reduction and barriers cheaper.  Terms
 // are summed in the reference's three groups (in-plane, up, down), each
 // group row by row.
-constexpr int CG_R = 3, CG_RNT = 512;
+constexpr int CG_R = 3, CG_RNT = 512, CG_W = CG_RNT / 64;
+// Points per thread: 2 where four wavefronts hold the level that way (up to
+// 9^3: 100 us per 100 iterations against 107 with 3; its LDS reads, 18 per
+// point against 15, then fit beside the multiply-adds), else 3 (11^3: 126
+// against 152).
+static int cg_threads(const Dim &d, int r) {
+  const int segs = (d.nx - 2 + r - 1) / r * (d.ny - 2) * (d.nz - 2);
+  return (segs + 63) / 64 * 64;
+}
+static int cg_points(const Dim &d) { return cg_threads(d, 2) <= 256 ? 2 : CG_R; }
+// The 27-point coarsest levels k_cg_rows takes.
+bool cg_rows_fits(const Dim &d, int numdia) {
+  return numdia == 27 && cg_fits(d) && cg_threads(d, CG_R) <= CG_RNT;
+}
+
+// Sums of four values over the workgroup, in every thread.  Each wavefront's
+// sums go to its slots of buf (those of wavefronts the workgroup does not
+// have hold zero), and every wavefront adds the slots up in one fixed tree:
+// the same bits at any workgroup width.  A barrier must lie between reading
+// the slots here and the next call (the one before the stencil).
+__device__ __forceinline__ void cg_sum4(const double (&a)[4],
+                                        double (*buf)[4], double (&out)[4]) {
+  static_assert(CG_W == 8, "two rows of 16 lanes hold the slots");
+  const int lane = threadIdx.x & 63;
+  const double c = wave_sum4(a);
+  if (lane < 4) buf[threadIdx.x >> 6][lane] = c;
+  __syncthreads();
+  double v = buf[(lane & 31) >> 2][lane & 3];
+  v += dpp_all<0x124>(v);
+  v += dpp_all<0x128>(v);
+  v = add_rows16(v);
+  out[0] = dpp_all<0x00>(v);  // quad_perm: the quad's lane 0, 1, 2, 3
+  out[1] = dpp_all<0x55>(v);
+  out[2] = dpp_all<0xAA>(v);
+  out[3] = dpp_all<0xFF>(v);
+}
+
+// 1 / x within an ulp or two for ordinary magnitudes (the hardware estimate
+// and two Newton steps, half the latency of a division); a true division for
+// negative values and at the ends of the range, where the steps would
+// overflow; 0 for 0 (everything underflown ends the progress, not the loop).
+// x is the same in all lanes, so the test runs on the scalar unit.
+__device__ __forceinline__ double cg_rcp(double x) {
+  const unsigned e = (unsigned)__builtin_amdgcn_readfirstlane(
+                         __double2hiint(x)) >> 20;  // sign and exponent
+  if (e - 64u > 1900u) return x != 0.0 ? 1.0 / x : 0.0;
+  double y = __builtin_amdgcn_rcp(x);
+  y = fma(fma(-x, y, 1.0), y, y);
+  return fma(fma(-x, y, 1.0), y, y);
+}
+
 // WARM: start from xout (else 0); ABS: the class solver's absolute
 // criterion (else Vcghs's relative one); ZT: errtol is 0, so Vcghs's test
 // sqrt(r.r)/sqrt(r0.r0) <= errtol is r.r == 0 (no square root or divide in
 // the loop).  The PMG cycle uses <T, 0, 0, 1> (errtol = epsiln = 0).
+//
+// An iteration is a chain of latencies on one compute unit (three or four
+// wavefronts, no other work): LDS write of p, barrier, 42 LDS reads, 78
+// multiply-adds, a reduction over the workgroup, the quotients.  So it has
+// one reduction, of p.Ap, r.Ap, Ap.Ap and r.r together: r.r of the new
+// residual is r.r - 2 a r.Ap + a^2 Ap.Ap, exact up to a rounding of the old
+// r.r, which each iteration sums anew from r itself, so nothing accumulates.
+// Beside it 1/(p.Ap) and 1/(r.r) run side by side without divisions, and p
+// stays in registers.  100 iterations with the damping factor (MI355X): 151
+// us on 11^3 and 126 on 9^3 with two reductions, three divisions and three
+// barriers per iteration; 126 and 100 so; to a relative 1e-2 on 9^3 in FP32
+// cycles 19 and 10.5.
 extern __shared__ double cg_lds[];
-template <class T, bool WARM, bool ABS, bool ZT>
+template <class T, bool WARM, bool ABS, bool ZT, int R>
 __device__ __forceinline__ void cg_rows_body(
     int nx, int ny, int nz, const double *__restrict__ ac,
     const double *__restrict__ cc, const T *__restrict__ f,
     T *__restrict__ xout, int itmax, double errtol, double *damp) {
-  constexpr int R = CG_R;
   double *P = cg_lds;
-  __shared__ double rbuf[2][CG_RNT / 64];
-  cg_zero_slots<CG_RNT / 64>(rbuf);
+  __shared__ double slots[CG_W][4];
   const int tid = threadIdx.x, NTB = blockDim.x;
+  if (tid < CG_W * 4) slots[tid >> 2][tid & 3] = 0.0;
   const size_t n = (size_t)nx * ny * nz;
   const long long sy = nx, sz = (long long)nx * ny;
   const int ni = nx - 2, nj = ny - 2, nk = nz - 2;
@@ -2148,7 +2209,7 @@ __device__ __forceinline__ void cg_rows_body(
   for (size_t q = tid; q < n + R + 2; q += NTB) P[q] = 0.0;
   int pidx[R];
   bool val[R];
-  double xr[R], rr[R], apv[R], dg[R];
+  double xr[R], rr[R], pp[R], dg[R];
   double cf[R][26];
   long long off[26];
 #pragma unroll
@@ -2158,7 +2219,6 @@ __device__ __forceinline__ void cg_rows_body(
     pidx[r] = (int)p;
     xr[r] = WARM && val[r] ? (double)xout[p] : 0.0;
     rr[r] = val[r] ? (double)f[p] : 0.0;  // r = f - A x (x = 0 unless warm)
-    apv[r] = 0.0;
     dg[r] = val[r] ? ac[p] + cc[p] : 0.0;
     cg_load_row<27>(ac, n, sy, sz, p, cf[r], off);
     if (!val[r]) {
@@ -2178,13 +2238,10 @@ __device__ __forceinline__ void cg_rows_body(
                                   1, 1, -1, -1, 0, 1, -1, 0, 0, 1, 1, -1, -1};
   constexpr signed char DK[26] = {0, 0, 0, 0, 0, 0, 0, 0, 1, 1, 1, 1, 1,
                                   1, 1, 1, 1, -1, -1, -1, -1, -1, -1, -1, -1, -1};
-  __syncthreads();
-  // With WARM the first pass through the loop computes r = f - A x0 with
-  // the loop's own stencil code (P = x0), then the CG proper starts.
-  bool warm_pass = WARM;
-  int b = 0;
-  double o[R], u[R], dd[R], pp[R];
+  double v[R];
+  // v = A pp, pp being the thread's points of P (0 at points it lacks)
   auto stencil = [&]() __attribute__((always_inline)) {
+    double o[R], u[R], dd[R];
 #pragma unroll
     for (int r = 0; r < R; r++) o[r] = u[r] = dd[r] = 0.0;
 #pragma unroll
@@ -2192,11 +2249,8 @@ __device__ __forceinline__ void cg_rows_body(
       const int dj = (a % 3) - 1, dk = (a / 3) - 1;
       double w[R + 2];
 #pragma unroll
-      for (int c = 0; c < R + 2; c++) w[c] = P[rb[a] + c];
-      if (dj == 0 && dk == 0) {
-#pragma unroll
-        for (int r = 0; r < R; r++) pp[r] = w[r + 1];
-      }
+      for (int c = 0; c < R + 2; c++)
+        w[c] = P[rb[a] + c];
 #pragma unroll
       for (int q = 0; q < 26; q++) {
         if (DJ[q] != dj || DK[q] != dk) continue;
@@ -2209,83 +2263,71 @@ __device__ __forceinline__ void cg_rows_body(
         }
       }
     }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      v[r] = -o[r] + -u[r] + -dd[r] + dg[r] * pp[r];
+      v[r] = val[r] ? v[r] : 0.0;
+    }
   };
-  double rhok2 = 0.0, denom = 0.0;
-  double s = 0.0;
-  if constexpr (!WARM) {
+  // a segment's places past the row end are boundary cells, whose 0 it
+  // writes again (x is 0 at points the thread lacks)
+  auto put = [&](const double (&x)[R]) __attribute__((always_inline)) {
+    if (act) {
 #pragma unroll
-    for (int r = 0; r < R; r++) s += rr[r] * rr[r];
-    rhok2 = cg_allsum<CG_RNT / 64>(s, rbuf[0]);
-    b = 1;
-    denom = sqrt(rhok2);
+      for (int r = 0; r < R; r++) P[rb[4] + 1 + r] = x[r];
+    }
+  };
+  double s4[4], t4[4];
+  __syncthreads();  // P and the slots are zero
+  if constexpr (WARM) {  // r = f - A x0
+#pragma unroll
+    for (int r = 0; r < R; r++) pp[r] = xr[r];
+    put(pp);
+    __syncthreads();
+    stencil();
+#pragma unroll
+    for (int r = 0; r < R; r++) rr[r] -= v[r];
   }
+  s4[0] = s4[1] = s4[2] = s4[3] = 0.0;
+#pragma unroll
+  for (int r = 0; r < R; r++) s4[3] += rr[r] * rr[r];
+  cg_sum4(s4, slots, t4);
+  double rhok2 = t4[3];
+  const double denom = sqrt(rhok2);
   int iters = 0;
-  double rhok1 = 0.0;
-  {
+#pragma unroll
+  for (int r = 0; r < R; r++) pp[r] = rr[r];
+  if (denom != 0.0) {
     for (;;) {
-      if (!warm_pass) {
-        if (denom == 0.0) break;
-        // ABS: the class solver's criterion, sqrt(r.r) > errtol, its first
-        // test made on sqrt(sqrt(r0.r0)) (CG_Solver.h:125-133)
-        if (ABS ? (iters == 0 ? sqrt(sqrt(rhok2)) : sqrt(rhok2)) <= errtol
-                : (ZT ? rhok2 == 0.0 : sqrt(rhok2) / denom <= errtol))
-          break;
-        if (iters >= itmax) break;
-        if (iters == 0) {
-#pragma unroll
-          for (int r = 0; r < R; r++)
-            if (val[r]) P[pidx[r]] = rr[r];
-        } else {
-          const double beta = rhok2 / rhok1;
-          const double ib = 1.0 / beta;
-#pragma unroll
-          for (int r = 0; r < R; r++)
-            if (val[r]) P[pidx[r]] = (P[pidx[r]] + ib * rr[r]) * beta;
-        }
-      } else {
-#pragma unroll
-        for (int r = 0; r < R; r++)
-          if (val[r]) P[pidx[r]] = xr[r];
-      }
+      // ABS: the class solver's criterion, sqrt(r.r) > errtol, its first
+      // test made on sqrt(sqrt(r0.r0)) (CG_Solver.h:125-133)
+      if (ABS ? (iters == 0 ? sqrt(sqrt(rhok2)) : sqrt(rhok2)) <= errtol
+              : (ZT ? rhok2 == 0.0 : sqrt(rhok2) / denom <= errtol))
+        break;
+      if (iters >= itmax) break;
+      put(pp);  // every read of P lies before the last reduction's barrier
       __syncthreads();
       stencil();
-      s = 0.0;
-      if (warm_pass) {  // r = f - A x0
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-          const double v = -o[r] + -u[r] + -dd[r] + dg[r] * pp[r];
-          if (val[r]) {
-            rr[r] -= v;
-            s += rr[r] * rr[r];
-          }
-        }
-        rhok2 = cg_allsum<CG_RNT / 64>(s, rbuf[b]);
-        b ^= 1;
-        denom = sqrt(rhok2);
-        warm_pass = false;
-        continue;
-      }
+      s4[0] = s4[1] = s4[2] = s4[3] = 0.0;
 #pragma unroll
       for (int r = 0; r < R; r++) {
-        const double v = -o[r] + -u[r] + -dd[r] + dg[r] * pp[r];
-        apv[r] = val[r] ? v : 0.0;
-        if (val[r]) s += pp[r] * v;
+        s4[0] += pp[r] * v[r];
+        s4[1] += rr[r] * v[r];
+        s4[2] += v[r] * v[r];
+        s4[3] += rr[r] * rr[r];
       }
-      const double pAp = cg_allsum<CG_RNT / 64>(s, rbuf[b]);
-      b ^= 1;
-      const double alpha = rhok2 / pAp;
-      rhok1 = rhok2;
-      s = 0.0;
+      cg_sum4(s4, slots, t4);
+      const double ipap = cg_rcp(t4[0]), irr = cg_rcp(t4[3]);
+      const double alpha = t4[3] * ipap;
+      rhok2 = fmax(t4[3] - alpha * (2.0 * t4[1] - alpha * t4[2]), 0.0);
+      const double beta = rhok2 * irr;
 #pragma unroll
       for (int r = 0; r < R; r++) {
-        if (!val[r]) continue;
         xr[r] += alpha * pp[r];
-        rr[r] += -alpha * apv[r];
-        s += rr[r] * rr[r];
+        rr[r] -= alpha * v[r];
+        pp[r] = rr[r] + beta * pp[r];
       }
       iters++;
-      rhok2 = cg_allsum<CG_RNT / 64>(s, rbuf[b]);
-      b ^= 1;
     }
   }
   for (size_t q = tid; q < n; q += NTB) {
@@ -2300,35 +2342,54 @@ __device__ __forceinline__ void cg_rows_body(
   // The Hackbusch-Reusken factor (x . f) / (x . A x) of the solution as
   // stored (mgcsd.cc:429-452; 0 when the denominator is 0): one more
   // application of the operator the threads hold, instead of a product
-  // kernel on a level of a few hundred points (4.8 us each).  Every read of
-  // P and of the other partial buffer lies before the last barrier.
+  // kernel on a level of a few hundred points (4.8 us each).
   if (damp) {
-    double s1 = 0.0;
-    s = 0.0;
 #pragma unroll
-    for (int r = 0; r < R; r++)
-      if (val[r]) P[pidx[r]] = (double)(T)xr[r];
+    for (int r = 0; r < R; r++) pp[r] = (double)(T)xr[r];
+    put(pp);
     __syncthreads();
     stencil();
+    s4[0] = s4[1] = s4[2] = s4[3] = 0.0;
 #pragma unroll
     for (int r = 0; r < R; r++) {
-      if (!val[r]) continue;
-      s += pp[r] * (double)f[pidx[r]];
-      s1 += pp[r] * (-o[r] + -u[r] + -dd[r] + dg[r] * pp[r]);
+      if (val[r]) s4[0] += pp[r] * (double)f[pidx[r]];
+      s4[1] += pp[r] * v[r];
     }
-    s = cg_allsum<CG_RNT / 64>(s, rbuf[b]);
-    s1 = cg_allsum<CG_RNT / 64>(s1, rbuf[b ^ 1]);
-    if (tid == 0) *damp = s1 != 0.0 ? s / s1 : 0.0;
+    cg_sum4(s4, slots, t4);
+    if (tid == 0) *damp = t4[1] != 0.0 ? t4[0] / t4[1] : 0.0;
   }
 }
 
-template <class T, bool WARM, bool ABS, bool ZT>
-__global__ __launch_bounds__(CG_RNT) void k_cg_rows(
+// NT: the largest workgroup; up to 256 threads (levels up to 11^3) the
+// compiler has the registers for everything a thread holds.
+template <class T, bool WARM, bool ABS, bool ZT, int R, int NT>
+__global__ __launch_bounds__(NT) void k_cg_rows(
     int nx, int ny, int nz, const double *__restrict__ ac,
     const double *__restrict__ cc, const T *__restrict__ f,
     T *__restrict__ xout, int itmax, double errtol, double *damp) {
-  cg_rows_body<T, WARM, ABS, ZT>(nx, ny, nz, ac, cc, f, xout, itmax, errtol,
-                                 damp);
+  cg_rows_body<T, WARM, ABS, ZT, R>(nx, ny, nz, ac, cc, f, xout, itmax,
+                                    errtol, damp);
+}
+
+template <class T, bool WARM, bool ABS>
+static void cg_rows_launch(const Dim &d, const double *ac, const double *cc,
+                           const T *f, T *x, int itmax, double errtol,
+                           hipStream_t s, double *damp) {
+  const int r = cg_points(d), nt = cg_threads(d, r);
+  const size_t lds = (d.n() + CG_R + 2) * sizeof(double);
+#define ROWS(ZT, R, NT)                                                     \
+  k_cg_rows<T, WARM, ABS, ZT, R, NT><<<1, nt, lds, s>>>(                    \
+      d.nx, d.ny, d.nz, ac, cc, f, x, itmax, errtol, damp)
+  if (!ABS && errtol == 0.0) {
+    if (r == 2) ROWS(!ABS, 2, 256);
+    else if (nt <= 256) ROWS(!ABS, CG_R, 256);
+    else ROWS(!ABS, CG_R, CG_RNT);
+  } else {
+    if (r == 2) ROWS(false, 2, 256);
+    else if (nt <= 256) ROWS(false, CG_R, 256);
+    else ROWS(false, CG_R, CG_RNT);
+  }
+#undef ROWS
 }
 
 template <class T, int ND>
@@ -2337,17 +2398,8 @@ static bool cg_launch(const Dim &d, const double *ac, const double *cc,
                       hipStream_t s, double *damp) {
   const size_t lds = d.n() * sizeof(double);
   const size_t ni = d.interior();
-  const int nrow = (int)((d.nx - 2 + CG_R - 1) / CG_R) * (d.ny - 2) * (d.nz - 2);
-  if (ND == 27 && nrow <= CG_RNT) {
-    const int nt = (nrow + 63) / 64 * 64;
-    if (errtol == 0.0)
-      k_cg_rows<T, false, false, true>
-          <<<1, nt, lds + (CG_R + 2) * sizeof(double), s>>>(
-              d.nx, d.ny, d.nz, ac, cc, f, x, itmax, errtol, damp);
-    else
-      k_cg_rows<T, false, false, false>
-          <<<1, nt, lds + (CG_R + 2) * sizeof(double), s>>>(
-              d.nx, d.ny, d.nz, ac, cc, f, x, itmax, errtol, damp);
+  if (ND == 27 && cg_rows_fits(d, ND)) {
+    cg_rows_launch<T, false, false>(d, ac, cc, f, x, itmax, errtol, s, damp);
     return damp != nullptr;
   }
   // one interior point per thread when they fit: as few wavefronts as the
@@ -2378,11 +2430,7 @@ bool cg_single(const Dim &d, int numdia, const double *ac, const double *cc,
   return done;
 }
 
-bool cg_class_fits(const Dim &d, int numdia) {
-  const int nrow = (int)((d.nx - 2 + CG_R - 1) / CG_R) * (d.ny - 2) * (d.nz - 2);
-  return numdia == 27 && d.n() * sizeof(double) <= CG_LDS_MAX &&
-         nrow <= CG_RNT;
-}
+bool cg_class_fits(const Dim &d, int numdia) { return cg_rows_fits(d, numdia); }
 
 template <class T>
 void cg_class(const Dim &d, int numdia, const double *ac, const double *cc,
@@ -2392,11 +2440,7 @@ void cg_class(const Dim &d, int numdia, const double *ac, const double *cc,
     fprintf(stderr, "pmg: coarsest level too large for cg_class\n");
     return;
   }
-  const int nrow = (int)((d.nx - 2 + CG_R - 1) / CG_R) * (d.ny - 2) * (d.nz - 2);
-  const int nt = (nrow + 63) / 64 * 64;
-  k_cg_rows<T, true, true, false>
-      <<<1, nt, d.n() * sizeof(double) + (CG_R + 2) * sizeof(double), s>>>(
-          d.nx, d.ny, d.nz, ac, cc, f, x, itmax, thresh, damp);
+  cg_rows_launch<T, true, true>(d, ac, cc, f, x, itmax, thresh, s, damp);
   check_launch("cg_class");
 }
 
@@ -3519,17 +3563,11 @@ struct A_cg {
   double errtol;
   double *damp;
 };
-template <class T, bool ZT>
-__global__ __launch_bounds__(CG_RNT) void kb_cg_rows(const GTab<A_cg<T>> t) {
+template <class T, bool ZT, int R, int NT>
+__global__ __launch_bounds__(NT) void kb_cg_rows(const GTab<A_cg<T>> t) {
   const A_cg<T> &a = t.a[blockIdx.y];
-  cg_rows_body<T, false, false, ZT>(a.nx, a.ny, a.nz, a.ac, a.cc, a.f, a.x,
-                                    a.itmax, a.errtol, a.damp);
-}
-
-// The 27-point coarsest levels k_cg_rows takes (cg_launch's first case).
-bool cg_rows_fits(const Dim &d, int numdia) {
-  const int nrow = (int)((d.nx - 2 + CG_R - 1) / CG_R) * (d.ny - 2) * (d.nz - 2);
-  return numdia == 27 && nrow <= CG_RNT && cg_fits(d);
+  cg_rows_body<T, false, false, ZT, R>(a.nx, a.ny, a.nz, a.ac, a.cc, a.f, a.x,
+                                       a.itmax, a.errtol, a.damp);
 }
 
 template <class T>
@@ -3543,33 +3581,37 @@ void g_cg(const GCoarse<T> *j, int n, int itmax, double errtol,
       cg_single<T>(j[q].d, j[q].numdia, j[q].ac, j[q].cc, j[q].f, j[q].x,
                    itmax, errtol, s);
   }
-  // One launch for every coarsest shape: the workgroup is as wide, and its
-  // LDS as large, as the largest shape needs.  k_cg_rows gives the same
-  // bits at any width: threads past a shape's rows hold no unknowns and add
-  // exact zeros to wavefront slots the reductions sum in a fixed order
-  // (cg_allsum), whether those wavefronts exist or not.
+  // One launch for the coarsest shapes of each number of points per thread:
+  // the workgroup is as wide, and its LDS as large, as the largest shape
+  // needs.  k_cg_rows gives the same bits at any width: threads past a
+  // shape's rows hold no unknowns and add exact zeros to wavefront slots the
+  // reductions sum in a fixed order (cg_sum4), whether those wavefronts
+  // exist or not.
   g_split<A_cg<T>>(
-      (int)ok.size(), [&](int) { return 0; },
+      (int)ok.size(), [&](int q) { return cg_points(j[ok[q]].d); },
       [&](int q) {
         const GCoarse<T> &J = j[ok[q]];
         return A_cg<T>{J.d.nx, J.d.ny, J.d.nz, J.ac, J.cc, J.f, J.x, itmax,
                        errtol, J.damp};
       },
-      [&](const GTab<A_cg<T>> &t, int m, int) {
+      [&](const GTab<A_cg<T>> &t, int m, int r) {
         int nt = 64;
         size_t lds = 0;
         for (int q = 0; q < m; q++) {
           const Dim d{t.a[q].nx, t.a[q].ny, t.a[q].nz};
-          const int nrow =
-              (int)((d.nx - 2 + CG_R - 1) / CG_R) * (d.ny - 2) * (d.nz - 2);
-          nt = std::max(nt, (nrow + 63) / 64 * 64);
-          lds = std::max(lds, d.n() * sizeof(double) +
-                                  (CG_R + 2) * sizeof(double));
+          nt = std::max(nt, cg_threads(d, r));
+          lds = std::max(lds, (d.n() + CG_R + 2) * sizeof(double));
         }
-        if (errtol == 0.0)
-          kb_cg_rows<T, true><<<dim3(1, m), nt, lds, s>>>(t);
-        else
-          kb_cg_rows<T, false><<<dim3(1, m), nt, lds, s>>>(t);
+        const dim3 g(1, m);
+        if (errtol == 0.0) {
+          if (r == 2) kb_cg_rows<T, true, 2, 256><<<g, nt, lds, s>>>(t);
+          else if (nt <= 256) kb_cg_rows<T, true, CG_R, 256><<<g, nt, lds, s>>>(t);
+          else kb_cg_rows<T, true, CG_R, CG_RNT><<<g, nt, lds, s>>>(t);
+        } else {
+          if (r == 2) kb_cg_rows<T, false, 2, 256><<<g, nt, lds, s>>>(t);
+          else if (nt <= 256) kb_cg_rows<T, false, CG_R, 256><<<g, nt, lds, s>>>(t);
+          else kb_cg_rows<T, false, CG_R, CG_RNT><<<g, nt, lds, s>>>(t);
+        }
       });
   check_launch("g_cg");
 }

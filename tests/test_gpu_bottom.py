@@ -5,7 +5,8 @@ potential, the bar of every FP64 solve here; mixed precision to 1e-6), alone
 and grouped with the same bits.  The level above the coarsest is 9 x 13 x 11
 (both precisions take the kernels), 5^3 over a single unknown, 17^3 (FP32
 only) and 17 x 25 x 21 (neither); sweep counts of 0 to 3, odd ones among
-them."""
+them.  Two-level grids over 11^3 and 13^3 take the coarsest CG with three
+points per thread, in workgroups of up to 256 threads and beyond."""
 import numpy as np
 import pytest
 
@@ -33,7 +34,8 @@ KEYS = ("xf", "yf", "zf", "gxcf", "gycf", "gzcf", "a1cf", "a2cf", "a3cf", "ccf",
 
 @pytest.mark.parametrize("dims,nlev,nu", [((17, 25, 21), 3, (2, 2)), ((33, 49, 41), 4, (1, 3)),
                                           ((17, 17, 17), 4, (2, 2)), ((33, 33, 33), 3, (3, 1)),
-                                          ((33, 49, 41), 3, (2, 2)), ((17, 25, 21), 3, (0, 2))])
+                                          ((33, 49, 41), 3, (2, 2)), ((17, 25, 21), 3, (0, 2)),
+                                          ((21, 21, 21), 2, (2, 2)), ((25, 25, 25), 2, (2, 2))])
 def test_bottom_levels(mg, orc, dims, nlev, nu):
     print(f"bottom dims={dims} nlev={nlev} nu={nu}", flush=True)
     inp = _inputs(dims, sum(dims) + nlev)
