@@ -11,8 +11,8 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libpmg_mi355x.so")
-SOURCES = ["pmg_kernels.hip", "pmg_pbe.hip", "pmg_band.hip", "pmg_bottom.hip", "pmg_solver.hip", "pmg_serve.hip", "pbinput.cpp",
-           "dxio.cpp"]
+SOURCES = ["pmg_kernels.hip", "pmg_pbe.hip", "pmg_band.hip", "pmg_bottom.hip", "pmg_hostcopy.hip",
+           "pmg_solver.hip", "pmg_serve.hip", "pbinput.cpp", "dxio.cpp"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

@@ -142,8 +142,10 @@ struct pmg_ctx {
     bytes += n * sizeof(T) + 256;
     return (T *)ptr;
   }
+  pmg_ctx() { pmg::host_ring_ref(); }
   ~pmg_ctx() {
     if (s) hipStreamSynchronize(s);
+    pmg::host_ring_unref();
     for (int m = 0; m < 2; m++) {
       if (gexec[m]) hipGraphExecDestroy(gexec[m]);
       if (graph[m]) hipGraphDestroy(graph[m]);

@@ -28,6 +28,21 @@ inline int corsr(int n) { return (n - 1) / 2 + 1; }
 // a level of dims d (the caller sizes the partials buffer with it).
 size_t max_partials(const Dim &d);
 
+// One contiguous piece of a result and where the caller wants it.
+struct HostSeg {
+  void *dst;
+  const void *src;
+  size_t bytes;
+};
+// Copies device segments to host memory after the work on s; returns when
+// they have landed (PMG_OK or PMG_EDEVICE).  Large copies to pageable
+// memory go through pinned rings that live as long as a context does
+// (ref / unref).  copy_host: the same threads, host to host.
+int copy_to_host(hipStream_t s, const HostSeg *seg, int n);
+void copy_host(void *dst, const void *src, size_t bytes);
+void host_ring_ref();
+void host_ring_unref();
+
 // Destination of a reduction computed alongside the kernel that produces
 // its terms: per-block partials (2 per block at most) and the device scalar
 // a final single-workgroup pass writes after summing them in block order.

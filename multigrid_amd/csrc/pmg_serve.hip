@@ -171,8 +171,8 @@ void copier_main(pmg_server *S) {
     S->copyq.pop_front();
     lk.unlock();
     const Params &p = r->ctx->p;
-    std::memcpy(r->u_out, r->ctx->u_pin,
-                sizeof(double) * (size_t)p.nx * p.ny * p.nz);
+    pmg::copy_host(r->u_out, r->ctx->u_pin,
+                   sizeof(double) * (size_t)p.nx * p.ny * p.nz);
     lk.lock();
     release_ctx(S, r->ctx);
     r->ctx = nullptr;

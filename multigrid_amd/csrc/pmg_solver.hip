@@ -1608,9 +1608,11 @@ int ctx_set_tru(pmg_ctx *c, const double *tcf) {
   return hipStreamSynchronize(c->s) == hipSuccess ? PMG_OK : PMG_EDEVICE;
 }
 
-// Fill iwork/rwork as the reference leaves them (mgdrvd.cc:145-166,
-// mgsubd.cc:266-373): iz, ipc per level; rpc | cc | fc | pc | ac.
-int export_work(pmg_ctx *c, int *iwork, double *rwork, bool newton) {
+// Copy out u and fill iwork/rwork as the reference leaves them
+// (mgdrvd.cc:145-166, mgsubd.cc:266-373): iz, ipc per level;
+// rpc | cc | fc | pc | ac.
+int export_work(pmg_ctx *c, int *iwork, double *rwork, double *u,
+                bool newton) {
   int sz[12];
   const Params &p = c->p;
   mgsz(p.mgcoar, p.mgdisc, p.mgsolv, p.nx, p.ny, p.nz, p.nlev, sz);
@@ -1657,34 +1659,40 @@ int export_work(pmg_ctx *c, int *iwork, double *rwork, bool newton) {
     if (lev == 1) ipcl[11] = 1;
   }
   size_t rtot = (size_t)sz[10] + (newton ? 2 * (size_t)nf : 0);
-  std::memset(rwork, 0, sizeof(double) * rtot);
   double *ccb = rwork + nrpc, *fcb = ccb + narr;
   double *after = fcb + narr + (newton ? 2 * (size_t)nf : 0);
   double *pcb = after, *acb = pcb + 27 * (size_t)narrc;
-  for (int lev = 1; lev <= p.nlev; lev++) {
-    Level &L = c->L[lev - 1];
-    size_t nl = L.d.n();
-    hipMemcpyAsync(ccb + IZ(1, lev) - 1, L.cc, nl * sizeof(double),
-                   hipMemcpyDeviceToHost, c->s);
-    hipMemcpyAsync(fcb + IZ(1, lev) - 1, L.fc, nl * sizeof(double),
-                   hipMemcpyDeviceToHost, c->s);
-    hipMemcpyAsync(acb + IZ(7, lev) - 1, L.ac,
-                   (lev == 1 ? 4 : 14) * nl * sizeof(double),
-                   hipMemcpyDeviceToHost, c->s);
-    if (lev > 1)
-      hipMemcpyAsync(pcb + IZ(11, lev - 1) - 1, L.pc,
-                     27 * nl * sizeof(double), hipMemcpyDeviceToHost, c->s);
-  }
+  HostSeg seg[4 * MAXLEV + 2];
+  int ns = 0;
+  auto out = [&](double *dst, const double *src, size_t cnt) {
+    seg[ns++] = HostSeg{dst, src, cnt * sizeof(double)};
+  };
+  // in the order of rwork, so that what lies between can be zeroed below
+  for (int lev = 1; lev <= p.nlev; lev++)
+    out(ccb + IZ(1, lev) - 1, c->L[lev - 1].cc, c->L[lev - 1].d.n());
+  for (int lev = 1; lev <= p.nlev; lev++)
+    out(fcb + IZ(1, lev) - 1, c->L[lev - 1].fc, c->L[lev - 1].d.n());
+  for (int lev = 2; lev <= p.nlev; lev++)
+    out(pcb + IZ(11, lev - 1) - 1, c->L[lev - 1].pc, 27 * c->L[lev - 1].d.n());
+  for (int lev = 1; lev <= p.nlev; lev++)
+    out(acb + IZ(7, lev) - 1, c->L[lev - 1].ac,
+        (lev == 1 ? 4 : 14) * c->L[lev - 1].d.n());
   if (p.mgsolv == 1) {  // factored band at ac(iz(7, nlev+1)) (mgsubd.cc:255)
     const Level &C = c->L[p.nlev - 1];
     const BandDims b = band_dims(C.d, C.numdia);
     int *ipcb = ipc + IZ(5, p.nlev + 1) - 1;  // buildBd.cc:82-85, 295
     ipcb[0] = b.n, ipcb[1] = b.m, ipcb[2] = b.lda, ipcb[3] = 1;
-    hipMemcpyAsync(acb + IZ(7, p.nlev + 1) - 1, c->band,
-                   (size_t)b.n * b.lda * sizeof(double),
-                   hipMemcpyDeviceToHost, c->s);
+    out(acb + IZ(7, p.nlev + 1) - 1, c->band, (size_t)b.n * b.lda);
   }
-  return hipStreamSynchronize(c->s) == hipSuccess ? PMG_OK : PMG_EDEVICE;
+  double *at = rwork, *const end = rwork + rtot;
+  for (int q = 0; q < ns; q++) {
+    double *d = (double *)seg[q].dst;
+    if (d > at) std::memset(at, 0, (d - at) * sizeof(double));
+    at = d + seg[q].bytes / sizeof(double);
+  }
+  if (end > at) std::memset(at, 0, (end - at) * sizeof(double));
+  out(u, c->u, c->L[0].d.n());
+  return copy_to_host(c->s, seg, ns);
 }
 
 int check_sizes(const Params &p, bool newton) {
@@ -1742,9 +1750,7 @@ int driver(int *iparm, double *rparm, int *iwork, double *rwork, double *u,
             : kind == 2 ? ctx_pcg(c, PMG_FP64, num_iters)
                         : ctx_solve(c, PMG_FP64);
   if (src == PMG_OK || src == PMG_ITMAX) {
-    hipMemcpyAsync(u, c->u, c->L[0].d.n() * sizeof(double),
-                   hipMemcpyDeviceToHost, c->s);
-    int erc = export_work(c, iwork, rwork, newton);
+    int erc = export_work(c, iwork, rwork, u, newton);
     if (erc) src = erc;
   }
   t_iters = c->iters;
@@ -2105,10 +2111,8 @@ int pmg_ctx_solve_group(pmg_ctx *const *ctx, int n, int mode) {
 
 int pmg_ctx_get_u(pmg_ctx *ctx, double *u) {
   if (!ctx || !u) return PMG_EBADPARM;
-  if (hipMemcpyAsync(u, ctx->u, ctx->L[0].d.n() * sizeof(double),
-                     hipMemcpyDeviceToHost, ctx->s) != hipSuccess)
-    return PMG_EDEVICE;
-  return hipStreamSynchronize(ctx->s) == hipSuccess ? PMG_OK : PMG_EDEVICE;
+  const pmg::HostSeg seg{u, ctx->u, ctx->L[0].d.n() * sizeof(double)};
+  return pmg::copy_to_host(ctx->s, &seg, 1);
 }
 
 int pmg_ctx_stats(pmg_ctx *ctx, int *iters, int *ierror, double *relres,
