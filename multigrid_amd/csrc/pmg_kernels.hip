@@ -2000,10 +2000,10 @@ __device__ inline void cg_load_row(const double *__restrict__ ac, size_t n,
 // times whatever has been reached.  Once r.r is 1e-40 of r0.r0 (or 0, where
 // that underflows) the iterations left move x by less than the condition
 // number times 1e-20 of its length, far under its last bit, so the loop
-// ends there with the x of iteration 100: after 39 to 78 iterations on the
-// coarsest levels of the benchmark workloads (condition 6 to 20).  A level
-// that converges too slowly for this (a condition beyond about 100) takes
-// all 100 as before.
+// ends there with the x of iteration 100: after about 75 iterations on the
+// coarsest levels of the benchmark workloads (condition 6 to 20), 45 with
+// the unit diagonal of k_cg_rows.  A level that converges too slowly for
+// this (a condition beyond about 100) takes all 100 as before.
 constexpr double CG_SETTLED = 1e-40;
 
 template <class T, int NPT, int ND>
@@ -2199,6 +2199,22 @@ __device__ __forceinline__ double cg_rcp(double x) {
 // us on 11^3 and 126 on 9^3 with two reductions, three divisions and three
 // barriers per iteration; 126 and 100 so; to a relative 1e-2 on 9^3 in FP32
 // cycles 19 and 10.5.
+//
+// ZT works on the operator scaled to a unit diagonal where that diagonal
+// spans at most CG_SPAN, for one pass over the couplings before the loop:
+// about 45 iterations until x has settled instead of 75 on the benchmark
+// workloads' 9^3 and 11^3 levels, and as close to the dense solution (4e-16
+// to 2e-15 of the largest value either way).  65^3 FP64 request 2224 -> 1990
+// us, Newton 4087 -> 3651.  The limit takes in a dielectric step of 2 : 78.54
+// (spans of 3 to 54, with Newton's term to 70).  Up to a span of 33 the
+// unscaled form settles within 100 iterations too on every level tried
+// (balls, half spaces, random media, unions of spheres, 9^3 to 13^3); from
+// 39 to 80 a low-dielectric region several coarse cells across can leave it
+// unsettled (4e-12 of the largest value for a ball on 11^3, 1e-7 for a half
+// space on 13^3), which the scaled form is not; beyond, the difference
+// grows (to 1e-2 at 8000) and the reference's iterates are kept.  The other
+// forms keep them everywhere: their criteria read the norm.
+constexpr float CG_SPAN = 96.f;
 extern __shared__ double cg_lds[];
 template <class T, bool WARM, bool ABS, bool ZT, int R>
 __device__ __forceinline__ void cg_rows_body(
@@ -2221,7 +2237,7 @@ __device__ __forceinline__ void cg_rows_body(
   for (size_t q = tid; q < n + R + 2; q += NTB) P[q] = 0.0;
   int pidx[R];
   bool val[R];
-  double xr[R], rr[R], pp[R], dg[R];
+  double xr[R], rr[R], pp[R], dg[R], sc[R];
   double cf[R][26];
   long long off[26];
 #pragma unroll
@@ -2250,6 +2266,53 @@ __device__ __forceinline__ void cg_rows_body(
                                   1, 1, -1, -1, 0, 1, -1, 0, 0, 1, 1, -1, -1};
   constexpr signed char DK[26] = {0, 0, 0, 0, 0, 0, 0, 0, 1, 1, 1, 1, 1,
                                   1, 1, 1, 1, -1, -1, -1, -1, -1, -1, -1, -1, -1};
+  // scale to a unit diagonal: the factors of the neighbours through P
+#pragma unroll
+  for (int r = 0; r < R; r++) sc[r] = 1.0;
+  if constexpr (ZT) {
+    __shared__ float span[CG_W][2];
+    float lo = HUGE_VALF, hi = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      lo = val[r] ? fminf(lo, (float)dg[r]) : lo;
+      hi = val[r] ? fmaxf(hi, (float)dg[r]) : hi;
+    }
+#pragma unroll
+    for (int m = 1; m < 64; m *= 2) {
+      lo = fminf(lo, __shfl_xor(lo, m, 64));
+      hi = fmaxf(hi, __shfl_xor(hi, m, 64));
+    }
+    if ((tid & 63) == 0) span[tid >> 6][0] = lo, span[tid >> 6][1] = hi;
+    __syncthreads();  // also: P and the slots are zero
+    for (int w = 0; w < NTB / 64; w++) {
+      lo = fminf(lo, span[w][0]);
+      hi = fmaxf(hi, span[w][1]);
+    }
+    if (hi <= CG_SPAN * lo) {
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        if (val[r]) P[pidx[r]] = sc[r] = 1.0 / sqrt(dg[r]);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int a = 0; a < 9; a++) {
+        double w[R + 2];
+#pragma unroll
+        for (int c = 0; c < R + 2; c++) w[c] = P[rb[a] + c];
+#pragma unroll
+        for (int q = 0; q < 26; q++) {
+          if (DJ[q] != (a % 3) - 1 || DK[q] != (a / 3) - 1) continue;
+#pragma unroll
+          for (int r = 0; r < R; r++) cf[r][q] *= sc[r] * w[r + 1 + DI[q]];
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        rr[r] *= sc[r];
+        dg[r] *= sc[r] * sc[r];
+      }
+    }
+  }
   double v[R];
   // v = A pp, pp being the thread's points of P (0 at points it lacks)
   auto stencil = [&]() __attribute__((always_inline)) {
@@ -2290,7 +2353,7 @@ __device__ __forceinline__ void cg_rows_body(
     }
   };
   double s4[4], t4[4];
-  __syncthreads();  // P and the slots are zero
+  __syncthreads();  // P and the slots are zero (ZT: the factors are read)
   if constexpr (WARM) {  // r = f - A x0
 #pragma unroll
     for (int r = 0; r < R; r++) pp[r] = xr[r];
@@ -2350,21 +2413,22 @@ __device__ __forceinline__ void cg_rows_body(
   }
 #pragma unroll
   for (int r = 0; r < R; r++)
-    if (val[r]) xout[pidx[r]] = (T)xr[r];
+    if (val[r]) xout[pidx[r]] = (T)(ZT ? sc[r] * xr[r] : xr[r]);
   // The Hackbusch-Reusken factor (x . f) / (x . A x) of the solution as
   // stored (mgcsd.cc:429-452; 0 when the denominator is 0): one more
   // application of the operator the threads hold, instead of a product
   // kernel on a level of a few hundred points (4.8 us each).
   if (damp) {
 #pragma unroll
-    for (int r = 0; r < R; r++) pp[r] = (double)(T)xr[r];
+    for (int r = 0; r < R; r++)
+      pp[r] = ZT ? (double)(T)(sc[r] * xr[r]) / sc[r] : (double)(T)xr[r];
     put(pp);
     __syncthreads();
     stencil();
     s4[0] = s4[1] = s4[2] = s4[3] = 0.0;
 #pragma unroll
     for (int r = 0; r < R; r++) {
-      if (val[r]) s4[0] += pp[r] * (double)f[pidx[r]];
+      if (val[r]) s4[0] += pp[r] * ((ZT ? sc[r] : 1.0) * (double)f[pidx[r]]);
       s4[1] += pp[r] * v[r];
     }
     cg_sum4(s4, slots, t4);
