@@ -108,6 +108,9 @@ struct pmg_ctx {
     int mode = PMG_FP64, iters = 0, rc = PMG_OK;
     int phase = 0;  // 0: start in flight, 1: iterating, 2: finishing
     bool done = true, pending = false;
+    // what the pending work is waited for by: the event, the host mirror of
+    // the denominator, that of the norm
+    bool by_event = false, wait_den = false, wait_nrm = false;
     double rsden = 1.0, rsnrm = 0.0;
   } ses;
   hipEvent_t cyc_ev = nullptr, t0_ev = nullptr, t1_ev = nullptr;

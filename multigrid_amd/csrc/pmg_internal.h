@@ -45,10 +45,12 @@ void host_ring_unref();
 
 // Destination of a reduction computed alongside the kernel that produces
 // its terms: per-block partials (2 per block at most) and the device scalar
-// a final single-workgroup pass writes after summing them in block order.
+// a final single-workgroup pass writes after summing them in block order;
+// that pass also stores it to host (pinned, coherent) when given.
 struct Red {
   double *part = nullptr;
   double *out = nullptr;
+  double *host = nullptr;
 };
 
 // ---- smoothers (pmgc/gsd.cc) ----

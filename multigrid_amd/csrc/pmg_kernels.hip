@@ -105,7 +105,8 @@ __device__ inline void red_store(const Red &r, double v0, double v1) {
 // t, t+1024, ...
 template <int NV, int MODE>
 __device__ __forceinline__ void red_final_body(const double *part,
-                                               unsigned nblk, double *out) {
+                                               unsigned nblk, double *out,
+                                               double *host) {
   __shared__ double lds[16];
   double a = 0.0, c = 0.0;
   for (unsigned q = threadIdx.x; q < nblk; q += 1024) {
@@ -115,24 +116,27 @@ __device__ __forceinline__ void red_final_body(const double *part,
   const double sa = block_sum<1024>(a, lds);
   const double sc = NV == 2 ? block_sum<1024>(c, lds) : 0.0;
   if (threadIdx.x == 0) {
-    if (MODE == 1)
-      out[0] = sc != 0.0 ? sa / sc : 0.0;
-    else if (MODE == 2)
-      out[0] = sc;
-    else
-      out[0] = sa;
+    const double v = MODE == 1   ? (sc != 0.0 ? sa / sc : 0.0)
+                     : MODE == 2 ? sc
+                                 : sa;
+    out[0] = v;
+    // the host waits for this one store, not for the kernel: nothing else
+    // it reads depends on it, so no fence
+    if (host)
+      __hip_atomic_store(host, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 template <int NV, int MODE>
 __global__ __launch_bounds__(1024) void k_red_final(const double *part,
-                                                    unsigned nblk,
-                                                    double *out) {
-  red_final_body<NV, MODE>(part, nblk, out);
+                                                    unsigned nblk, double *out,
+                                                    double *host) {
+  red_final_body<NV, MODE>(part, nblk, out, host);
 }
 
 template <int NV, int MODE>
 static void red_final(const Red &r, const dim3 &g, hipStream_t s) {
-  k_red_final<NV, MODE><<<1, 1024, 0, s>>>(r.part, g.x * g.y * g.z, r.out);
+  k_red_final<NV, MODE><<<1, 1024, 0, s>>>(r.part, g.x * g.y * g.z, r.out,
+                                          r.host);
 }
 
 // ---------------------------------------------------------------------------
@@ -3421,7 +3425,7 @@ struct A_rf {
 template <int NV, int MODE>
 __global__ __launch_bounds__(1024) void kb_red_final(const GTab<A_rf> t) {
   const A_rf &a = t.a[blockIdx.y];
-  red_final_body<NV, MODE>(a.part, a.nblk, a.out);
+  red_final_body<NV, MODE>(a.part, a.nblk, a.out, nullptr);
   if (threadIdx.x == 0 && a.out2) a.out2[0] = a.out[0];
 }
 

@@ -120,8 +120,42 @@ Red red_to(pmg_ctx *c, int slot) {
   return r;
 }
 
-// read a device scalar back (waits for the stream)
+// Stopping scalars reach the host by the reduction's own store to the
+// pinned mirror: the host marks the slot (host_arm) before it enqueues the
+// reduction and spins until the mark is gone.  A copy and an event behind
+// each iteration cost about 15 us of idle GPU before the next one could be
+// enqueued (33^3 mixed: 7 iterations of 100 us).
+constexpr uint64_t kAwait = 0xfff8c0dec0dec0deULL;  // a NaN no sum produces
+void host_arm(pmg_ctx *c, int slot) {
+  __atomic_store_n((uint64_t *)(c->hscal + slot), kAwait, __ATOMIC_RELEASE);
+}
+bool host_landed(const pmg_ctx *c, int slot) {
+  return __atomic_load_n((const uint64_t *)(c->hscal + slot),
+                         __ATOMIC_ACQUIRE) != kAwait;
+}
+// The slot's value once it has landed.  The spin is bounded: a long
+// iteration (or a device error) is waited for through the stream.
 double host_scalar(pmg_ctx *c, int slot) {
+  using clock = std::chrono::steady_clock;
+  const auto limit = clock::now() + std::chrono::milliseconds(2);
+  for (int q = 0; !host_landed(c, slot); q++) {
+    __builtin_ia32_pause();
+    if ((q & 63) == 63 && clock::now() > limit) {
+      hipStreamSynchronize(c->s);
+      break;
+    }
+  }
+  return c->hscal[slot];
+}
+Red red_host(pmg_ctx *c, int slot) {
+  Red r = red_to(c, slot);
+  r.host = c->hscal + slot;
+  host_arm(c, slot);
+  return r;
+}
+
+// a device scalar no reduction writes (waits for the stream)
+double copy_scalar(pmg_ctx *c, int slot) {
   hipMemcpyAsync(c->hscal + slot, c->scal + slot, sizeof(double),
                  hipMemcpyDeviceToHost, c->s);
   hipStreamSynchronize(c->s);
@@ -299,9 +333,8 @@ int linear_fp64(pmg_ctx *c, LV<double> *L, const double *frhs,
                 int *iters_out, double *rel_out, int l0 = 0) {
   Level &F = c->L[l0];
   double rsden = 1.0;
-  const Red rden = red_to(c, S_RSDEN), rnrm = red_to(c, S_RSNRM);
   if (istop == 1) {
-    nrm1<double>(F.d, frhs, rden, c->s);
+    nrm1<double>(F.d, frhs, red_host(c, S_RSDEN), c->s);
     rsden = host_scalar(c, S_RSDEN);
   }
   if (rsden == 0.0) rsden = 1.0;
@@ -309,6 +342,7 @@ int linear_fp64(pmg_ctx *c, LV<double> *L, const double *frhs,
   const int nlev = c->nlev - l0;
   if (nlev == 1) {  // direct coarse solve on the only level (mgcsd.cc:170-291)
     coarse_solve<double>(c, l0, F.ac, L[0].cc, frhs, L[0].x);
+    const Red rnrm = red_host(c, S_RSNRM);
     resid<double, double>(F.d, F.numdia, F.ac, L[0].cc, frhs, L[0].x,
                           (double *)nullptr, &rnrm, c->s, L[0].dg);
     rsnrm = host_scalar(c, S_RSNRM);
@@ -320,6 +354,7 @@ int linear_fp64(pmg_ctx *c, LV<double> *L, const double *frhs,
   do {
     vcycle<double>(c, L, frhs, c->L[c->nlev - 1].ac, cc64c, false, 0.0, nlev);
     iters++;
+    const Red rnrm = red_host(c, S_RSNRM);
     resid<double, double>(F.d, F.numdia, F.ac, L[0].cc, frhs, L[0].x,
                           (double *)nullptr, &rnrm, c->s, L[0].dg);
     rsnrm = host_scalar(c, S_RSNRM);
@@ -341,9 +376,8 @@ int linear_mixed(pmg_ctx *c, LV<double> *L64, LV<float> *L32,
                  double *rel_out, int l0 = 0) {
   Level &F = c->L[l0];
   double rsden = 1.0;
-  const Red rden = red_to(c, S_RSDEN), rnrm = red_to(c, S_RSNRM);
   if (istop == 1) {
-    nrm1<double>(F.d, frhs, rden, c->s);
+    nrm1<double>(F.d, frhs, red_host(c, S_RSDEN), c->s);
     rsden = host_scalar(c, S_RSDEN);
   }
   if (rsden == 0.0) rsden = 1.0;
@@ -364,6 +398,7 @@ int linear_mixed(pmg_ctx *c, LV<double> *L64, LV<float> *L32,
     }
     if (!added) add_correction<float>(F.d, L32[0].x, u, c->s);
     iters++;
+    const Red rnrm = red_host(c, S_RSNRM);
     resid<double, float>(F.d, F.numdia, F.ac, L64[0].cc, frhs, u, r32, &rnrm,
                          c->s, L64[0].dg);
     rsnrm = host_scalar(c, S_RSNRM);
@@ -405,7 +440,8 @@ int alloc_hierarchy(pmg_ctx *c) {
   c->u = c->alloc<double>(nf);
   c->part = c->alloc<double>(max_partials(c->L[0].d) * 2);
   c->scal = c->alloc<double>(16);
-  if (hipHostMalloc((void **)&c->hscal, 16 * sizeof(double)) != hipSuccess)
+  if (hipHostMalloc((void **)&c->hscal, 16 * sizeof(double),
+                    hipHostMallocCoherent) != hipSuccess)
     c->ok = false;
   return c->ok ? PMG_OK : PMG_ENOMEM;
 }
@@ -536,7 +572,7 @@ int setup_wait(pmg_ctx *c) {
   hipEventElapsedTime(&ms, c->su0_ev, c->su1_ev);
   c->setup_ms = ms;
   // the reference stops when Vdpbfa finds a non-positive pivot
-  if (c->p.mgsolv == 1 && host_scalar(c, S_BINFO) != 0.0) return PMG_ENOTSPD;
+  if (c->p.mgsolv == 1 && copy_scalar(c, S_BINFO) != 0.0) return PMG_ENOTSPD;
   return PMG_OK;
 }
 
@@ -651,7 +687,7 @@ void views(pmg_ctx *c, LV<double> *L64, LV<float> *L32, int mode) {
 // its product with A.
 void stop_measure(pmg_ctx *c, int slot) {
   Level &F = c->L[0];
-  const Red rd = red_to(c, slot);
+  const Red rd = red_host(c, slot);
   const int istop = c->p.istop;
   if (istop == 2) {
     stop_diff(F.d, 2, c->tru, c->u, nullptr, rd, c->s);
@@ -670,7 +706,7 @@ void step_body(pmg_ctx *c, int mode) {
   Level &F = c->L[0];
   const int nlev = c->nlev;
   const double *cc64c = c->L[nlev - 1].cc;
-  const Red rnrm = red_to(c, S_RSNRM);
+  const Red rnrm = red_host(c, S_RSNRM);
   // istop 0, 1: the L1 norm of the FP64 residual; 2-5 their own measure
   const bool resid_norm = c->p.istop <= 1;
   if (mode == PMG_MIXED) {
@@ -737,8 +773,7 @@ int capture(pmg_ctx *c, int mode) {
 
 // Start a solve: Vazeros + VfboundPMG00 on u (mgdrvd.cc:419, 439), the
 // stopping-test denominator (mgcsd.cc:133-163) and, for PMG_MIXED, the
-// first residual; the two scalars come back with the start event, which
-// lin_poll reads.  Never blocks.
+// first residual; lin_poll waits for the scalars.  Never blocks.
 int lin_begin(pmg_ctx *c, int mode) {
   const Params &p = c->p;
   Level &F = c->L[0];
@@ -773,10 +808,9 @@ int lin_begin(pmg_ctx *c, int mode) {
   if (p.istop == 4 || p.istop == 5) build_alg(c);
   fill<double>(c->u, F.d.n(), 0.0, c->s);
   if (p.istop == 1) {
-    const Red rden = red_to(c, S_RSDEN);
-    nrm1<double>(F.d, F.fc, rden, c->s);
+    nrm1<double>(F.d, F.fc, red_host(c, S_RSDEN), c->s);
   } else if (p.istop >= 3) {  // ||tru||_2^2, or tru . A tru (u = 0 here)
-    const Red rden = red_to(c, S_RSDEN);
+    const Red rden = red_host(c, S_RSDEN);
     if (p.istop == 5) {
       stop_diff(F.d, 5, c->tru, c->u, F.r, rden, c->s);
       dot_energy<double>(F.d, F.numdia, F.ac, F.cc, F.r, F.t, rden, c->s);
@@ -786,14 +820,19 @@ int lin_begin(pmg_ctx *c, int mode) {
   }
   if (mode == PMG_MIXED) {
     // residual of u = 0, the first right-hand side of the FP32 cycle
-    const Red rnrm = red_to(c, S_RSNRM);
+    const Red rnrm = red_host(c, S_RSNRM);
     resid<double, float>(F.d, F.numdia, F.ac, F.cc, F.fc, c->u, F.w032,
                          p.istop <= 1 ? &rnrm : nullptr, c->s, F.dg);
   }
-  // the two scalars and the band factor's info (slot S_BINFO)
-  hipMemcpyAsync(c->hscal, c->scal, 4 * sizeof(double), hipMemcpyDeviceToHost,
-                 c->s);
-  hipEventRecord(c->cyc_ev, c->s);
+  S.wait_den = p.istop == 1 || p.istop >= 3;
+  S.wait_nrm = mode == PMG_MIXED && p.istop <= 1;
+  // the band factor's info (slot S_BINFO), or nothing to read
+  S.by_event = p.mgsolv == 1 || !(S.wait_den || S.wait_nrm);
+  if (S.by_event) {
+    hipMemcpyAsync(c->hscal + S_BINFO, c->scal + S_BINFO, sizeof(double),
+                   hipMemcpyDeviceToHost, c->s);
+    hipEventRecord(c->cyc_ev, c->s);
+  }
   S.pending = true;
   return PMG_OK;
 }
@@ -801,13 +840,13 @@ int lin_begin(pmg_ctx *c, int mode) {
 void lin_enqueue(pmg_ctx *c) {
   auto &S = c->ses;
   if (S.done || S.pending || S.phase != 1) return;
+  S.by_event = S.wait_den = false;
+  S.wait_nrm = true;
+  host_arm(c, S_RSNRM);
   if (c->gexec[S.mode] && !c->ktime)
     hipGraphLaunch(c->gexec[S.mode], c->s);
   else
     step_body(c, S.mode);
-  hipMemcpyAsync(c->hscal + S_RSNRM, c->scal + S_RSNRM, sizeof(double),
-                 hipMemcpyDeviceToHost, c->s);
-  hipEventRecord(c->cyc_ev, c->s);
   S.pending = true;
 }
 
@@ -818,8 +857,12 @@ int lin_poll(pmg_ctx *c, bool wait) {
   if (S.done) return 1;
   if (!S.pending) return 0;
   if (wait) {
-    hipEventSynchronize(c->cyc_ev);
-  } else if (hipEventQuery(c->cyc_ev) != hipSuccess) {
+    if (S.by_event) hipEventSynchronize(c->cyc_ev);
+    if (S.wait_den) host_scalar(c, S_RSDEN);
+    if (S.wait_nrm) host_scalar(c, S_RSNRM);
+  } else if ((S.by_event && hipEventQuery(c->cyc_ev) != hipSuccess) ||
+             (S.wait_den && !host_landed(c, S_RSDEN)) ||
+             (S.wait_nrm && !host_landed(c, S_RSNRM))) {
     return 0;
   }
   S.pending = false;
@@ -1248,7 +1291,7 @@ int alloc_newton(pmg_ctx *c) {
 // r receives the residual.
 double nm_norm(pmg_ctx *c, int l, const double *x, double *r) {
   Level &F = c->L[l];
-  const Red rd = red_to(c, S_TMP);
+  const Red rd = red_host(c, S_TMP);
   nmresid(F.d, F.numdia, F.ac, F.cc, F.fc, x, r, &rd, c->s);
   return host_scalar(c, S_TMP);
 }
@@ -1386,7 +1429,7 @@ int ctx_newton(pmg_ctx *c, int mode) {
     if (!c->ok) return PMG_ENOMEM;
   }
   if (!coarse_fits(c)) return PMG_EBADPARM;
-  if (p.mgsolv == 1 && host_scalar(c, S_BINFO) != 0.0) return PMG_ENOTSPD;
+  if (p.mgsolv == 1 && copy_scalar(c, S_BINFO) != 0.0) return PMG_ENOTSPD;
   Level &F = c->L[0];
   const Dim d = F.d;
   hipStream_t s = c->s;
@@ -1528,9 +1571,8 @@ int ctx_pcg(pmg_ctx *c, int mode, int num_iters) {
     fill<float>(c->L[c->nlev - 1].x32, C.d.n(), 0.0f, s);
   else
     fill<double>(c->L[c->nlev - 1].x, C.d.n(), 0.0, s);
-  const Red rden = red_to(c, S_RSDEN), rn1 = red_to(c, S_PCG_RN1),
-            rpap = red_to(c, S_PCG_PAP);
-  nrm1<double>(d, F.fc, rden, s);
+  const Red rpap = red_host(c, S_PCG_PAP);
+  nrm1<double>(d, F.fc, red_host(c, S_RSDEN), s);
   double rsden = host_scalar(c, S_RSDEN);
   if (rsden == 0.0) rsden = 1.0;
   // r = f - A x0, s = M r, p = s, rs = r.s, pap = p.A p
@@ -1540,12 +1582,9 @@ int ctx_pcg(pmg_ctx *c, int mode, int num_iters) {
   dot_interior(d, r, sv, red_to(c, S_PCG_RS), s);
   matvec_dots<double>(d, F.numdia, F.ac, F.cc, pv, pv, q, nullptr, s);
   dot_interior(d, pv, q, rpap, s);
-  nrm1<double>(d, r, rn1, s);
-  hipMemcpyAsync(c->hscal + S_PCG_PAP, c->scal + S_PCG_PAP,
-                 2 * sizeof(double), hipMemcpyDeviceToHost, s);
-  hipStreamSynchronize(s);
-  const double pap0 = c->hscal[S_PCG_PAP];
-  double rel = c->hscal[S_PCG_RN1] / rsden;
+  nrm1<double>(d, r, red_host(c, S_PCG_RN1), s);
+  const double pap0 = host_scalar(c, S_PCG_PAP);
+  double rel = host_scalar(c, S_PCG_RN1) / rsden;
   int iters = 0, ierr = 0;
   if (pap0 != 0.0) {  // CG_Solver.h:124-125
     for (;;) {
@@ -1570,13 +1609,13 @@ int ctx_pcg(pmg_ctx *c, int mode, int num_iters) {
       matvec_dots<double>(d, F.numdia, F.ac, F.cc, pv, pv, q, nullptr, s);
       dot_interior(d, pv, q, rpap, s);
       if (num_iters == 0) {
-        nrm1<double>(d, r, rn1, s);
+        nrm1<double>(d, r, red_host(c, S_PCG_RN1), s);
         rel = host_scalar(c, S_PCG_RN1) / rsden;
       }
     }
   }
   // the reported residual: that of the final u
-  const Red rnrm = red_to(c, S_RSNRM);
+  const Red rnrm = red_host(c, S_RSNRM);
   resid<double, double>(d, F.numdia, F.ac, F.cc, F.fc, c->u, (double *)nullptr,
                         &rnrm, s);
   const double rsnrm = host_scalar(c, S_RSNRM);
