@@ -214,6 +214,10 @@ void axpy_interior(const Dim &d, double alpha, const T *x, T *y,
                    hipStream_t s);
 template <class TA, class TB>
 void convert(const TA *a, TB *b, size_t n, hipStream_t s);
+// The start of a mixed solve in one pass: u = 0, and the residual of that
+// iterate, f, as the FP32 right-hand side r (interior); red: its L1 norm.
+void start_mixed(const Dim &d, const double *f, float *r, double *u,
+                 const Red *red, hipStream_t s);
 // u(interior) += e(interior) (u FP64, e any type)
 template <class T>
 void add_correction(const Dim &d, const T *e, double *u, hipStream_t s);

@@ -2525,6 +2525,51 @@ void cg_class(const Dim &d, int numdia, const double *ac, const double *cc,
 }
 
 // ---------------------------------------------------------------------------
+// Start of a mixed solve.  At u = 0 the residual is f itself, so one pass
+// over f replaces the fill of u, the residual (six more arrays) and, where
+// the norm is wanted, the pass of k_nrm1.  Bound by the 20 bytes per point;
+// consecutive points of a plane across row ends, a grid of plane pieces of
+// ST_PTS points.  The residual of u = 0 took 265 us at 289^3 and 50 at
+// 161^3 (MI355X); Newton at 129^3, which starts 19 inner solves, spent 22 +
+// 6 us on each.
+// ---------------------------------------------------------------------------
+constexpr int ST_PTS = 1024;
+__global__ __launch_bounds__(256) void k_start_mixed(
+    int nx, int ny, int nz, const double *__restrict__ f,
+    float *__restrict__ r, double *__restrict__ u, Red rd, int do_red) {
+  __shared__ double red[4];
+  const unsigned pts = (unsigned)nx * ny;
+  const size_t p0 = (size_t)blockIdx.y * pts;
+  const bool kin = blockIdx.y > 0 && (int)blockIdx.y < nz - 1;
+  double acc = 0.0;
+#pragma unroll
+  for (int m = 0; m < ST_PTS / 256; m++) {
+    const unsigned q = blockIdx.x * ST_PTS + m * 256 + threadIdx.x;
+    if (q >= pts) break;
+    const int i = q % nx, j = q / nx;
+    u[p0 + q] = 0.0;
+    if (kin && i > 0 && i < nx - 1 && j > 0 && j < ny - 1) {
+      const double v = f[p0 + q];
+      r[p0 + q] = (float)v;
+      acc += fabs(v);
+    }
+  }
+  if (do_red) {
+    const double t = block_sum<256>(acc, red);
+    red_store<1>(rd, t, 0.0);
+  }
+}
+
+void start_mixed(const Dim &d, const double *f, float *r, double *u,
+                 const Red *red, hipStream_t s) {
+  const dim3 g(cdiv(d.nx * d.ny, ST_PTS), d.nz);
+  k_start_mixed<<<g, 256, 0, s>>>(d.nx, d.ny, d.nz, f, r, u,
+                                  red ? *red : Red{}, red ? 1 : 0);
+  if (red) red_final<1, 0>(*red, g, s);
+  check_launch("start_mixed");
+}
+
+// ---------------------------------------------------------------------------
 // Class-style PCG (CG_Solver.h:152-237): dot product and the two vector
 // updates, their coefficients read from device scalars so the loop needs
 // no host round trip.

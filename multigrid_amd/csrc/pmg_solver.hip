@@ -364,7 +364,8 @@ int linear_fp64(pmg_ctx *c, LV<double> *L, const double *frhs,
   return iters < itmax ? PMG_OK : PMG_ITMAX;
 }
 
-// Mixed precision: FP64 defect correction around FP32 V-cycles.
+// Mixed precision: FP64 defect correction around FP32 V-cycles, from u = 0
+// (set here).
 //   r = f - A u (FP64, stored as the FP32 right-hand side of the cycle)
 //   e = V-cycle_FP32(0, r);  u += e (FP64)
 // The stopping test is the FP64 L1 residual, made after each cycle as in
@@ -382,8 +383,7 @@ int linear_mixed(pmg_ctx *c, LV<double> *L64, LV<float> *L32,
   }
   if (rsden == 0.0) rsden = 1.0;
   float *r32 = F.w032;  // fine right-hand side of the FP32 cycle
-  resid<double, float>(F.d, F.numdia, F.ac, L64[0].cc, frhs, u, r32,
-                       (const Red *)nullptr, c->s, L64[0].dg);
+  start_mixed(F.d, frhs, r32, u, nullptr, c->s);
   double rsnrm = 0.0;
   int iters = 0;
   const int nlev = c->nlev - l0;
@@ -806,8 +806,16 @@ int lin_begin(pmg_ctx *c, int mode) {
   c->hist.clear();
   hipEventRecord(c->t0_ev, c->s);
   if (p.istop == 4 || p.istop == 5) build_alg(c);
-  fill<double>(c->u, F.d.n(), 0.0, c->s);
-  if (p.istop == 1) {
+  // mixed: u = 0 and the first right-hand side of the FP32 cycle, whose norm
+  // is the denominator of istop 1 too
+  const bool nrm_mixed = mode == PMG_MIXED && p.istop <= 1;
+  if (mode == PMG_MIXED) {
+    const Red rnrm = red_host(c, S_RSNRM);
+    start_mixed(F.d, F.fc, F.w032, c->u, nrm_mixed ? &rnrm : nullptr, c->s);
+  } else {
+    fill<double>(c->u, F.d.n(), 0.0, c->s);
+  }
+  if (p.istop == 1 && !nrm_mixed) {
     nrm1<double>(F.d, F.fc, red_host(c, S_RSDEN), c->s);
   } else if (p.istop >= 3) {  // ||tru||_2^2, or tru . A tru (u = 0 here)
     const Red rden = red_host(c, S_RSDEN);
@@ -818,14 +826,8 @@ int lin_begin(pmg_ctx *c, int mode) {
       stop_diff(F.d, 3, c->tru, c->u, nullptr, rden, c->s);
     }
   }
-  if (mode == PMG_MIXED) {
-    // residual of u = 0, the first right-hand side of the FP32 cycle
-    const Red rnrm = red_host(c, S_RSNRM);
-    resid<double, float>(F.d, F.numdia, F.ac, F.cc, F.fc, c->u, F.w032,
-                         p.istop <= 1 ? &rnrm : nullptr, c->s, F.dg);
-  }
-  S.wait_den = p.istop == 1 || p.istop >= 3;
-  S.wait_nrm = mode == PMG_MIXED && p.istop <= 1;
+  S.wait_nrm = nrm_mixed;
+  S.wait_den = (p.istop == 1 && !nrm_mixed) || p.istop >= 3;
   // the band factor's info (slot S_BINFO), or nothing to read
   S.by_event = p.mgsolv == 1 || !(S.wait_den || S.wait_nrm);
   if (S.by_event) {
@@ -874,11 +876,12 @@ int lin_poll(pmg_ctx *c, bool wait) {
       return 1;
     }
     // the stopping-test denominator (mgcsd.cc:133-157)
-    if (p.istop == 1) S.rsden = c->hscal[S_RSDEN];
+    if (p.istop == 1)
+      S.rsden = c->hscal[S.wait_nrm ? S_RSNRM : S_RSDEN];
     else if (p.istop == 2) S.rsden = std::sqrt((double)c->L[0].d.n());
     else if (p.istop >= 3) S.rsden = std::sqrt(c->hscal[S_RSDEN]);
     if (S.rsden == 0.0) S.rsden = 1.0;  // mgcsd.cc:154-157
-    const bool mixed_res = S.mode == PMG_MIXED && p.istop <= 1;
+    const bool mixed_res = S.wait_nrm;
     S.rsnrm = mixed_res ? c->hscal[S_RSNRM] : S.rsden;
     // mixed: while (iters < itmax && relres > errtol) may do nothing
     if (mixed_res && !(S.iters < p.itmax && S.rsnrm / S.rsden > p.errtol)) {
@@ -1352,16 +1355,17 @@ int newton_level(pmg_ctx *c, int mode, int l0, double *x, int itmax,
                 c->L[l - 1].cpr, c->L[l].rhs, c->L[l].cpr, c->L[l].pc, s,
                 nullptr, m32 ? c->L[l].cpr32 : nullptr);
     const double errtol_s = std::min(0.9 * xold, 1.0 * std::pow(xold, 2.0));
-    fill<double>(xtmp, nf, 0.0, s);
     int its = 0;
     double rel = 0.0;
     const double *cc64c = c->L[c->nlev - 1].cpr;
-    if (mode == PMG_MIXED)
+    if (mode == PMG_MIXED) {
       linear_mixed(c, L64 + l0, L32 + l0, w0n, cc64c, xtmp, 0, errtol_s,
                    1000, &its, &rel, l0);
-    else
+    } else {
+      fill<double>(xtmp, nf, 0.0, s);
       linear_fp64(c, L64 + l0, w0n, cc64c, 0, errtol_s, 1000, &its, &rel,
                   l0);
+    }
     if (idamp == 1) {  // damping (newtond.cc:313-376)
       xpay_interior(d, x, 1.0, xtmp, w1, s);
       xnew = nm_norm(c, l0, w1, w0n);
