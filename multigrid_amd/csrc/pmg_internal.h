@@ -177,9 +177,13 @@ void dot_interior(const Dim &d, const double *x, const double *y,
                   const Red &red, hipStream_t s);
 // x += (rs/pap) p, r -= (rs/pap) q; p = s + (rsn/rs) p (interior; device
 // scalars, a zero denominator gives a zero coefficient)
+// y = A x of the fine level and x . y; dg: oC + cc when precomputed.
+void matvec7_dot(const Dim &d, const double *ac, const double *cc,
+                 const double *dg, const double *x, double *y, const Red &red,
+                 hipStream_t s);
 void pcg_xr(const Dim &d, double *x, double *r, const double *p,
             const double *q, const double *rs, const double *pap,
-            hipStream_t s);
+            const Red *red, hipStream_t s);
 void pcg_p(const Dim &d, double *p, const double *sv, const double *rsn,
            const double *rs, hipStream_t s);
 

@@ -1061,8 +1061,11 @@ __global__ __launch_bounds__(256) void k_resid27(
 // the caches, every element is fetched once per tile.  The sum is
 // resid_body's, term for term, so r has the same bits; the L1 norm is
 // summed per thread over its planes, then over the workgroup.
+// MV: the product y = A x (into r; fc is not read) with its x.y in place of
+// the norm, matvec_dots_body's sum term for term: 161^3 FP64 57 + 14 (k_dot)
+// -> 36 us.
 constexpr int RM_TX = 64, RM_TY = 16;
-template <class T, class TO>
+template <class T, class TO, bool MV = false>
 __device__ __forceinline__ void resid7m_body(
     int nx, int ny, int nz, const T *__restrict__ ac,
     const T *__restrict__ fc, const T *__restrict__ x, TO *__restrict__ r,
@@ -1095,7 +1098,8 @@ __device__ __forceinline__ void resid7m_body(
   };
   auto load = [&](int q, Co &P) {
     const size_t p = at(q);
-    P.dg = dg[p], P.fc = fc[p], P.oE = oE[p], P.oN = oN[p], P.uC = uC[p];
+    P.dg = dg[p], P.oE = oE[p], P.oN = oN[p], P.uC = uC[p];
+    if constexpr (!MV) P.fc = fc[p];
   };
   // plane q in slot (q - kb) mod 5 of both rings; step k reads the operator
   // of planes k-1 (uC) and k and x of planes k-1, k, k+1; the operator is
@@ -1124,7 +1128,15 @@ __device__ __forceinline__ void resid7m_body(
     SE[s][ty][tx] = P.oE;
     SN[s][ty][tx] = P.oN;
     __syncthreads();
-    if (owned) {
+    if (MV && owned) {
+      const T v = -P.oN * SX[s][ty + 1][tx] -
+                  SN[s][ty - 1][tx] * SX[s][ty - 1][tx] -
+                  P.oE * SX[s][ty][tx + 1] -
+                  SE[s][ty][tx - 1] * SX[s][ty][tx - 1] - uCm * xm -
+                  P.uC * xp + P.dg * x0;
+      r[p0 + (size_t)(k - 1) * sz] = (TO)v;
+      acc += (double)x0 * (double)v;
+    } else if (owned) {
       const T v = P.fc + P.oN * SX[s][ty + 1][tx] +
                   SN[s][ty - 1][tx] * SX[s][ty - 1][tx] +
                   P.oE * SX[s][ty][tx + 1] +
@@ -1156,14 +1168,14 @@ __device__ __forceinline__ void resid7m_body(
     red_store_at<1>(rd, bid, tsum, 0.0);
   }
 }
-template <class T, class TO>
+template <class T, class TO, bool MV = false>
 __global__ __launch_bounds__(RM_TX *RM_TY) void k_resid7m(
     int nx, int ny, int nz, const T *__restrict__ ac,
     const T *__restrict__ fc, const T *__restrict__ x, TO *__restrict__ r,
     const T *__restrict__ dg, Red rd, int do_red, int kc, int gx, int gy,
     int gz) {
-  resid7m_body<T, TO>(nx, ny, nz, ac, fc, x, r, dg, rd, do_red, kc, gx, gy,
-                      gz, blockIdx.x);
+  resid7m_body<T, TO, MV>(nx, ny, nz, ac, fc, x, r, dg, rd, do_red, kc, gx,
+                          gy, gz, blockIdx.x);
 }
 
 // Launch shape of k_resid7m: one round of workgroups (one per compute
@@ -1478,6 +1490,25 @@ void matvec_dots(const Dim &d, int numdia, const T *ac, const T *cc,
                  hipStream_t s) {
   const unsigned nb = matvec_launch<T>(d, numdia, ac, cc, x, w0, y, red, s);
   if (red) red_final<2, 1>(*red, dim3(nb), s);
+}
+
+// y = A x of a 7-point level with x . y: the march where it serves the
+// residual (resid7m_fits), else the column kernel.
+void matvec7_dot(const Dim &d, const double *ac, const double *cc,
+                 const double *dg, const double *x, double *y, const Red &red,
+                 hipStream_t s) {
+  if (dg && resid7m_fits(d)) {
+    int kc, gx, gy, gz;
+    const unsigned nb = resid7m_shape(d, kc, gx, gy, gz);
+    k_resid7m<double, double, true><<<nb, dim3(RM_TX, RM_TY), 0, s>>>(
+        d.nx, d.ny, d.nz, ac, nullptr, x, y, dg, red, 1, kc, gx, gy, gz);
+    red_final<1, 0>(red, dim3(nb), s);
+  } else {
+    const unsigned nb =
+        matvec_launch<double>(d, 7, ac, cc, x, nullptr, y, &red, s);
+    red_final<2, 2>(red, dim3(nb), s);
+  }
+  check_launch("matvec7_dot");
 }
 
 template <class T>
@@ -2602,19 +2633,36 @@ void dot_interior(const Dim &d, const double *x, const double *y,
   check_launch("dot_interior");
 }
 
-// x += a p, r -= a q with a = rs / pap (0 when pap == 0), interior
+// x += a p, r -= a q with a = rs / pap (0 when pap == 0), interior; rd: the
+// L1 norm of the new r, in k_nrm1's order (a pass of its own took 10.6 us at
+// 161^3).
 __global__ __launch_bounds__(256) void k_pcg_xr(
     int nx, int ny, int nz, double *__restrict__ x, double *__restrict__ r,
     const double *__restrict__ p, const double *__restrict__ q,
-    const double *__restrict__ rs, const double *__restrict__ pap) {
+    const double *__restrict__ rs, const double *__restrict__ pap, Red rd,
+    int do_red) {
+  __shared__ double red[4];
   const int i = 2 + blockIdx.x * BX + threadIdx.x;
   const int j = 2 + blockIdx.y * BY + threadIdx.y;
-  const int k = 2 + blockIdx.z;
-  if (i > nx - 1 || j > ny - 1) return;
-  const double a = pap[0] == 0.0 ? 0.0 : rs[0] / pap[0];
-  const size_t o = ix(nx, ny, i, j, k);
-  x[o] += a * p[o];
-  r[o] -= a * q[o];
+  const int k0 = 2 + blockIdx.z * KCH;
+  double acc = 0.0;
+  if (i <= nx - 1 && j <= ny - 1) {
+    const double a = pap[0] == 0.0 ? 0.0 : rs[0] / pap[0];
+#pragma unroll
+    for (int kk = 0; kk < KCH; kk++) {
+      const int k = k0 + kk;
+      if (k > nz - 1) break;
+      const size_t o = ix(nx, ny, i, j, k);
+      x[o] += a * p[o];
+      const double v = r[o] - a * q[o];
+      r[o] = v;
+      acc += fabs(v);
+    }
+  }
+  if (do_red) {
+    const double t = block_sum<256>(acc, red);
+    red_store<1>(rd, t, 0.0);
+  }
 }
 
 // p = s + b p with b = rsn / rs (0 when rs == 0), interior
@@ -2633,9 +2681,11 @@ __global__ __launch_bounds__(256) void k_pcg_p(
 
 void pcg_xr(const Dim &d, double *x, double *r, const double *p,
             const double *q, const double *rs, const double *pap,
-            hipStream_t s) {
-  dim3 g(cdiv(d.nx - 2, BX), cdiv(d.ny - 2, BY), d.nz - 2);
-  k_pcg_xr<<<g, dim3(BX, BY), 0, s>>>(d.nx, d.ny, d.nz, x, r, p, q, rs, pap);
+            const Red *red, hipStream_t s) {
+  dim3 g(cdiv(d.nx - 2, BX), cdiv(d.ny - 2, BY), cdiv(d.nz - 2, KCH));
+  k_pcg_xr<<<g, dim3(BX, BY), 0, s>>>(d.nx, d.ny, d.nz, x, r, p, q, rs, pap,
+                                      red ? *red : Red{}, red ? 1 : 0);
+  if (red) red_final<1, 0>(*red, g, s);
   check_launch("pcg_xr");
 }
 

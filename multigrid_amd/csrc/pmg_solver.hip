@@ -1492,9 +1492,10 @@ void class_vcycle(pmg_ctx *c, LV<T> *L, const T *frhs) {
   const int last = bot ? nlev - 2 : nlev - 1;  // as vcycle
   for (int l = 0; l < last; l++) {
     const T *rhs = l == 0 ? frhs : L[l].w0;
-    smooth<T>(c, L[l], rhs, L[l].x, 2, 0, false, true);
+    // the fine iterate's boundary entries are zero already, as in vcycle
+    smooth<T>(c, L[l], rhs, L[l].x, 2, 0, false, true, l == 0);
     resid<T, T>(L[l].d, L[l].numdia, L[l].ac, L[l].cc, rhs, L[l].x, L[l].r,
-                nullptr, s);
+                nullptr, s, l == 0 ? L[0].dg : nullptr);
     restrict_<T>(L[l].d, L[l + 1].d, L[l].r, L[l + 1].w0, L[l + 1].pc, s);
   }
   const GBottom<T> gb = bottom_of<T>(c, L, nlev);
@@ -1577,21 +1578,21 @@ int ctx_pcg(pmg_ctx *c, int mode, int num_iters) {
     fill<double>(c->L[c->nlev - 1].x, C.d.n(), 0.0, s);
   const Red rpap = red_host(c, S_PCG_PAP);
   nrm1<double>(d, F.fc, red_host(c, S_RSDEN), s);
-  double rsden = host_scalar(c, S_RSDEN);
-  if (rsden == 0.0) rsden = 1.0;
-  // r = f - A x0, s = M r, p = s, rs = r.s, pap = p.A p
-  resid<double, double>(d, F.numdia, F.ac, F.cc, F.fc, c->u, r, nullptr, s);
+  const double nf1 = host_scalar(c, S_RSDEN);
+  const double rsden = nf1 == 0.0 ? 1.0 : nf1;
+  // r = f (x0 = 0), s = M r, p = s, rs = r.s, pap = p.A p
+  copy_interior(d, F.fc, r, s);
   pcg_precond(c, mode, L64, L32, r, sv);
   copy_interior(d, sv, pv, s);
   dot_interior(d, r, sv, red_to(c, S_PCG_RS), s);
-  matvec_dots<double>(d, F.numdia, F.ac, F.cc, pv, pv, q, nullptr, s);
-  dot_interior(d, pv, q, rpap, s);
-  nrm1<double>(d, r, red_host(c, S_PCG_RN1), s);
+  matvec7_dot(d, F.ac, F.cc, F.dg, pv, q, rpap, s);
   const double pap0 = host_scalar(c, S_PCG_PAP);
-  double rel = host_scalar(c, S_PCG_RN1) / rsden;
+  double rel = nf1 / rsden;
   int iters = 0, ierr = 0;
   if (pap0 != 0.0) {  // CG_Solver.h:124-125
     for (;;) {
+      // x and r are those of iteration `iters`; the next direction (a cycle
+      // and a product) is made only once it is known to be wanted
       if (num_iters > 0) {
         if (iters >= num_iters) break;
       } else {
@@ -1601,27 +1602,30 @@ int ctx_pcg(pmg_ctx *c, int mode, int num_iters) {
           break;
         }
       }
-      const double *rs_old = c->scal + S_PCG_RS + (iters & 1);
-      double *rs_new = c->scal + S_PCG_RS + ((iters + 1) & 1);
+      const double *rs_old = c->scal + S_PCG_RS + ((iters + 1) & 1);
+      double *rs_new = c->scal + S_PCG_RS + (iters & 1);
+      if (iters > 0) {
+        pcg_precond(c, mode, L64, L32, r, sv);
+        Red rrs = red_to(c, S_PCG_RS);
+        rrs.out = rs_new;
+        dot_interior(d, r, sv, rrs, s);
+        pcg_p(d, pv, sv, rs_new, rs_old, s);
+        matvec7_dot(d, F.ac, F.cc, F.dg, pv, q, rpap, s);
+      }
       iters++;
-      pcg_xr(d, c->u, r, pv, q, rs_old, c->scal + S_PCG_PAP, s);
-      pcg_precond(c, mode, L64, L32, r, sv);
-      Red rrs = red_to(c, S_PCG_RS);
-      rrs.out = rs_new;
-      dot_interior(d, r, sv, rrs, s);
-      pcg_p(d, pv, sv, rs_new, rs_old, s);
-      matvec_dots<double>(d, F.numdia, F.ac, F.cc, pv, pv, q, nullptr, s);
-      dot_interior(d, pv, q, rpap, s);
       if (num_iters == 0) {
-        nrm1<double>(d, r, red_host(c, S_PCG_RN1), s);
+        const Red rn1 = red_host(c, S_PCG_RN1);
+        pcg_xr(d, c->u, r, pv, q, rs_new, c->scal + S_PCG_PAP, &rn1, s);
         rel = host_scalar(c, S_PCG_RN1) / rsden;
+      } else {
+        pcg_xr(d, c->u, r, pv, q, rs_new, c->scal + S_PCG_PAP, nullptr, s);
       }
     }
   }
   // the reported residual: that of the final u
   const Red rnrm = red_host(c, S_RSNRM);
   resid<double, double>(d, F.numdia, F.ac, F.cc, F.fc, c->u, (double *)nullptr,
-                        &rnrm, s);
+                        &rnrm, s, F.dg);
   const double rsnrm = host_scalar(c, S_RSNRM);
   fbound_dirichlet(d, c->u, c->gx, c->gy, c->gz, s);
   hipEventRecord(e1, s);
