@@ -1063,12 +1063,14 @@ __global__ __launch_bounds__(256) void k_resid27(
 // summed per thread over its planes, then over the workgroup.
 // MV: the product y = A x (into r; fc is not read) with its x.y in place of
 // the norm, matvec_dots_body's sum term for term: 161^3 FP64 57 + 14 (k_dot)
-// -> 36 us.
+// -> 36 us.  DG false (the residual entry points on a caller's arrays): oC
+// and cc are read and added here; 161^3 FP64 -> FP32 with its norm 64.4 ->
+// 62.6 us a call against the column kernel.
 constexpr int RM_TX = 64, RM_TY = 16;
-template <class T, class TO, bool MV = false>
+template <class T, class TO, bool MV = false, bool DG = true>
 __device__ __forceinline__ void resid7m_body(
     int nx, int ny, int nz, const T *__restrict__ ac,
-    const T *__restrict__ fc, const T *__restrict__ x, TO *__restrict__ r,
+    const T *__restrict__ cc, const T *__restrict__ fc, const T *__restrict__ x, TO *__restrict__ r,
     const T *__restrict__ dg, const Red &rd, int do_red, int kc, int gx,
     int gy, int gz, unsigned bid) {
   __shared__ T SX[2][RM_TY][RM_TX], SE[2][RM_TY][RM_TX], SN[2][RM_TY][RM_TX];
@@ -1094,11 +1096,13 @@ __device__ __forceinline__ void resid7m_body(
   const size_t p0 = ix(nx, ny, min(i, nx), min(j, ny), 1);
   auto at = [&](int q) { return p0 + (size_t)(min(max(q, 1), nz) - 1) * sz; };
   struct Co {
-    T dg, fc, oE, oN, uC;
+    T dg, cc, fc, oE, oN, uC;  // dg: oC + cc, or oC without it
   };
   auto load = [&](int q, Co &P) {
     const size_t p = at(q);
-    P.dg = dg[p], P.oE = oE[p], P.oN = oN[p], P.uC = uC[p];
+    P.dg = DG ? dg[p] : ac[p];
+    if constexpr (!DG) P.cc = cc[p];
+    P.oE = oE[p], P.oN = oN[p], P.uC = uC[p];
     if constexpr (!MV) P.fc = fc[p];
   };
   // plane q in slot (q - kb) mod 5 of both rings; step k reads the operator
@@ -1141,7 +1145,7 @@ __device__ __forceinline__ void resid7m_body(
                   SN[s][ty - 1][tx] * SX[s][ty - 1][tx] +
                   P.oE * SX[s][ty][tx + 1] +
                   SE[s][ty][tx - 1] * SX[s][ty][tx - 1] + uCm * xm +
-                  P.uC * xp - P.dg * x0;
+                  P.uC * xp - (DG ? P.dg : P.dg + P.cc) * x0;
       if (r) r[p0 + (size_t)(k - 1) * sz] = (TO)v;
       acc += fabs((double)v);
     }
@@ -1168,14 +1172,14 @@ __device__ __forceinline__ void resid7m_body(
     red_store_at<1>(rd, bid, tsum, 0.0);
   }
 }
-template <class T, class TO, bool MV = false>
+template <class T, class TO, bool MV = false, bool DG = true>
 __global__ __launch_bounds__(RM_TX *RM_TY) void k_resid7m(
     int nx, int ny, int nz, const T *__restrict__ ac,
-    const T *__restrict__ fc, const T *__restrict__ x, TO *__restrict__ r,
+    const T *__restrict__ cc, const T *__restrict__ fc, const T *__restrict__ x, TO *__restrict__ r,
     const T *__restrict__ dg, Red rd, int do_red, int kc, int gx, int gy,
     int gz) {
-  resid7m_body<T, TO, MV>(nx, ny, nz, ac, fc, x, r, dg, rd, do_red, kc, gx,
-                          gy, gz, blockIdx.x);
+  resid7m_body<T, TO, MV, DG>(nx, ny, nz, ac, cc, fc, x, r, dg, rd, do_red,
+                              kc, gx, gy, gz, blockIdx.x);
 }
 
 // Launch shape of k_resid7m: one round of workgroups (one per compute
@@ -1190,7 +1194,7 @@ static unsigned resid7m_shape(const Dim &d, int &kc, int &gx, int &gy,
   return 8u * (unsigned)cdiv(gx * gy * gz, 8);
 }
 
-// The march serves a 7-point level with the precomputed diagonal when its
+// The march serves a 7-point level when its
 // tiles of RM_TX - 2 owned columns need no more tiles across i than
 // resid_body's blocks of BX columns, and its k chunks are long enough to
 // hide the four planes its rings load before the first result.  With 63
@@ -1214,13 +1218,18 @@ size_t resid_partials(const Dim &d) {
 template <class T, class TO>
 void resid(const Dim &d, int numdia, const T *ac, const T *cc, const T *fc,
            const T *x, TO *r, const Red *red, hipStream_t s, const T *dg) {
-  if (numdia == 7 && dg && resid7m_fits(d)) {
+  if (numdia == 7 && resid7m_fits(d)) {
     int kcm, gx, gy, gz;
     const unsigned nb = resid7m_shape(d, kcm, gx, gy, gz);
     const Red rdm = red ? *red : Red{};
-    k_resid7m<T, TO><<<nb, dim3(RM_TX, RM_TY), 0, s>>>(
-        d.nx, d.ny, d.nz, ac, fc, x, r, dg, rdm, red ? 1 : 0, kcm, gx, gy,
-        gz);
+    if (dg)
+      k_resid7m<T, TO><<<nb, dim3(RM_TX, RM_TY), 0, s>>>(
+          d.nx, d.ny, d.nz, ac, cc, fc, x, r, dg, rdm, red ? 1 : 0, kcm, gx,
+          gy, gz);
+    else
+      k_resid7m<T, TO, false, false><<<nb, dim3(RM_TX, RM_TY), 0, s>>>(
+          d.nx, d.ny, d.nz, ac, cc, fc, x, r, dg, rdm, red ? 1 : 0, kcm, gx,
+          gy, gz);
     if (red) red_final<1, 0>(rdm, dim3(nb), s);
     check_launch("resid");
     return;
@@ -1501,7 +1510,8 @@ void matvec7_dot(const Dim &d, const double *ac, const double *cc,
     int kc, gx, gy, gz;
     const unsigned nb = resid7m_shape(d, kc, gx, gy, gz);
     k_resid7m<double, double, true><<<nb, dim3(RM_TX, RM_TY), 0, s>>>(
-        d.nx, d.ny, d.nz, ac, nullptr, x, y, dg, red, 1, kc, gx, gy, gz);
+        d.nx, d.ny, d.nz, ac, nullptr, nullptr, x, y, dg, red, 1, kc, gx, gy,
+        gz);
     red_final<1, 0>(red, dim3(nb), s);
   } else {
     const unsigned nb =
@@ -3508,7 +3518,7 @@ __global__ __launch_bounds__(RM_TX *RM_TY) void kb_resid7m(
     const GTab<A_res<T, TO>> t) {
   const A_res<T, TO> &a = t.a[blockIdx.y];
   if (blockIdx.x >= a.nblk) return;
-  resid7m_body<T, TO>(a.nx, a.ny, a.nz, a.ac, a.fc, a.x, a.r, a.dg, a.rd,
+  resid7m_body<T, TO>(a.nx, a.ny, a.nz, a.ac, a.cc, a.fc, a.x, a.r, a.dg, a.rd,
                       a.do_red, a.kc, a.xg.gx, a.xg.gy, a.xg.gz, blockIdx.x);
 }
 
