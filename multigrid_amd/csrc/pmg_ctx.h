@@ -41,9 +41,9 @@ struct Level {
   double *x = nullptr, *w0 = nullptr, *r = nullptr, *t = nullptr;
   float *ac32 = nullptr, *cc32 = nullptr, *pc32 = nullptr, *x32 = nullptr,
         *w032 = nullptr, *r32 = nullptr, *t32 = nullptr;
-  // Newton: Jacobian diagonal term and right-hand side per level, and the
-  // Newton iterate of a coarse level (nested iteration)
-  double *cpr = nullptr, *rhs = nullptr, *xn = nullptr;
+  // Newton: Jacobian diagonal term per level, and the Newton iterate of a
+  // coarse level (nested iteration)
+  double *cpr = nullptr, *xn = nullptr;
   float *cpr32 = nullptr;
   // Newton, fine level: the diagonal oC + cpr of the Jacobian (FP64, and the
   // FP32 sum of the FP32 copies for mixed inner solves)

@@ -874,14 +874,15 @@ void gs27(const Dim &d, const T *ac, const T *cc, const T *fc, T *x,
 // ---------------------------------------------------------------------------
 // Residual (Vmresid7_1s / Vmresid27_1s) with optional L1 partial sums.
 // 7-point levels: one thread per (i, j) column of a chunk of kc planes (the
-// march k_resid7m below where it fits).
+// march k_resid7m below where it fits).  DG: the diagonal oC + cc comes
+// precomputed in dg (the same bits, one array less: DGFIG).
 // ---------------------------------------------------------------------------
-template <class T, class TO>
+template <class T, class TO, bool DG>
 __device__ __forceinline__ void resid_body(
     int nx, int ny, int nz, const T *__restrict__ ac,
     const T *__restrict__ cc, const T *__restrict__ fc,
-    const T *__restrict__ x, TO *__restrict__ r, Red rd, int do_red, int kc,
-    XG xg, unsigned bid) {
+    const T *__restrict__ x, TO *__restrict__ r, const T *__restrict__ dg,
+    Red rd, int do_red, int kc, XG xg, unsigned bid) {
   __shared__ double red[4];
   const size_t n = (size_t)nx * ny * nz, sy = nx, sz = (size_t)nx * ny;
   int bx, by, bz;
@@ -892,7 +893,7 @@ __device__ __forceinline__ void resid_body(
   double acc = 0.0;
   const T *oE = ac + n, *oN = ac + 2 * n, *uC = ac + 3 * n;
   auto value = [&](size_t p) -> T {
-    const T dgp = ac[p] + cc[p];
+    const T dgp = DG ? dg[p] : ac[p] + cc[p];
     return fc[p] + oN[p] * x[p + sy] + oN[p - sy] * x[p - sy] +
            oE[p] * x[p + 1] + oE[p - 1] * x[p - 1] + uC[p - sz] * x[p - sz] +
            uC[p] * x[p + sz] - dgp * x[p];
@@ -926,14 +927,14 @@ __device__ __forceinline__ void resid_body(
   }
 }
 
-template <class T, class TO>
+template <class T, class TO, bool DG>
 __global__ __launch_bounds__(256) void k_resid(
     int nx, int ny, int nz, const T *__restrict__ ac,
     const T *__restrict__ cc, const T *__restrict__ fc,
-    const T *__restrict__ x, TO *__restrict__ r, Red rd, int do_red, int kc,
-    XG xg) {
-  resid_body<T, TO>(nx, ny, nz, ac, cc, fc, x, r, rd, do_red, kc, xg,
-                    blockIdx.x);
+    const T *__restrict__ x, TO *__restrict__ r, const T *__restrict__ dg,
+    Red rd, int do_red, int kc, XG xg) {
+  resid_body<T, TO, DG>(nx, ny, nz, ac, cc, fc, x, r, dg, rd, do_red, kc, xg,
+                        blockIdx.x);
 }
 
 // Residual and operator product on 27-point levels: a thread takes pairs of
@@ -1246,8 +1247,12 @@ void resid(const Dim &d, int numdia, const T *ac, const T *cc, const T *fc,
   }
   const int kc = kchunk(d, red ? 40 : 80);
   dim3 g(cdiv(d.nx - 2, BX), cdiv(d.ny - 2, BY), cdiv(d.nz - 2, kc));
-  k_resid<T, TO><<<xcd_blocks(g), b, 0, s>>>(d.nx, d.ny, d.nz, ac, cc, fc, x,
-                                             r, rd, red ? 1 : 0, kc, xg_of(g));
+  if (dg)
+    k_resid<T, TO, true><<<xcd_blocks(g), b, 0, s>>>(
+        d.nx, d.ny, d.nz, ac, cc, fc, x, r, dg, rd, red ? 1 : 0, kc, xg_of(g));
+  else
+    k_resid<T, TO, false><<<xcd_blocks(g), b, 0, s>>>(
+        d.nx, d.ny, d.nz, ac, cc, fc, x, r, dg, rd, red ? 1 : 0, kc, xg_of(g));
   if (red) red_final<1, 0>(rd, dim3(xcd_blocks(g)), s);
   check_launch("resid");
 }
@@ -1566,8 +1571,7 @@ __device__ __forceinline__ bool pr_pair(const PR &s, unsigned bid, int rows,
   return row < rows;
 }
 
-// NS sources restricted in one pass (the setup's cc and fc; Newton's
-// right-hand side and Jacobian term): every P plane is loaded once for all of
+// NS sources restricted in one pass (the setup's cc and fc): every P plane is loaded once for all of
 // them; each sum keeps its term order, so the results do not depend on NS.
 template <class T, int NS>
 struct RSrc {
@@ -3497,12 +3501,12 @@ struct A_res {
   const T *dg;
   P27 s27;
 };
-template <class T, class TO>
+template <class T, class TO, bool DG>
 __global__ __launch_bounds__(256) void kb_resid(const GTab<A_res<T, TO>> t) {
   const A_res<T, TO> &a = t.a[blockIdx.y];
   if (blockIdx.x >= a.nblk) return;
-  resid_body<T, TO>(a.nx, a.ny, a.nz, a.ac, a.cc, a.fc, a.x, a.r, a.rd,
-                    a.do_red, a.kc, a.xg, blockIdx.x);
+  resid_body<T, TO, DG>(a.nx, a.ny, a.nz, a.ac, a.cc, a.fc, a.x, a.r, a.dg,
+                        a.rd, a.do_red, a.kc, a.xg, blockIdx.x);
 }
 template <class T, class TO>
 __global__ __launch_bounds__(256) void kb_resid27(const GTab<A_res<T, TO>> t) {
@@ -3537,16 +3541,18 @@ __global__ __launch_bounds__(1024) void kb_red_final(const GTab<A_rf> t) {
 template <class T, class TO>
 void g_resid(const GResid<T, TO> *j, int n, hipStream_t s) {
   if (n <= 0) return;
+  std::vector<char> march(n, 0);
   std::vector<A_res<T, TO>> a(n);
   for (int q = 0; q < n; q++) {  // the launch shape of resid
     const Dim &d = j[q].d;
     const bool red = j[q].red != nullptr;
-    const T *dg = j[q].numdia == 7 && resid7m_fits(d) ? j[q].dg : nullptr;
+    const T *dg = j[q].numdia == 7 ? j[q].dg : nullptr;
+    march[q] = dg && resid7m_fits(d);
     int kc = 0;
     XG xg{};
     unsigned nblk;
     P27 s27{};
-    if (dg) {
+    if (march[q]) {
       nblk = resid7m_shape(d, kc, xg.gx, xg.gy, xg.gz);
     } else if (j[q].numdia == 27) {
       s27 = p27_shape(d);
@@ -3562,22 +3568,25 @@ void g_resid(const GResid<T, TO> *j, int n, hipStream_t s) {
                         red ? *j[q].red : Red{}, red ? 1 : 0, kc,
                         xg,      nblk,    dg,     s27};
   }
-  // variant key: 7 (7-point), 8 (7-point with dg), 26 + wavefronts per
-  // workgroup (27-point)
+  // variant key: 7 (7-point), 8 (7-point with dg), 9 (its march), 26 +
+  // wavefronts per workgroup (27-point)
   g_split<A_res<T, TO>>(
       n,
       [&](int q) {
-        return j[q].numdia == 7 ? (a[q].dg ? 8 : 7) : 26 + a[q].s27.rows;
+        return j[q].numdia == 7 ? (march[q] ? 9 : a[q].dg ? 8 : 7)
+                                : 26 + a[q].s27.rows;
       },
       [&](int q) { return a[q]; },
       [&](const GTab<A_res<T, TO>> &t, int m, int key) {
         unsigned mx = 0;
         for (int q = 0; q < m; q++) mx = std::max(mx, t.a[q].nblk);
         const dim3 grid(mx, m), b(BX, BY);
-        if (key == 8)
+        if (key == 9)
           kb_resid7m<T, TO><<<grid, dim3(RM_TX, RM_TY), 0, s>>>(t);
+        else if (key == 8)
+          kb_resid<T, TO, true><<<grid, b, 0, s>>>(t);
         else if (key == 7)
-          kb_resid<T, TO><<<grid, b, 0, s>>>(t);
+          kb_resid<T, TO, false><<<grid, b, 0, s>>>(t);
         else
           kb_resid27<T, TO><<<grid, dim3(BX, key - 26), 0, s>>>(t);
       });

@@ -1279,7 +1279,6 @@ int alloc_newton(pmg_ctx *c) {
   for (int l = 0; l < c->nlev; l++) {
     Level &L = c->L[l];
     L.cpr = c->alloc<double>(L.d.n());
-    L.rhs = c->alloc<double>(L.d.n());
     if (l == 0) L.dgn = c->alloc<double>(L.d.n());
     // the Newton iterate of a coarse level (nested iteration, mgkey 1)
     if (l > 0 && c->p.mgkey == 1) L.xn = c->alloc<double>(L.d.n());
@@ -1343,7 +1342,8 @@ int newton_level(pmg_ctx *c, int mode, int l0, double *x, int itmax,
     iters++;
     // Vgetjac (newtond.cc:488-531)
     // the right-hand side of the Newton correction is the nonlinear
-    // residual w0n itself (interior; the boundary is zero), read in place;
+    // residual w0n itself (interior; the boundary is zero), read in place:
+    // the cycles restrict their own residuals, so no coarse level needs it;
     // the FP32 copies of the Helmholtz term for mixed inner solves are
     // written by the kernels that produce it
     const bool m32 = mode == PMG_MIXED;
@@ -1351,9 +1351,9 @@ int newton_level(pmg_ctx *c, int mode, int l0, double *x, int itmax,
            fine7 ? F.ac : nullptr, fine7 ? F.dgn : nullptr,
            fine7 && m32 ? F.ac32 : nullptr, fine7 && m32 ? F.dgn32 : nullptr);
     for (int l = l0 + 1; l < c->nlev; l++)
-      restrict2(c->L[l - 1].d, c->L[l].d, l - 1 == l0 ? w0n : c->L[l - 1].rhs,
-                c->L[l - 1].cpr, c->L[l].rhs, c->L[l].cpr, c->L[l].pc, s,
-                nullptr, m32 ? c->L[l].cpr32 : nullptr);
+      restrict_<double>(c->L[l - 1].d, c->L[l].d, c->L[l - 1].cpr,
+                        c->L[l].cpr, c->L[l].pc, s,
+                        m32 ? c->L[l].cpr32 : nullptr);
     const double errtol_s = std::min(0.9 * xold, 1.0 * std::pow(xold, 2.0));
     int its = 0;
     double rel = 0.0;
