@@ -10,8 +10,8 @@
 // Threads live for one call only (about 20 us each to start), which leaves
 // no state behind; below kLeast bytes they cost more than they save and the
 // runtime's copy is used.  A potential to a new array (MI355X, 16 cores):
-// 289^3 (193 MB) 18.8 -> 5.2 ms, 161^3 (33 MB) 2.19 -> 1.0, 129^3 1.14 ->
-// 0.6, 97^3 (7 MB) 0.53 -> 0.3.
+// 289^3 (193 MB) 18.8 -> 4.1 ms, 161^3 (33 MB) 2.19 -> 0.88, 129^3 1.14 ->
+// 0.56, 97^3 (7 MB) 0.53 -> 0.26.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -30,6 +30,7 @@ namespace {
 
 constexpr size_t kPiece = (size_t)2 << 20;
 constexpr size_t kLeast = (size_t)4 << 20;
+constexpr size_t kTwoStreams = (size_t)32 << 20;
 constexpr int kThreads = 8, kSlots = 2 * kThreads;
 
 // Pinned rings (kSlots * kPiece = 32 MB), at most kRings of them, made when
@@ -40,6 +41,13 @@ std::mutex ring_mu;
 struct Ring {
   char *p = nullptr;
   bool busy = false;
+  // a second stream (of device dev) for every other piece of a large copy:
+  // between two copies of one stream the link idles about 19 us (289^3 5000
+  // -> 4130 us, the drop-in's 45 MB in 20 arrays 9.0 -> 6.6 ms a call).
+  // From kTwoStreams on: with 17 MB the solve that follows lost more to the
+  // further stream (129^3 Newton 8234 -> 8490 us) than the copy gained
+  hipStream_t s2 = nullptr;
+  int dev = -1;
 } rings[kRings];
 int ring_users = 0;
 
@@ -107,18 +115,34 @@ int copy_plain(hipStream_t s, const HostSeg *seg, int n) {
   return hipStreamSynchronize(s) == hipSuccess && ok ? PMG_OK : PMG_EDEVICE;
 }
 
-int copy_pieces(hipStream_t s, const std::vector<HostSeg> &pc, char *ring,
-                int nt) {
+int copy_pieces(hipStream_t s, const std::vector<HostSeg> &pc, Ring &r, int nt,
+                bool two) {
   int dev = 0;
-  hipEvent_t ev[kSlots] = {};
+  char *const ring = r.p;
+  hipEvent_t ev[kSlots] = {}, start = nullptr;
   std::atomic<bool> ok{hipGetDevice(&dev) == hipSuccess};
   const int np = (int)pc.size(), ns = 2 * nt;
+  // the second stream starts behind what s holds already
+  hipStream_t st[2] = {s, s};
+  if (ok && two && !r.s2) {
+    if (hipStreamCreateWithFlags(&r.s2, hipStreamNonBlocking) == hipSuccess) {
+      r.dev = dev;
+    } else {
+      hipGetLastError();
+      r.s2 = nullptr;
+    }
+  }
+  if (ok && two && r.s2 && r.dev == dev &&
+      hipEventCreateWithFlags(&start, hipEventDisableTiming) == hipSuccess &&
+      hipEventRecord(start, s) == hipSuccess &&
+      hipStreamWaitEvent(r.s2, start, 0) == hipSuccess)
+    st[1] = r.s2;
   // slot q % ns holds piece q; piece q is thread (q % nt)'s
   auto fetch = [&](int q) {
     const int b = q % ns;
     if (hipMemcpyAsync(ring + b * kPiece, pc[q].src, pc[q].bytes,
-                       hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipEventRecord(ev[b], s) != hipSuccess)
+                       hipMemcpyDeviceToHost, st[q & 1]) != hipSuccess ||
+        hipEventRecord(ev[b], st[q & 1]) != hipSuccess)
       ok = false;
   };
   for (int b = 0; b < ns; b++)
@@ -138,9 +162,11 @@ int copy_pieces(hipStream_t s, const std::vector<HostSeg> &pc, char *ring,
     }
   });
   // nothing may still write the ring, also after a failure
-  if (hipStreamSynchronize(s) != hipSuccess) ok = false;
+  for (hipStream_t t : st)
+    if (hipStreamSynchronize(t) != hipSuccess) ok = false;
   for (hipEvent_t e : ev)
     if (e) hipEventDestroy(e);
+  if (start) hipEventDestroy(start);
   return ok ? PMG_OK : PMG_EDEVICE;
 }
 
@@ -156,8 +182,9 @@ void host_ring_unref() {
   if (--ring_users) return;
   for (Ring &r : rings)
     if (r.p && !r.busy) {
+      if (r.s2) hipStreamDestroy(r.s2);
       hipHostFree(r.p);
-      r.p = nullptr;
+      r = Ring{};
     }
 }
 
@@ -180,7 +207,8 @@ int copy_to_host(hipStream_t s, const HostSeg *seg, int n) {
   }
   Ring *r = ring_take();
   if (!r) return copy_plain(s, seg, n);
-  const int rc = copy_pieces(s, pc, r->p, threads_for(pc.size()));
+  const int rc = copy_pieces(s, pc, *r, threads_for(pc.size()),
+                             total >= kTwoStreams);
   ring_give(r);
   return rc;
 }

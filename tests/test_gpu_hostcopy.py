@@ -17,14 +17,16 @@ D = ctypes.POINTER(ctypes.c_double)
 
 @pytest.mark.parametrize("n,nlev", [(65, 4), (81, 4), (97, 5), (145, 5), (161, 5), (193, 6)])
 def test_potential_pageable_and_pinned(mg, n, nlev):
-    import torch
     print(f"host copy n={n}", flush=True)
     iparm, rparm = mg.make_params(n, nlev)
     ctx = mg.Context(iparm, rparm, pbe=(0.5, 0.15, mg.pbe_molecule(100, 12.0, 0, 3)))
     ctx.solve(mg.PMG_FP64)
-    pinned = torch.empty(n ** 3, dtype=torch.float64, pin_memory=True)
-    assert mg.lib().pmg_ctx_get_u(ctx._h, ctypes.cast(pinned.data_ptr(), D)) == 0
-    want = pinned.numpy()
+    hip = ctypes.CDLL("libamdhip64.so.7")  # the runtime the library uses
+    pinned = ctypes.c_void_p()
+    assert hip.hipHostMalloc(ctypes.byref(pinned), ctypes.c_size_t(8 * n ** 3), 0) == 0
+    assert mg.lib().pmg_ctx_get_u(ctx._h, ctypes.cast(pinned, D)) == 0
+    want = np.ctypeslib.as_array(ctypes.cast(pinned, D), (n ** 3,)).copy()
+    assert hip.hipHostFree(pinned) == 0
     assert np.any(want != 0.0)
     odd = np.full(n ** 3 + 3, np.nan)  # not page aligned, neighbours kept
     assert mg.lib().pmg_ctx_get_u(ctx._h, odd[1:].ctypes.data_as(D)) == 0
