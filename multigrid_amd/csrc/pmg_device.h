@@ -220,7 +220,13 @@ __device__ __forceinline__ void g27_rows(const T *xN, const T *xU,
 }
 
 // The terms of one point that do not involve the two in-row neighbours,
-// summed in the reference's order as far as they go.
+// summed in the reference's order as far as they go.  The multiply-adds are
+// written out: of a sum of two products the compiler may round either one
+// first, and its choice differed between the colours of a sweep (1 of 14
+// points an ulp off after two FP32 sweeps).  The coarsest CG of a mixed
+// cycle stops after up to 25 iterations at 1e-2, where its iterates have
+// grown such an ulp into a different iteration count now and then, which
+// moves a potential by up to 1.4e-9 of its norm.
 template <class T>
 struct G27Part {
   T a;             // oN(p) x(p+sy) + oN(p-sy) x(p-sy): the first two terms
@@ -235,7 +241,7 @@ __device__ __forceinline__ G27Part<T> g27_part(const G27C<T> &r,
                                                const G27X<T> &x, bool zN) {
   auto Z = [](T v, bool z) -> T { return z ? (T)0 : v; };
   G27Part<T> g;
-  g.a = r.cN[s] * Z(x.xN[s + 1], zN) + r.cS[s] * Z(x.xS[s + 1], zN);
+  g.a = fma(r.cN[s], Z(x.xN[s + 1], zN), r.cS[s] * Z(x.xS[s + 1], zN));
   g.cE = r.cE[s];
   g.cW = s ? r.cE[0] : r.cW;
   const T xv[4] = {x.xN[s + 2], x.xN[s], x.xS[s + 2], x.xS[s]};
@@ -245,12 +251,13 @@ __device__ __forceinline__ G27Part<T> g27_part(const G27C<T> &r,
   // in it
   constexpr int tr[9] = {0, 1, 2, 0, 0, 1, 1, 2, 2};
   constexpr int te[9] = {1, 1, 1, 2, 0, 2, 0, 2, 0};
-  T u = r.cu[0][s] * x.xu[0][s + 1];
+  T u = fma(r.cu[0][s], x.xu[0][s + 1], r.cu[1][s] * x.xu[1][s + 1]);
+  T dd = fma(r.cd[0][s], x.xd[0][s + 1], r.cd[1][s] * x.xd[1][s + 1]);
 #pragma unroll
-  for (int m = 1; m < 9; m++) u += r.cu[m][s] * x.xu[tr[m]][s + te[m]];
-  T dd = r.cd[0][s] * x.xd[0][s + 1];
-#pragma unroll
-  for (int m = 1; m < 9; m++) dd += r.cd[m][s] * x.xd[tr[m]][s + te[m]];
+  for (int m = 2; m < 9; m++) {
+    u = fma(r.cu[m][s], x.xu[tr[m]][s + te[m]], u);
+    dd = fma(r.cd[m][s], x.xd[tr[m]][s + te[m]], dd);
+  }
   g.u = u;
   g.dd = dd;
   g.dg = r.oC[s] + r.cc[s];
@@ -259,8 +266,10 @@ __device__ __forceinline__ G27Part<T> g27_part(const G27C<T> &r,
 // The in-plane sum from the part and the in-row neighbours xw, xe.
 template <class T>
 __device__ __forceinline__ T g27_plane(const G27Part<T> &g, T xw, T xe) {
-  return g.a + g.cE * xe + g.cW * xw + g.c[0] * g.xv[0] + g.c[1] * g.xv[1] +
-         g.c[2] * g.xv[2] + g.c[3] * g.xv[3];
+  T o = fma(g.cW, xw, fma(g.cE, xe, g.a));
+#pragma unroll
+  for (int m = 0; m < 4; m++) o = fma(g.c[m], g.xv[m], o);
+  return o;
 }
 
 __host__ __device__ inline int count_parity(int n, int par) {  // #{v in [2, n-1] : v%2 == par}
