@@ -229,6 +229,8 @@ __global__ __launch_bounds__(BOT_NT<T>) void k_bottom_down(
   const int ni = cx - 2, nj = cy - 2, nint = ni * nj * (cz - 2);
   const size_t nc = (size_t)cx * cy * cz;
   for (int q = tid; q < nint; q += BOT_NT<T>) {
+    // separate multiplies and adds, as restrict_body: the same bits
+#pragma clang fp contract(off)
     const int ii = 2 + q % ni, jj = 2 + (q / ni) % nj, kk = 2 + q / (ni * nj);
     const size_t pC = ix(cx, cy, ii, jj, kk);
     const int f = (int)ix(nx, ny, 2 * ii - 1, 2 * jj - 1, 2 * kk - 1);
@@ -274,11 +276,13 @@ __global__ __launch_bounds__(BOT_NT<T>) void k_bottom_up(
       T v[8];
       // fine point (di, dj, dk) of the cell: the corners e <= d that can
       // reach it, in the order x, y, z of the reference's sums; P plane of
-      // the offset from the corner's fine point
+      // the offset from the corner's fine point.  Multiply-adds written out
+      // as interp_body's are, the first product on top of the second
 #pragma unroll
       for (int d = 0; d < 8; d++) {
         const int dx = d & 1, dy = (d >> 1) & 1, dz = d >> 2;
-        T acc = (T)0;
+        T acc = (T)0, w0 = (T)0, x0 = (T)0;
+        int m = 0;
 #pragma unroll
         for (int e = 0; e < 8; e++) {
           const int ex = e & 1, ey = (e >> 1) & 1, ez = e >> 2;
@@ -287,16 +291,24 @@ __global__ __launch_bounds__(BOT_NT<T>) void k_bottom_up(
                     oz = dz ? (ez ? -1 : 1) : 0;
           const size_t pe = c0 + ex + (size_t)ey * cx + (size_t)ez * cx * cy;
           const T x = a.xc[pe];
-          acc += d == 0 ? x : a.pc[(size_t)pplane(ox, oy, oz) * nc + pe] * x;
+          const T w = d ? a.pc[(size_t)pplane(ox, oy, oz) * nc + pe] : (T)1;
+          if (m == 0)
+            w0 = w, x0 = x;
+          else
+            acc = m == 1 ? fma(w0, x0, w * x) : fma(w, x, acc);
+          m++;
         }
+        if (d == 0) acc = x0;
         v[d] = acc;
       }
       const int i = 2 * ii - 1, j = 2 * jj - 1, k = 2 * kk - 1;
 #pragma unroll
       for (int d = 0; d < 8; d++) {
         const int fi = i + (d & 1), fj = j + ((d >> 1) & 1), fk = k + (d >> 2);
-        if (fi >= 2 && fj >= 2 && fk >= 2)
-          X[(int)ix(nx, ny, fi, fj, fk)] += damp * v[d];
+        if (fi >= 2 && fj >= 2 && fk >= 2) {
+          T &x = X[(int)ix(nx, ny, fi, fj, fk)];
+          x = fma(damp, v[d], x);
+        }
       }
     }
   }

@@ -1788,20 +1788,25 @@ __device__ __forceinline__ void interp_body(int nxc, int nyc, int nzc,
     const T x000 = x[0][e], x100 = x[0][e + 1], x010 = x[1][e],
             x110 = x[1][e + 1], x001 = x[2][e], x101 = x[2][e + 1],
             x011 = x[3][e], x111 = x[3][e + 1];
+    // two, four and eight terms in the reference's order; the multiply-adds
+    // are written out, the first product on top of the second, so that they
+    // do not hang on the compiler's choice of which to round first
+    auto two = [&](int a, T xa, int b, T xb) {
+      return fma(w[a][e], xa, w[b][e] * xb);
+    };
+    auto add = [&](T s, int a, T xa) { return fma(w[a][e], xa, s); };
     v[0][2 * e] = x000;
-    v[0][2 * e + 1] = w[oPE][e] * x000 + w[oPW][e] * x100;
-    v[1][2 * e] = w[oPN][e] * x000 + w[oPS][e] * x010;
-    v[2][2 * e] = w[uPC][e] * x000 + w[dPC][e] * x001;
-    v[1][2 * e + 1] = w[oPNE][e] * x000 + w[oPNW][e] * x100 +
-                      w[oPSE][e] * x010 + w[oPSW][e] * x110;
-    v[2][2 * e + 1] = w[uPE][e] * x000 + w[uPW][e] * x100 + w[dPE][e] * x001 +
-                      w[dPW][e] * x101;
-    v[3][2 * e] = w[uPN][e] * x000 + w[uPS][e] * x010 + w[dPN][e] * x001 +
-                  w[dPS][e] * x011;
-    v[3][2 * e + 1] = +w[uPNE][e] * x000 + w[uPNW][e] * x100 +
-                      w[uPSE][e] * x010 + w[uPSW][e] * x110 +
-                      w[dPNE][e] * x001 + w[dPNW][e] * x101 +
-                      w[dPSE][e] * x011 + w[dPSW][e] * x111;
+    v[0][2 * e + 1] = two(oPE, x000, oPW, x100);
+    v[1][2 * e] = two(oPN, x000, oPS, x010);
+    v[2][2 * e] = two(uPC, x000, dPC, x001);
+    v[1][2 * e + 1] =
+        add(add(two(oPNE, x000, oPNW, x100), oPSE, x010), oPSW, x110);
+    v[2][2 * e + 1] =
+        add(add(two(uPE, x000, uPW, x100), dPE, x001), dPW, x101);
+    v[3][2 * e] = add(add(two(uPN, x000, uPS, x010), dPN, x001), dPS, x011);
+    T s = add(add(two(uPNE, x000, uPNW, x100), uPSE, x010), uPSW, x110);
+    s = add(add(s, dPNE, x001), dPNW, x101);
+    v[3][2 * e + 1] = add(add(s, dPSE, x011), dPSW, x111);
   }
   if (!live) return;
 #pragma unroll
@@ -1811,7 +1816,8 @@ __device__ __forceinline__ void interp_body(int nxc, int nyc, int nzc,
     if (ADD && ((!(r & 1) && jj == 1) || (!(r & 2) && kk == 1))) continue;
     T o[4];
 #pragma unroll
-    for (int q = 0; q < 4; q++) o[q] = ADD ? old[r][q] + damp * v[r][q] : v[r][q];
+    for (int q = 0; q < 4; q++)
+      o[q] = ADD ? fma(damp, v[r][q], old[r][q]) : v[r][q];
     if (ADD && ii == 1) o[0] = old[r][0];
     T *g = xf + f0 + ((r & 1) ? fy : 0) + ((r & 2) ? fz : 0);
     if (both)
@@ -2185,7 +2191,7 @@ constexpr int CG_R = 3, CG_RNT = 512, CG_W = CG_RNT / 64;
 // Points per thread: 2 where four wavefronts hold the level that way (up to
 // 9^3: 100 us per 100 iterations against 107 with 3; its LDS reads, 18 per
 // point against 15, then fit beside the multiply-adds), else 3 (11^3: 126
-// against 152).
+// against 152).  The form of the mixed cycles takes 3 (see cg_rows_body).
 static int cg_threads(const Dim &d, int r) {
   const int segs = (d.nx - 2 + r - 1) / r * (d.ny - 2) * (d.nz - 2);
   return (segs + 63) / 64 * 64;
@@ -2236,19 +2242,30 @@ __device__ __forceinline__ double cg_rcp(double x) {
 // criterion (else Vcghs's relative one); ZT: errtol is 0, so Vcghs's test
 // sqrt(r.r)/sqrt(r0.r0) <= errtol is that x has settled (CG_SETTLED; no
 // square root or divide in the loop).  The PMG cycle uses <T, 0, 0, 1>
-// (errtol = epsiln = 0).
+// (errtol = epsiln = 0), with FP32 vectors <T, 0, 0, 0>.
 //
 // An iteration is a chain of latencies on one compute unit (three or four
 // wavefronts, no other work): LDS write of p, barrier, 42 LDS reads, 78
-// multiply-adds, a reduction over the workgroup, the quotients.  So it has
-// one reduction, of p.Ap, r.Ap, Ap.Ap and r.r together: r.r of the new
+// multiply-adds, a reduction over the workgroup, the quotients.  So the ZT
+// and ABS forms have one reduction, of p.Ap, r.Ap, Ap.Ap and r.r together: r.r of the new
 // residual is r.r - 2 a r.Ap + a^2 Ap.Ap, exact up to a rounding of the old
 // r.r, which each iteration sums anew from r itself, so nothing accumulates.
 // Beside it 1/(p.Ap) and 1/(r.r) run side by side without divisions, and p
 // stays in registers.  100 iterations with the damping factor (MI355X): 151
 // us on 11^3 and 126 on 9^3 with two reductions, three divisions and three
-// barriers per iteration; 126 and 100 so; to a relative 1e-2 on 9^3 in FP32
-// cycles 19 and 10.5.
+// barriers per iteration; 126 and 100 so.
+//
+// The remaining form, errtol > 0 in the mixed cycles (REL), keeps the
+// reference's recurrences with two reductions and true quotients, three
+// points per thread, every sum in one written-out order.  It stops at 1e-2
+// after 5 to 30 iterations on diagonals spanning 10 to 3000 (molecules at
+// 65^3 to 161^3), and where the span is in the hundreds its iterates grow
+// one rounding by 1e7 and more until then: with other sums the iteration
+// count changed in one of fifty solves, and a potential by up to 1.4e-9 of
+// its norm.  The result is within the solve's 1e-6 either way, but no caller
+// expects it to move.  With one reduction and two points per thread it took
+// 23.7 us a call on the 9^3 level of a 33^3 request and 11.7 on the 7^3 one
+// of 97^3; so 26.7 and 14.0 (the whole requests 2.6% and 0.9% longer).
 //
 // ZT works on the operator scaled to a unit diagonal where that diagonal
 // spans at most CG_SPAN, for one pass over the couplings before the loop:
@@ -2271,10 +2288,13 @@ __device__ __forceinline__ void cg_rows_body(
     int nx, int ny, int nz, const double *__restrict__ ac,
     const double *__restrict__ cc, const T *__restrict__ f,
     T *__restrict__ xout, int itmax, double errtol, double *damp) {
+  constexpr bool REL = !ABS && !ZT;
+  static_assert(!REL || (!WARM && R == CG_R), "the reference's iterates");
   double *P = cg_lds;
-  __shared__ double slots[CG_W][4];
+  __shared__ double slots[CG_W][4], rbuf[2][CG_W];
   const int tid = threadIdx.x, NTB = blockDim.x;
   if (tid < CG_W * 4) slots[tid >> 2][tid & 3] = 0.0;
+  if constexpr (REL) cg_zero_slots<CG_W>(rbuf);
   const size_t n = (size_t)nx * ny * nz;
   const long long sy = nx, sz = (long long)nx * ny;
   const int ni = nx - 2, nj = ny - 2, nk = nz - 2;
@@ -2416,8 +2436,16 @@ __device__ __forceinline__ void cg_rows_body(
   s4[0] = s4[1] = s4[2] = s4[3] = 0.0;
 #pragma unroll
   for (int r = 0; r < R; r++) s4[3] += rr[r] * rr[r];
-  cg_sum4(s4, slots, t4);
-  double rhok2 = t4[3];
+  double rhok2, rhok1 = 0.0;
+  if constexpr (REL) {  // the segment's middle point rounds first
+    double s = fma(rr[0], rr[0], rr[1] * rr[1]);
+#pragma unroll
+    for (int r = 2; r < R; r++) s = fma(rr[r], rr[r], s);
+    rhok2 = cg_allsum<CG_W>(s, rbuf[1]);
+  } else {
+    cg_sum4(s4, slots, t4);
+    rhok2 = t4[3];
+  }
   const double denom = sqrt(rhok2), settled = CG_SETTLED * rhok2;
   int iters = 0;
 #pragma unroll
@@ -2430,9 +2458,30 @@ __device__ __forceinline__ void cg_rows_body(
               : (ZT ? rhok2 <= settled : sqrt(rhok2) / denom <= errtol))
         break;
       if (iters >= itmax) break;
+      if (REL && iters > 0) {
+        const double beta = rhok2 / rhok1, ib = 1.0 / beta;
+#pragma unroll
+        for (int r = 0; r < R; r++) pp[r] = (pp[r] + ib * rr[r]) * beta;
+      }
       put(pp);  // every read of P lies before the last reduction's barrier
       __syncthreads();
       stencil();
+      iters++;
+      if constexpr (REL) {
+        double s = 0.0;
+#pragma unroll
+        for (int r = 0; r < R; r++) s = fma(pp[r], v[r], s);
+        const double alpha = rhok2 / cg_allsum<CG_W>(s, rbuf[0]);
+        rhok1 = rhok2;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+          xr[r] += alpha * pp[r];
+          rr[r] -= alpha * v[r];
+          s = r ? fma(rr[r], rr[r], s) : rr[r] * rr[r];
+        }
+        rhok2 = cg_allsum<CG_W>(s, rbuf[1]);
+        continue;
+      }
       s4[0] = s4[1] = s4[2] = s4[3] = 0.0;
 #pragma unroll
       for (int r = 0; r < R; r++) {
@@ -2452,7 +2501,6 @@ __device__ __forceinline__ void cg_rows_body(
         rr[r] -= alpha * v[r];
         pp[r] = rr[r] + beta * pp[r];
       }
-      iters++;
     }
   }
   for (size_t q = tid; q < n; q += NTB) {
@@ -2467,19 +2515,54 @@ __device__ __forceinline__ void cg_rows_body(
   // The Hackbusch-Reusken factor (x . f) / (x . A x) of the solution as
   // stored (mgcsd.cc:429-452; 0 when the denominator is 0): one more
   // application of the operator the threads hold, instead of a product
-  // kernel on a level of a few hundred points (4.8 us each).
+  // kernel on a level of a few hundred points (4.8 us each).  FP32 cycles
+  // take the product in FP32 with the FP32 operator and matvec27_body's sums,
+  // so the factor is the one of every other level's kind.
   if (damp) {
-#pragma unroll
-    for (int r = 0; r < R; r++)
-      pp[r] = ZT ? (double)(T)(sc[r] * xr[r]) / sc[r] : (double)(T)xr[r];
-    put(pp);
-    __syncthreads();
-    stencil();
     s4[0] = s4[1] = s4[2] = s4[3] = 0.0;
+    if constexpr (sizeof(T) == 4 && !ZT) {
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-      if (val[r]) s4[0] += pp[r] * ((ZT ? sc[r] : 1.0) * (double)f[pidx[r]]);
-      s4[1] += pp[r] * v[r];
+      for (int r = 0; r < R; r++) pp[r] = (double)(T)xr[r];
+      put(pp);
+      __syncthreads();
+      T w[9][R + 2];
+#pragma unroll
+      for (int a = 0; a < 9; a++)
+#pragma unroll
+        for (int c = 0; c < R + 2; c++) w[a][c] = (T)P[rb[a] + c];
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        auto co = [&](int q) { return (T)cf[r][q]; };
+        auto xv = [&](int q) {
+          return w[DJ[q] + 1 + 3 * (DK[q] + 1)][r + 1 + DI[q]];
+        };
+        // terms [q0, q1) in order
+        auto sum = [&](int q0, int q1) {
+          T s = fma(co(q0), xv(q0), co(q0 + 1) * xv(q0 + 1));
+#pragma unroll
+          for (int q = q0 + 2; q < q1; q++) s = fma(co(q), xv(q), s);
+          return s;
+        };
+        const T x = (T)xr[r];
+        const T dgt = val[r] ? (T)ac[pidx[r]] + (T)cc[pidx[r]] : (T)0;
+        const T y = fma(dgt, x, (-sum(0, 8) + -sum(8, 17)) + -sum(17, 26));
+        if (val[r]) {
+          s4[0] += (double)x * (double)f[pidx[r]];
+          s4[1] += (double)x * (double)y;
+        }
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; r++)
+        pp[r] = ZT ? (double)(T)(sc[r] * xr[r]) / sc[r] : (double)(T)xr[r];
+      put(pp);
+      __syncthreads();
+      stencil();
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        if (val[r]) s4[0] += pp[r] * ((ZT ? sc[r] : 1.0) * (double)f[pidx[r]]);
+        s4[1] += pp[r] * v[r];
+      }
     }
     cg_sum4(s4, slots, t4);
     if (tid == 0) *damp = t4[1] != 0.0 ? t4[0] / t4[1] : 0.0;
@@ -2501,19 +2584,23 @@ template <class T, bool WARM, bool ABS>
 static void cg_rows_launch(const Dim &d, const double *ac, const double *cc,
                            const T *f, T *x, int itmax, double errtol,
                            hipStream_t s, double *damp) {
-  const int r = cg_points(d), nt = cg_threads(d, r);
+  const bool rel = !ABS && errtol > 0.0;
+  const int r = rel ? CG_R : cg_points(d), nt = cg_threads(d, r);
   const size_t lds = (d.n() + CG_R + 2) * sizeof(double);
 #define ROWS(ZT, R, NT)                                                     \
   k_cg_rows<T, WARM, ABS, ZT, R, NT><<<1, nt, lds, s>>>(                    \
       d.nx, d.ny, d.nz, ac, cc, f, x, itmax, errtol, damp)
-  if (!ABS && errtol == 0.0) {
-    if (r == 2) ROWS(!ABS, 2, 256);
-    else if (nt <= 256) ROWS(!ABS, CG_R, 256);
-    else ROWS(!ABS, CG_R, CG_RNT);
-  } else {
+  if constexpr (ABS) {
     if (r == 2) ROWS(false, 2, 256);
     else if (nt <= 256) ROWS(false, CG_R, 256);
     else ROWS(false, CG_R, CG_RNT);
+  } else if (rel) {
+    if (nt <= 256) ROWS(false, CG_R, 256);
+    else ROWS(false, CG_R, CG_RNT);
+  } else {
+    if (r == 2) ROWS(true, 2, 256);
+    else if (nt <= 256) ROWS(true, CG_R, 256);
+    else ROWS(true, CG_R, CG_RNT);
   }
 #undef ROWS
 }
@@ -3783,7 +3870,8 @@ void g_cg(const GCoarse<T> *j, int n, int itmax, double errtol,
   // reductions sum in a fixed order (cg_sum4), whether those wavefronts
   // exist or not.
   g_split<A_cg<T>>(
-      (int)ok.size(), [&](int q) { return cg_points(j[ok[q]].d); },
+      (int)ok.size(),
+      [&](int q) { return errtol > 0.0 ? CG_R : cg_points(j[ok[q]].d); },
       [&](int q) {
         const GCoarse<T> &J = j[ok[q]];
         return A_cg<T>{J.d.nx, J.d.ny, J.d.nz, J.ac, J.cc, J.f, J.x, itmax,
@@ -3803,8 +3891,7 @@ void g_cg(const GCoarse<T> *j, int n, int itmax, double errtol,
           else if (nt <= 256) kb_cg_rows<T, true, CG_R, 256><<<g, nt, lds, s>>>(t);
           else kb_cg_rows<T, true, CG_R, CG_RNT><<<g, nt, lds, s>>>(t);
         } else {
-          if (r == 2) kb_cg_rows<T, false, 2, 256><<<g, nt, lds, s>>>(t);
-          else if (nt <= 256) kb_cg_rows<T, false, CG_R, 256><<<g, nt, lds, s>>>(t);
+          if (nt <= 256) kb_cg_rows<T, false, CG_R, 256><<<g, nt, lds, s>>>(t);
           else kb_cg_rows<T, false, CG_R, CG_RNT><<<g, nt, lds, s>>>(t);
         }
       });

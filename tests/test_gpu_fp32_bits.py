@@ -100,3 +100,160 @@ def test_sweep27(mg, dims, adj):
     want = x.copy()
     _sweep(ac, cc, f, want, adj)
     assert np.array_equal(got, want)
+
+
+def _wave_sum(v):
+    """Sums over wavefronts of 64 by shifts of 1, 2, 4 and 8 within rows of
+    16 lanes, then row 0 into 1 and 2 into 3, then lane 31 into the rest."""
+    v = v.reshape(-1, 64).copy()
+    lane = np.arange(64)
+    for s in (1, 2, 4, 8):
+        v += np.where(lane % 16 >= s, np.roll(v, s, axis=1), 0.0)
+    v[:, 16:32] += v[:, 15:16]
+    v[:, 48:64] += v[:, 47:48]
+    v[:, 32:64] += v[:, 31:32]
+    return v[:, 63]
+
+
+def _all_sum(v):
+    p = np.zeros(8)
+    w = _wave_sum(v)
+    p[:w.size] = w
+    for h in (1, 2, 4):
+        p[:8 - h:2 * h] += p[h::2 * h]
+    return p[0]
+
+
+def _coarse_cg(ac, cc, f, tol=1e-2, itmax=100):
+    """The coarsest CG of a mixed cycle, arrays indexed [k, j, i]: three
+    i-adjacent points per thread, the reference's recurrences (cgd.cc:60-124),
+    sums by thread, wavefront and workgroup.  Returns the FP32 solution and
+    the iterations."""
+    nz, ny, nx = f.shape
+    nseg = (nx - 2 + 2) // 3
+    t = np.arange(nseg * (ny - 2) * (nz - 2))
+    lanes = (t.size + 63) // 64 * 64
+    jj, kk = 1 + t // nseg % (ny - 2), 1 + t // (nseg * (ny - 2))
+    ii = [1 + t % nseg * 3 + r for r in range(3)]
+    val = [i <= nx - 2 for i in ii]
+    ii = [np.minimum(i, nx - 2) for i in ii]
+
+    def thread_sum(first, rest):
+        s = np.zeros(lanes)
+        s[:t.size] = first
+        for a, b in rest:
+            s[:t.size] = fma64(a, b, s[:t.size])
+        return _all_sum(s)
+
+    coef, dg = [], []
+    for r in range(3):
+        c = []
+        for (dx, dy, dz), pl, at in TERMS:
+            q = (kk + dz, jj + dy, ii[r] + dx) if at else (kk, jj, ii[r])
+            c.append(np.where(val[r], ac[(pl,) + q], 0.0))
+        coef.append(c)
+        dg.append(np.where(val[r], ac[0, kk, jj, ii[r]] + cc[kk, jj, ii[r]], 0.0))
+    x = [np.zeros(t.size) for _ in range(3)]
+    rr = [np.where(val[r], f[kk, jj, ii[r]].astype(np.float64), 0.0) for r in range(3)]
+    p = [v.copy() for v in rr]
+    P = np.zeros((nz, ny, nx))
+    # the middle point of a segment first, the first on top of it
+    rho = thread_sum(fma64(rr[0], rr[0], rr[1] * rr[1]), [(rr[2], rr[2])])
+    denom, old, its = np.sqrt(rho), 0.0, 0
+    while denom != 0.0 and np.sqrt(rho) / denom > tol and its < itmax:
+        if its:
+            beta = rho / old
+            p = [fma64(1.0 / beta, rr[r], p[r]) * beta for r in range(3)]
+        for r in range(3):
+            P[kk[val[r]], jj[val[r]], ii[r][val[r]]] = p[r][val[r]]
+        ap = []
+        for r in range(3):
+            part = {}
+            for dz in (0, 1, -1):
+                s = np.zeros(t.size)
+                for row in (-1, 0, 1):  # row by row, in the terms' order
+                    for (dx, dy, ez), c in zip((o for o, _, _ in TERMS), coef[r]):
+                        if ez == dz and dy == row:
+                            s = fma64(c, P[kk + dz, jj + dy, ii[r] + dx], s)
+                part[dz] = s
+            v = fma64(dg[r], p[r], (-part[0] + -part[1]) + -part[-1])
+            ap.append(np.where(val[r], v, 0.0))
+        its += 1
+        alpha = rho / thread_sum(0.0, [(p[r], ap[r]) for r in range(3)])
+        x = [fma64(alpha, p[r], x[r]) for r in range(3)]
+        rr = [fma64(-alpha, ap[r], rr[r]) for r in range(3)]
+        old = rho
+        rho = thread_sum(rr[0] * rr[0], [(rr[1], rr[1]), (rr[2], rr[2])])
+    out = np.zeros((nz, ny, nx), F32)
+    for r in range(3):
+        out[kk[val[r]], jj[val[r]], ii[r][val[r]]] = x[r][val[r]]
+    return out, its
+
+
+def _cycle(mg, ctx, dims, nlev, fc, nu=2):
+    """The correction of one mixed cycle for the right-hand side fc, level by
+    level through the single-kernel entry points."""
+    lev = []
+    for q in range(nlev):
+        ac, cc, _, pc = ctx.level(q + 1)
+        lev.append((dims, ac, cc, pc))
+        dims = tuple((d - 1) // 2 + 1 for d in dims)
+    f32 = [np.ascontiguousarray(a, F32) for a in [fc]] + [None] * (nlev - 1)
+    x = [None] * nlev
+    for q, (d, ac, cc, pc) in enumerate(lev):
+        nd, N = (7 if q == 0 else 27), d[0] * d[1] * d[2]
+        if q == nlev - 1:
+            g = d[::-1]
+            x[q], its = _coarse_cg(ac.reshape((14,) + g), cc.reshape(g), f32[q].reshape(g))
+            x[q] = np.ascontiguousarray(x[q].ravel())
+            break
+        a, c = ac.astype(F32), cc.astype(F32)
+        x[q] = np.zeros(N, F32)
+        _call(mg, "pmg_gsrb_f32", *d, nd, fp(a), fp(c), fp(f32[q]), fp(x[q]), nu, 0, 1)
+        r = np.zeros(N, F32)
+        _call(mg, "pmg_mresid_f32", *d, nd, fp(a), fp(c), fp(f32[q]), fp(x[q]), fp(r))
+        dc = lev[q + 1][0]
+        f32[q + 1] = np.zeros(dc[0] * dc[1] * dc[2], F32)
+        _call(mg, "pmg_restrc_f32", *d, *dc, fp(r), fp(f32[q + 1]), fp(pc.astype(F32)))
+    for q in range(nlev - 2, -1, -1):
+        d, ac, cc, pc = lev[q]
+        dc, acc, ccc, _ = lev[q + 1]
+        _call(mg, "pmg_correct_f32", *dc, *d, 27, fp(acc.astype(F32)), fp(ccc.astype(F32)),
+              fp(x[q + 1]), fp(f32[q + 1]), fp(pc.astype(F32)), fp(x[q]))
+        _call(mg, "pmg_gsrb_f32", *d, 7 if q == 0 else 27, fp(ac.astype(F32)),
+              fp(cc.astype(F32)), fp(f32[q]), fp(x[q]), nu, 1, 0)
+    return x[0], its
+
+
+# Levels above the coarsest in the bottom kernels (9 x 13 x 11; 5^3 over one
+# unknown; 17^3) and beyond them (17 x 25 x 21); coarsest levels up to 13^3,
+# whose workgroups have 192 to 512 threads.  Damping factors are quotients of
+# FP64 sums rounded to FP32: their order, not restated here, shows once in
+# 1e8.
+@pytest.mark.parametrize("dims,nlev", [((17, 25, 21), 3), ((17, 17, 17), 4), ((33, 33, 33), 3),
+                                       ((33, 49, 41), 3), ((21, 21, 21), 2), ((25, 25, 25), 2)])
+def test_mixed_cycle(mg, dims, nlev):
+    print(f"mixed cycle bits dims={dims} nlev={nlev}", flush=True)
+    nx, ny, nz = dims
+    N = nx * ny * nz
+    rng = np.random.default_rng(sum(dims) + nlev)
+    inp = {k: np.arange(n) * 0.5 for k, n in zip(("xf", "yf", "zf"), dims)}
+    for k, n in (("gxcf", ny * nz), ("gycf", nx * nz), ("gzcf", nx * ny)):
+        inp[k] = np.zeros(4 * n)
+    k, j, i = np.meshgrid(*(np.linspace(-1, 1, n) for n in (nz, ny, nx)), indexing="ij")
+    eps = np.where(i * i + j * j + k * k < 0.5, 0.05, 78.54).ravel()
+    for a in ("a1cf", "a2cf", "a3cf"):
+        inp[a] = eps * rng.uniform(0.9, 1.0, N)
+    inp["ccf"] = np.where(eps < 1.0, 0.0, 0.8)
+    inp["fcf"] = rng.standard_normal(N)
+    inp["tcf"] = np.zeros(N)
+    sz = mg.Vmgsz(2, 0, 0, *dims, nlev)
+    iparm, rparm = mg.Vpackmg(sz["iretot"], sz["iintot"], *dims, nlev, itmax=1)
+    ctx = mg.Context(iparm, rparm, inp)
+    ctx.solve(mg.PMG_MIXED)
+    inner = np.s_[1:-1, 1:-1, 1:-1]
+    got = ctx.u().reshape(nz, ny, nx)[inner]
+    want, its = _cycle(mg, ctx, dims, nlev, ctx.level(1)[2])
+    print("coarsest iterations", its, flush=True)
+    assert np.array_equal(got, want.astype(np.float64).reshape(nz, ny, nx)[inner])
+    ctx.close()
