@@ -185,17 +185,18 @@ __global__ __launch_bounds__(256) void k_pb_nodes(
   fcf[p] = acc;
 }
 
-// exp(-kappa r) by Tang's table-driven method (P. T. P. Tang,
+// exp(x) for -708 <= x <= 0 by Tang's table-driven method (P. T. P. Tang,
 // "Table-driven implementation of the exponential function in IEEE
-// floating-point arithmetic", ACM TOMS 15(2):144-157, 1989) in units of
-// ln2/64: c r = 64 m + j + R with c = -64 kappa / ln2 and |R| <= 1/2,
-// exp = 2^m 2^(j/64) 2^(R/64), 2^(R/64) - 1 by its Taylor polynomial of
-// degree 5 (truncation error below 3.5e-17), 2^(j/64) as lead + trail
-// (tables in LDS).  c comes as two doubles and enters only fused
-// multiply-adds, so R carries the rounding of r alone; adding 1.5 2^52 leaves 64 m + j in the sum's low word, for
-// |c r| < 2^31 (face_terms bounds r).
-// ln2 / 64 as the nearest double and the nearest to the remainder
-constexpr double LN2_64 = 0x1.62e42fefa39efp-7, LN2_64_LO = 0x1.abc9e3b39803fp-62;
+// floating-point arithmetic", ACM TOMS 15(2):144-157, 1989):
+// x = (64 m + j) ln2/64 + R with |R| <= ln2/128, exp(x) = 2^m 2^(j/64) e^R,
+// e^R - 1 by its Taylor polynomial of degree 5 (truncation error below
+// 3.5e-17), ln2/64 split as L1 + L2 with N L1 exact, 2^(j/64) as lead +
+// trail (tables in LDS).  Within one ulp of exp (checked against the C
+// library on 2e6 arguments in [-60, 0], as with degree 6); about half the
+// instructions of the general routine.
+constexpr double EXP_INV_L = 0x1.71547652b82fep+6;  // 64 / ln2
+constexpr double EXP_L1 = 0x1.62e42fef00000p-7;      // ln2/64, low 20 bits zero
+constexpr double EXP_L2 = 0x1.473de6af278edp-40;      // ln2/64 - L1
 // 2^(j/64), j = 0..63: the double nearest to it (lead) and the double
 // nearest to the remainder (trail), computed from the definition
 __constant__ double c_exp2_lead[64] = {
@@ -248,22 +249,21 @@ __constant__ double c_exp2_trail[64] = {
 };
 
 // lead, trail: 2^(j/64) as lead + trail; sum: lead + trail, added once.
-__device__ __forceinline__ double exp_tab(double c, double cl, double r,
-                                          const double *lead,
+__device__ __forceinline__ double exp_tab(double x, const double *lead,
                                           const double *trail,
                                           const double *sum) {
-  constexpr double MAGIC = 0x1.8p52, L = LN2_64;
-  const double s = fma(c, r, MAGIC);
-  const int n = __double2loint(s);
-  const double R = fma(cl, r, fma(c, r, -(s - MAGIC)));
-  // degree-5 Taylor polynomial: on |R| <= 1/2 the next term is below
+  const double N = rint(x * EXP_INV_L);
+  const int n = (int)N;
+  const double R = fma(-N, EXP_L2, fma(-N, EXP_L1, x));
+  // degree-5 Taylor polynomial: on |R| <= ln2/128 the next term is below
   // 3.5e-17 relative
-  double q = fma(R, L * L * L * L * L / 120.0, L * L * L * L / 24.0);
-  q = fma(R, q, L * L * L / 6.0);
-  q = fma(R, q, L * L / 2.0);
-  const double p = R * fma(R, q, L);  // 2^(R/64) - 1
+  double q = fma(R, 1.0 / 120.0, 1.0 / 24.0);
+  q = fma(R, q, 1.0 / 6.0);
+  q = fma(R, q, 0.5);
+  const double p = fma(R * R, q, R);  // e^R - 1
   const int j = n & 63, m = n >> 6;   // n = 64 m + j, 0 <= j < 64
-  return ldexp(lead[j] + fma(sum[j], p, trail[j]), m);
+  const double sl = lead[j], st = trail[j];
+  return ldexp(sl + fma(sum[j], p, st), m);
 }
 
 // 1/sqrt(x) for a positive, finite x: the hardware estimate y0 with one
@@ -280,27 +280,30 @@ __device__ __forceinline__ double rsqrt_pos(double x) {
 constexpr int FACE_NT = 256, FACE_NODES = 64, FACE_SPLIT = FACE_NT / FACE_NODES;
 
 // Atoms [t0, t1) of the staged chunk for the node pair at in-plane
-// coordinates (va, vb): su/sw hold the atoms' in-plane coordinates, s0n/s1n
-// the squares of their distances to the low and the high face, which no
-// node has to form again, and the in-plane part of a squared distance
-// serves both nodes: three FP64 instructions per term for the distance
-// instead of six.  cap keeps |c r| below 2^31 where exp is 0 long since.
+// coordinates (va, vb) of axis AX: su/sw hold the atoms' in-plane
+// coordinates, s0n/s1n the squares of their distances to the low and the
+// high face, which no node has to form again.  The squared distance is summed
+// in x, y, z order, as the serial restatement does.
+template <int AX>
 __device__ __forceinline__ void face_terms(int t0, int t1, double va, double vb,
-                                           double c, double cl, double cap,
-                                           const double *su, const double *sw,
+                                           double kap, const double *su,
+                                           const double *sw,
                                            const double *s0n,
                                            const double *s1n,
-                                           const double *sc,
-                                           const double *tl, const double *tt,
-                                           const double *ts, double &s0,
-                                           double &s1) {
+                                           const double *sc, const double *tl,
+                                           const double *tt, const double *ts,
+                                           double &s0, double &s1) {
+#pragma clang fp contract(off)
   for (int t = t0; t < t1; t++) {
     const double du = va - su[t], dw = vb - sw[t];
-    const double e = fmin(fma(du, du, dw * dw), cap);
-    const double r0 = e + s0n[t], r1 = e + s1n[t];
+    const double d0s = s0n[t], d1s = s1n[t], dus = du * du, dws = dw * dw;
+    const double r0 = AX == 0 ? d0s + dus + dws
+                              : (AX == 1 ? dus + d0s + dws : dus + dws + d0s);
+    const double r1 = AX == 0 ? d1s + dus + dws
+                              : (AX == 1 ? dus + d1s + dws : dus + dws + d1s);
     const double i0 = rsqrt_pos(r0), i1 = rsqrt_pos(r1);
-    s0 = fma(sc[t] * exp_tab(c, cl, r0 * i0, tl, tt, ts), i0, s0);
-    s1 = fma(sc[t] * exp_tab(c, cl, r1 * i1, tl, tt, ts), i1, s1);
+    s0 = fma(sc[t] * exp_tab(-kap * (r0 * i0), tl, tt, ts), i0, s0);
+    s1 = fma(sc[t] * exp_tab(-kap * (r1 * i1), tl, tt, ts), i1, s1);
   }
 }
 
@@ -312,12 +315,14 @@ __device__ __forceinline__ void face_terms(int t0, int t1, double va, double vb,
 // and the four partial sums are added in a fixed order.  Per term the atom
 // factor lambda_B q exp(kappa r) / (eps_w (1 + kappa r)) is staged once,
 // leaving one exp (exp_tab) and one reciprocal square root per (node,
-// atom); atoms without a charge are left out.  Bound by instruction issue,
-// FP64 ones above all: 23 per term against 29 with the distance formed per
-// node and the exponent reduced in three steps.  289^3 with 5000 atoms, a
-// fifth of them uncharged, 3.38 -> 2.42 ms (MI355X); the error against 64
-// bits is the same, 1e-16 to 3e-16 of the sum of magnitudes.  The sum is
-// deterministic; its order differs from the serial one by rounding only.
+// atom); atoms whose term is 0 at every node, those without a charge, are
+// left out of their quarter, which changes no sum.  Bound by instruction
+// issue, FP64 ones above all: 289^3 with 5000 atoms, a fifth of them
+// uncharged, 3.38 -> 2.54 ms with the normal distances squared once and those
+// atoms left out (MI355X).  The sum is deterministic; its order differs
+// from the serial one by rounding only.  Its bits are kept by intent: a
+// mixed solve rounds the right-hand side the faces enter to FP32, and its
+// coarsest CG can grow one changed rounding to 1e-9 of the potential.
 __global__ __launch_bounds__(FACE_NT) void k_pb_faces(
     int n, double c0, double h, double lb, double kap, double eps_out,
     int natoms,
@@ -325,7 +330,7 @@ __global__ __launch_bounds__(FACE_NT) void k_pb_faces(
 #pragma clang fp contract(off)
   __shared__ double su[FACE_NT], sw[FACE_NT], s0n[FACE_NT], s1n[FACE_NT],
       sc[FACE_NT];
-  __shared__ int kept[FACE_SPLIT];
+  __shared__ unsigned long long kept[FACE_SPLIT];
   __shared__ double part[2][FACE_SPLIT][FACE_NODES];
   // exp_tab's tables (read after a barrier)
   __shared__ double tl[64], tt[64], ts[64];
@@ -342,41 +347,55 @@ __global__ __launch_bounds__(FACE_NT) void k_pb_faces(
   const int a = valid ? (int)(idx % n) : 0, b = valid ? (int)(idx / n) : 0;
   const double lo = c0, hi = c0 + (n - 1) * h;
   const double va = c0 + a * h, vb = c0 + b * h;
-  const double c = -kap / LN2_64;
-  const double cl = fma(-c, LN2_64_LO, fma(-c, LN2_64, -kap)) / LN2_64;
-  // half the square of the r at which c r is -2^30 (kappa r = 1.1e7)
-  const double rmax = 0x1p30 / -c, cap = kap > 0.0 ? 0.5 * rmax * rmax : 1e300;
   const int in0 = axis == 0 ? 1 : 0, in1 = axis == 2 ? 1 : 2;
-  double s0 = 0.0, s1 = 0.0;
-  for (int base = 0; base < natoms; base += FACE_NT) {
-    __syncthreads();
-    // the chunk's atoms that carry a charge, in order (of a molecule with
-    // charges of -1 to 1 in halves a fifth does not)
-    const int g = base + (int)threadIdx.x;
-    const double *A = atoms + 5 * (size_t)min(g, natoms - 1);
-    const double q = A[4];
-    const unsigned long long ball = __ballot(g < natoms && q != 0.0);
-    if (lane == 0) kept[split] = __popcll(ball);
-    __syncthreads();
-    int at = __popcll(ball & ((1ull << lane) - 1ull)), m = 0;
+  // kept atoms of the chunk before its atom i (0 to FACE_NT)
+  auto rank = [&](int i) {
+    int c = 0;
 #pragma unroll
     for (int v = 0; v < FACE_SPLIT; v++) {
-      if (v < split) at += kept[v];
-      m += kept[v];
+      const int w = min(max(i - 64 * v, 0), 64);
+      c += __popcll(w < 64 ? kept[v] & ((1ull << w) - 1ull) : kept[v]);
     }
+    return c;
+  };
+  double s0 = 0.0, s1 = 0.0;
+  for (int base = 0; base < natoms; base += FACE_NT) {
+    const int m = min(FACE_NT, natoms - base);
+    __syncthreads();
+    const int tid = threadIdx.x;
+    const double *A = atoms + 5 * (size_t)(base + min(tid, m - 1));
+    const double c =
+        lb * A[4] / (eps_out * (1.0 + kap * A[3])) * exp(kap * A[3]);
+    // a coordinate that is no finite number stays, and shows in the sums
+    const bool finite =
+        (A[0] - A[0]) + (A[1] - A[1]) + (A[2] - A[2]) == 0.0;
+    const unsigned long long ball =
+        __ballot(tid < m && !(c == 0.0 && finite));
+    if (lane == 0) kept[split] = ball;
+    __syncthreads();
     if ((ball >> lane) & 1ull) {
+      const int at = rank(tid);
       su[at] = A[in0];
       sw[at] = A[in1];
       const double d0 = lo - A[axis], d1 = hi - A[axis];
-      s0n[at] = fmin(d0 * d0, cap);
-      s1n[at] = fmin(d1 * d1, cap);
-      sc[at] = lb * q / (eps_out * (1.0 + kap * A[3])) * exp(kap * A[3]);
+      s0n[at] = d0 * d0;
+      s1n[at] = d1 * d1;
+      sc[at] = c;
     }
-    __syncthreads();
+    // the quarter by the atoms' places in the chunk
     const int per = (m + FACE_SPLIT - 1) / FACE_SPLIT;
-    const int t0 = min(m, split * per), t1 = min(m, t0 + per);
-    face_terms(t0, t1, va, vb, c, cl, cap, su, sw, s0n, s1n, sc, tl, tt, ts, s0,
-               s1);
+    const int t0 = rank(min(m, split * per)),
+              t1 = rank(min(m, split * per + per));
+    __syncthreads();
+    if (axis == 0)
+      face_terms<0>(t0, t1, va, vb, kap, su, sw, s0n, s1n, sc, tl, tt, ts, s0,
+                    s1);
+    else if (axis == 1)
+      face_terms<1>(t0, t1, va, vb, kap, su, sw, s0n, s1n, sc, tl, tt, ts, s0,
+                    s1);
+    else
+      face_terms<2>(t0, t1, va, vb, kap, su, sw, s0n, s1n, sc, tl, tt, ts, s0,
+                    s1);
   }
   part[0][split][lane] = s0;
   part[1][split][lane] = s1;

@@ -33,3 +33,43 @@ def test_faces_staging(mg, orc, natoms, zeros):
     got = mg.pbe_assemble(n, h, 0.15, at)
     for k in ("gxcf", "gycf", "gzcf"):
         assert np.max(np.abs(got[k] - want[k])) <= 1e-13 * np.max(np.abs(want[k])), k
+
+
+FACES = ("gxcf", "gycf", "gzcf")
+
+
+def _atoms(natoms, seed):
+    rng = np.random.default_rng(seed)
+    return np.column_stack([rng.uniform(-8, 8, (natoms, 3)), rng.uniform(1.2, 2.0, natoms),
+                            rng.choice([-1.0, 0.5, 1.0], natoms)])
+
+
+@pytest.mark.parametrize("field", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("charge", [1.0, 0.0])
+def test_faces_nan(mg, orc, field, charge):
+    """A record that is no number shows in every boundary value, as in the
+    oracle, whether or not the atom carries a charge."""
+    print(f"faces nan field={field} charge={charge}", flush=True)
+    at = _atoms(300, field)
+    at[270, 4] = charge
+    at[270, field] = np.nan
+    want = orc.pbe_assemble(17, 1.5, 0.15, at)
+    got = mg.pbe_assemble(17, 1.5, 0.15, at)
+    for k in FACES:
+        assert np.array_equal(np.isnan(got[k]), np.isnan(want[k])), k
+        assert np.isnan(got[k]).any(), k
+
+
+@pytest.mark.parametrize("natoms", [3, 255, 256, 257, 511])
+def test_faces_uncharged(mg, natoms):
+    """Uncharged atoms change no bit of the sums: as charges too small to
+    show they give the same faces."""
+    print(f"faces uncharged natoms={natoms}", flush=True)
+    at = _atoms(natoms, natoms)
+    none = np.random.default_rng(1).random(natoms) < 0.4
+    got = []
+    for q in (0.0, 1e-290):
+        at[none, 4] = q
+        got.append(mg.pbe_assemble(17, 1.5, 0.15, at))
+    for k in FACES:
+        assert np.array_equal(got[0][k], got[1][k]), k
