@@ -207,6 +207,10 @@ int ses_cycle_done(pmg_ctx *c);
 // once for all of them; context q's stopping scalar also goes to norm[q]
 // (device memory).  Bit-identical to each context's own iteration.
 bool group_ok(const pmg_ctx *c);
+// Orders stream s behind everything c's own stream holds (the start of its
+// session, whose scalars lin_poll may have seen before that work is done):
+// once, before the first group_step that c takes part in.
+void group_join(pmg_ctx *c, hipStream_t s);
 void group_step(pmg_ctx *const *c, int n, int mode, hipStream_t s,
                 double *norm);
 

@@ -219,6 +219,7 @@ void group_launch(Group &g, std::deque<Request *> &ready) {
     }
     g.mode = r->mode;
     g.mem.push_back(r);
+    group_join(r->ctx, g.s);
     ready.pop_front();
   }
   if (g.mem.empty()) return;

@@ -973,6 +973,14 @@ bool group_ok(const pmg_ctx *c) {
   return c->p.istop <= 1 && c->nlev >= 2 && !c->ktime;
 }
 
+void group_join(pmg_ctx *c, hipStream_t s) {
+  if (hipEventRecord(c->cyc_ev, c->s) != hipSuccess ||
+      hipStreamWaitEvent(s, c->cyc_ev, 0) != hipSuccess) {
+    hipGetLastError();
+    hipStreamSynchronize(c->s);
+  }
+}
+
 // smooth() of level lev for the contexts qs (x = L[lev].x, f[k] its
 // right-hand side).
 template <class T>
@@ -1199,6 +1207,8 @@ int ctx_solve_group(pmg_ctx *const *cs, int n, int mode) {
       hipMalloc((void **)&dn, sizeof(double) * (n + 1)) != hipSuccess ||
       hipHostMalloc((void **)&hn, sizeof(double) * (n + 1)) != hipSuccess)
     rc = PMG_EDEVICE;
+  if (!rc)
+    for (pmg_ctx *c : act) group_join(c, gs);
   while (!rc && !act.empty()) {
     group_step(act.data(), (int)act.size(), mode, gs, dn);
     hipMemcpyAsync(hn, dn, sizeof(double) * act.size(), hipMemcpyDeviceToHost,
