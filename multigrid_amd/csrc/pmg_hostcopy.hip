@@ -117,10 +117,15 @@ int copy_plain(hipStream_t s, const HostSeg *seg, int n) {
 
 int copy_pieces(hipStream_t s, const std::vector<HostSeg> &pc, Ring &r, int nt,
                 bool two) {
-  int dev = 0;
+  // events, threads and the second stream are those of the stream's device,
+  // whatever the caller's current one is
+  int cur = 0;
+  hipDevice_t dev = 0;
   char *const ring = r.p;
   hipEvent_t ev[kSlots] = {}, start = nullptr;
-  std::atomic<bool> ok{hipGetDevice(&dev) == hipSuccess};
+  std::atomic<bool> ok{hipGetDevice(&cur) == hipSuccess &&
+                       hipStreamGetDevice(s, &dev) == hipSuccess &&
+                       (cur == dev || hipSetDevice(dev) == hipSuccess)};
   const int np = (int)pc.size(), ns = 2 * nt;
   // the second stream starts behind what s holds already
   hipStream_t st[2] = {s, s};
@@ -167,6 +172,7 @@ int copy_pieces(hipStream_t s, const std::vector<HostSeg> &pc, Ring &r, int nt,
   for (hipEvent_t e : ev)
     if (e) hipEventDestroy(e);
   if (start) hipEventDestroy(start);
+  if (cur != dev && hipSetDevice(cur) != hipSuccess) ok = false;
   return ok ? PMG_OK : PMG_EDEVICE;
 }
 

@@ -128,3 +128,12 @@ def test_served_group_starts_behind_its_members(host, mg, mode):
         assert s.wait(t) == OK
     assert host.fk_unordered() == 0
     host.pmg_server_destroy(s.h)
+
+
+@pytest.mark.parametrize("bytes_", [4096, (4 << 20) + 24, (33 << 20) + 8])
+@pytest.mark.parametrize("on,cur", [(0, 0), (1, 1), (0, 1), (1, 0)])
+def test_copy_from_another_device(host, bytes_, on, cur):
+    """A copy takes the device of its stream; the calling thread's current
+    device need not be that one, and stays."""
+    host.fk_reset(2)
+    assert host.fk_copy(bytes_, on, cur) == OK
