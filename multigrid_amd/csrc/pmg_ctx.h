@@ -99,6 +99,7 @@ struct pmg_ctx {
   double *band = nullptr, *band_rt = nullptr, *band_ct = nullptr;
   double *scal = nullptr;    // device scalars
   double *hscal = nullptr;   // pinned host mirror
+  bool lost = false;  // a scalar of this solve never reached it
   bool have32 = false, haveN = false;
   bool ops32_ok = false;  // FP32 operator copies match the FP64 hierarchy
   int iters = 0, ierror = 0;
@@ -111,6 +112,7 @@ struct pmg_ctx {
     // what the pending work is waited for by: the event, the host mirror of
     // the denominator, that of the norm
     bool by_event = false, wait_den = false, wait_nrm = false;
+    unsigned polls = 0;  // lin_poll calls that found nothing
     double rsden = 1.0, rsnrm = 0.0;
   } ses;
   hipEvent_t cyc_ev = nullptr, t0_ev = nullptr, t1_ev = nullptr;

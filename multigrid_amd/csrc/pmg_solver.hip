@@ -14,6 +14,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <limits>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -134,18 +135,22 @@ bool host_landed(const pmg_ctx *c, int slot) {
                          __ATOMIC_ACQUIRE) != kAwait;
 }
 // The slot's value once it has landed.  The spin is bounded: a long
-// iteration (or a device error) is waited for through the stream.
+// iteration is waited for through the stream.  A device error or a launch
+// that failed leaves the slot as it was armed: then c->lost is set, for the
+// caller to end with PMG_EDEVICE, and the value is NaN, which ends every
+// loop that tests it.
 double host_scalar(pmg_ctx *c, int slot) {
   using clock = std::chrono::steady_clock;
   const auto limit = clock::now() + std::chrono::milliseconds(2);
-  for (int q = 0; !host_landed(c, slot); q++) {
+  for (int q = 0; !c->lost && !host_landed(c, slot); q++) {
     __builtin_ia32_pause();
     if ((q & 63) == 63 && clock::now() > limit) {
-      hipStreamSynchronize(c->s);
+      if (hipStreamSynchronize(c->s) != hipSuccess || !host_landed(c, slot))
+        c->lost = true;
       break;
     }
   }
-  return c->hscal[slot];
+  return c->lost ? std::numeric_limits<double>::quiet_NaN() : c->hscal[slot];
 }
 Red red_host(pmg_ctx *c, int slot) {
   Red r = red_to(c, slot);
@@ -349,7 +354,7 @@ int linear_fp64(pmg_ctx *c, LV<double> *L, const double *frhs,
     rsnrm = host_scalar(c, S_RSNRM);
     *iters_out = 1;
     *rel_out = rsnrm / rsden;
-    return PMG_OK;
+    return c->lost ? PMG_EDEVICE : PMG_OK;
   }
   int iters = 0;
   do {
@@ -362,6 +367,7 @@ int linear_fp64(pmg_ctx *c, LV<double> *L, const double *frhs,
   } while (iters < itmax && rsnrm / rsden > errtol);
   *iters_out = iters;
   *rel_out = rsnrm / rsden;
+  if (c->lost) return PMG_EDEVICE;
   return iters < itmax ? PMG_OK : PMG_ITMAX;
 }
 
@@ -406,6 +412,7 @@ int linear_mixed(pmg_ctx *c, LV<double> *L64, LV<float> *L32,
   } while (iters < itmax && rsnrm / rsden > errtol);
   *iters_out = iters;
   *rel_out = rsnrm / rsden;
+  if (c->lost) return PMG_EDEVICE;
   return (iters < itmax || rsnrm / rsden <= errtol) ? PMG_OK : PMG_ITMAX;
 }
 
@@ -803,6 +810,7 @@ int lin_begin(pmg_ctx *c, int mode) {
   S.mode = mode;
   S.done = false;
   S.phase = 0;
+  c->lost = false;
   c->nev = 0;
   c->hist.clear();
   hipEventRecord(c->t0_ev, c->s);
@@ -840,17 +848,52 @@ int lin_begin(pmg_ctx *c, int mode) {
   return PMG_OK;
 }
 
+// A scalar of the session will never land: it ends with PMG_EDEVICE.
+void ses_failed(pmg_ctx *c) {
+  auto &S = c->ses;
+  c->lost = true;
+  S.pending = false;
+  S.done = true;
+  S.rc = PMG_EDEVICE;
+}
+
 void lin_enqueue(pmg_ctx *c) {
   auto &S = c->ses;
   if (S.done || S.pending || S.phase != 1) return;
   S.by_event = S.wait_den = false;
   S.wait_nrm = true;
   host_arm(c, S_RSNRM);
-  if (c->gexec[S.mode] && !c->ktime)
-    hipGraphLaunch(c->gexec[S.mode], c->s);
-  else
+  if (!c->gexec[S.mode] || c->ktime)
     step_body(c, S.mode);
+  else if (hipGraphLaunch(c->gexec[S.mode], c->s) != hipSuccess)
+    return ses_failed(c);
   S.pending = true;
+}
+
+// What the session waits for: 1 landed, 0 not yet, -1 never will.
+int lin_landed(pmg_ctx *c, bool wait) {
+  auto &S = c->ses;
+  if (wait) {
+    if (S.by_event && hipEventSynchronize(c->cyc_ev) != hipSuccess) return -1;
+    if (S.wait_den) host_scalar(c, S_RSDEN);
+    if (S.wait_nrm) host_scalar(c, S_RSNRM);
+    return c->lost ? -1 : 1;
+  }
+  if (S.by_event) {
+    const hipError_t e = hipEventQuery(c->cyc_ev);
+    if (e != hipSuccess) return e == hipErrorNotReady ? 0 : -1;
+  }
+  auto here = [&] {
+    return (!S.wait_den || host_landed(c, S_RSDEN)) &&
+           (!S.wait_nrm || host_landed(c, S_RSNRM));
+  };
+  if (here()) return 1;
+  // a slot says nothing of a launch that failed; the stream, once it is idle,
+  // does (asked every 256th time: a server polls each session in turn)
+  if (++S.polls % 256) return 0;
+  const hipError_t e = hipStreamQuery(c->s);
+  if (e == hipErrorNotReady) return 0;
+  return e == hipSuccess && here() ? 1 : -1;
 }
 
 // Returns 1 when the session has finished (after this poll), 0 otherwise.
@@ -859,14 +902,11 @@ int lin_poll(pmg_ctx *c, bool wait) {
   const Params &p = c->p;
   if (S.done) return 1;
   if (!S.pending) return 0;
-  if (wait) {
-    if (S.by_event) hipEventSynchronize(c->cyc_ev);
-    if (S.wait_den) host_scalar(c, S_RSDEN);
-    if (S.wait_nrm) host_scalar(c, S_RSNRM);
-  } else if ((S.by_event && hipEventQuery(c->cyc_ev) != hipSuccess) ||
-             (S.wait_den && !host_landed(c, S_RSDEN)) ||
-             (S.wait_nrm && !host_landed(c, S_RSNRM))) {
-    return 0;
+  const int landed = lin_landed(c, wait);
+  if (!landed) return 0;
+  if (landed < 0) {
+    ses_failed(c);
+    return 1;
   }
   S.pending = false;
   if (S.phase == 0) {  // the start has landed
@@ -953,7 +993,8 @@ int lin_end(pmg_ctx *c) {
       c->ktime_ms += kms;
     }
   }
-  if (se != hipSuccess || hipGetLastError() != hipSuccess) return PMG_EDEVICE;
+  if (se != hipSuccess || hipGetLastError() != hipSuccess || c->lost)
+    return PMG_EDEVICE;
   c->iters = S.iters;
   c->relres = S.rsnrm / S.rsden;
   c->ierror = S.rc == PMG_ITMAX ? 1 : 0;
@@ -1407,6 +1448,7 @@ int newton_level(pmg_ctx *c, int mode, int l0, double *x, int itmax,
       xold = xnew;
     }
     rsnrm = xnew;
+    if (c->lost) break;
     if (l0 == 0) {
       c->hist.push_back(rsnrm / rsden);
       if (p.iinfo > 0)  // Vprtstp (mgsubd.cc:486-536)
@@ -1418,6 +1460,7 @@ int newton_level(pmg_ctx *c, int mode, int l0, double *x, int itmax,
   }
   *iters_out = iters;
   *rel_out = rsnrm / rsden;
+  if (c->lost) return PMG_EDEVICE;
   return *rel_out <= p.errtol ? PMG_OK : PMG_ITMAX;
 }
 
@@ -1458,12 +1501,13 @@ int ctx_newton(pmg_ctx *c, int mode) {
   else
     fill<double>(c->u, d.n(), 0.0, s);
   c->u_given = false;
+  c->lost = false;
   int iters = 0;
   double rel = 0.0;
   if (p.mgkey == 1) {
     for (int l = 1; l < c->nlev; l++)
       fill<double>(c->L[l].xn, c->L[l].d.n(), 0.0, s);
-    for (int l = c->nlev - 1; l >= 1; l--) {
+    for (int l = c->nlev - 1; l >= 1 && !c->lost; l--) {
       newton_level(c, mode, l, c->L[l].xn, 1000, &iters, &rel);
       interp<double>(c->L[l].d, c->L[l - 1].d, c->L[l].xn, c->L[l].pc,
                      l - 1 == 0 ? c->u : c->L[l - 1].xn, nullptr, s);
@@ -1478,7 +1522,7 @@ int ctx_newton(pmg_ctx *c, int mode) {
   c->solve_ms = ms;
   hipEventDestroy(e0);
   hipEventDestroy(e1);
-  if (se != hipSuccess) return PMG_EDEVICE;
+  if (se != hipSuccess || c->lost) return PMG_EDEVICE;
   c->iters = iters;
   c->relres = rel;
   c->ierror = rc == PMG_OK ? 0 : 1;
@@ -1581,6 +1625,7 @@ int ctx_pcg(pmg_ctx *c, int mode, int num_iters) {
   hipEventCreate(&e0);
   hipEventCreate(&e1);
   hipEventRecord(e0, s);
+  c->lost = false;
   // x0 = 0; the coarsest solution, which the class CG starts from, too
   fill<double>(c->u, nf, 0.0, s);
   if (mode == PMG_MIXED)
@@ -1601,7 +1646,7 @@ int ctx_pcg(pmg_ctx *c, int mode, int num_iters) {
   double rel = nf1 / rsden;
   int iters = 0, ierr = 0;
   if (pap0 != 0.0) {  // CG_Solver.h:124-125
-    for (;;) {
+    while (!c->lost) {
       // x and r are those of iteration `iters`; the next direction (a cycle
       // and a product) is made only once it is known to be wanted
       if (num_iters > 0) {
@@ -1646,7 +1691,8 @@ int ctx_pcg(pmg_ctx *c, int mode, int num_iters) {
   c->solve_ms = ms;
   hipEventDestroy(e0);
   hipEventDestroy(e1);
-  if (se != hipSuccess || hipGetLastError() != hipSuccess) return PMG_EDEVICE;
+  if (se != hipSuccess || hipGetLastError() != hipSuccess || c->lost)
+    return PMG_EDEVICE;
   c->iters = iters;
   c->relres = rsnrm / rsden;
   c->ierror = ierr;

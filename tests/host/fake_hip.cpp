@@ -258,7 +258,7 @@ void resid<double, float>(const Dim &, int, const double *, const double *,
 void nmresid(const Dim &, int, const double *, const double *, const double *,
              const double *, double *, const Red *red, hipStream_t s) {
   tick(s);
-  put(red, 1.0);
+  put(red, fk.value);
 }
 void matvec7_dot(const Dim &, const double *, const double *, const double *,
                  const double *, double *, const Red &red, hipStream_t s) {

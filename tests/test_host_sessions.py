@@ -137,3 +137,48 @@ def test_copy_from_another_device(host, bytes_, on, cur):
     device need not be that one, and stays."""
     host.fk_reset(2)
     assert host.fk_copy(bytes_, on, cur) == OK
+
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("kind,kw", [("solve", {}), ("pcg", {}), ("newton", dict(nonlin=1)),
+                                     ("newton", dict(nonlin=1, mgkey=1))])
+@pytest.mark.parametrize("fault", ["none", "no store", "sync", "launch"])
+def test_scalar_that_never_lands(host, mg, mode, kind, kw, fault):
+    """A stopping scalar that never reaches the host (a failed launch, a lost
+    device) ends a solve with PMG_EDEVICE, not with a NaN that passes for
+    convergence; and the same context solves again afterwards."""
+    host.fk_reset(1)
+    c = Ctx(host, mg, **kw)
+    graphs = kind == "solve" and fault == "launch"
+    host.pmg_ctx_set_graphs(c.h, int(graphs))
+
+    def run():
+        return host.pmg_ctx_pcg(c.h, mode, 0) if kind == "pcg" else host.pmg_ctx_solve(c.h, mode)
+
+    if fault == "no store":
+        host.fk_set(0, 0.0, 0.0, 0, 0)
+    elif fault == "sync":
+        host.fk_set(0, 0.0, 0.0, 0, LOST)
+    elif fault == "launch":
+        host.fk_set(1 if graphs else 0, 0.0, 0.0, LOST, 0)
+    rc = run()
+    host.fk_set(1, 0.0, 0.0, 0, 0)
+    host.pmg_ctx_set_graphs(c.h, 0)
+    assert rc == (OK if fault == "none" else EDEVICE)
+    assert graphs or run() == OK
+    c.close()
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("fault", [(0, 0, 0), (0, LOST, 0), (0, 0, LOST)])
+def test_served_scalar_that_never_lands(host, mg, mode, fault):
+    """A served request whose scalar never lands is answered with
+    PMG_EDEVICE; its worker does not poll for ever."""
+    host.fk_reset(1)
+    s = Server(host, mg)
+    host.fk_set(fault[0], 0.0, 0.0, fault[1], fault[2])
+    t = [s.submit(mode) for _ in range(3)]
+    assert [s.wait(q, 10000) for q in t] == [EDEVICE] * 3
+    host.fk_set(1, 0.0, 0.0, 0, 0)
+    host.pmg_server_destroy(s.h)
