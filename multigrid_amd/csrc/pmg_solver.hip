@@ -935,12 +935,38 @@ int lin_poll(pmg_ctx *c, bool wait) {
   return ses_cycle_done(c);
 }
 
+// Whether the residual of u = 0 is NaN (c->L[0].x is free in a linear solve).
+// A mixed solve starts from f, which is that residual only if the operator
+// holds finite numbers: with an inf or NaN in it no cycle is wanted, and the
+// solve ends at the iterate 0.  Asked after a first cycle that gave NaN, so
+// that no other solve pays for it.
+bool operator_nan(pmg_ctx *c) {
+  Level &F = c->L[0];
+  fill<double>(F.x, F.d.n(), 0.0, c->s);
+  const Red rd = red_host(c, S_TMP);
+  resid<double, double>(F.d, F.numdia, F.ac, F.cc, F.fc, F.x,
+                        (double *)nullptr, &rd, c->s, F.dg);
+  return std::isnan(host_scalar(c, S_TMP));
+}
+
 // An iteration of the session has landed, its stopping scalar in
 // c->hscal[S_RSNRM]: count it, record and report it, decide whether the
 // session goes on (mgcsd.cc:483-527).  Returns 1 when it has finished.
 int ses_cycle_done(pmg_ctx *c) {
   auto &S = c->ses;
   const Params &p = c->p;
+  if (S.iters == 0 && S.mode == PMG_MIXED && p.istop <= 1 &&
+      std::isnan(c->hscal[S_RSNRM]) && operator_nan(c)) {
+    if (c->lost) {
+      ses_failed(c);
+      return 1;
+    }
+    fill<double>(c->u, c->L[0].d.n(), 0.0, c->s);
+    S.rsnrm = c->hscal[S_RSNRM];
+    S.rc = PMG_OK;
+    S.done = true;
+    return 1;
+  }
   S.iters++;
   const double orsnrm = S.rsnrm;
   S.rsnrm = p.istop >= 3 ? std::sqrt(c->hscal[S_RSNRM]) : c->hscal[S_RSNRM];

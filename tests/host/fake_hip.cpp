@@ -242,18 +242,20 @@ void fill<double>(double *x, size_t n, double v, hipStream_t s) {
   for (size_t q = 0; q < n; q++) x[q] = v;
 }
 template <>
-void resid<double, double>(const Dim &, int, const double *, const double *,
-                           const double *, const double *, double *,
+void resid<double, double>(const Dim &d, int, const double *, const double *,
+                           const double *, const double *x, double *r,
                            const Red *red, hipStream_t s, const double *) {
   tick(s);
-  put(red, fk.value);
+  bool zero = !r;
+  for (size_t q = 0; q < d.n(); q++) zero &= x[q] == 0.0;
+  put(red, zero ? fk.zero_value : fk.value);
 }
 template <>
 void resid<double, float>(const Dim &, int, const double *, const double *,
-                          const double *, const double *, float *r,
+                          const double *, const double *, float *,
                           const Red *red, hipStream_t s, const double *) {
   tick(s);
-  put(red, r ? fk.value : fk.zero_value);
+  put(red, fk.value);
 }
 void nmresid(const Dim &, int, const double *, const double *, const double *,
              const double *, double *, const Red *red, hipStream_t s) {

@@ -182,3 +182,23 @@ def test_served_scalar_that_never_lands(host, mg, mode, fault):
     assert [s.wait(q, 10000) for q in t] == [EDEVICE] * 3
     host.fk_set(1, 0.0, 0.0, 0, 0)
     host.pmg_server_destroy(s.h)
+
+
+@pytest.mark.parametrize("group", [False, True])
+@pytest.mark.parametrize("zero,iters", [(np.nan, 0), (1.0, 1)])
+def test_mixed_first_residual_nan(host, mg, group, zero, iters):
+    """A mixed solve whose first cycle gives NaN took no cycle if the
+    residual of u = 0 is NaN already (an inf or NaN in the operator), and one
+    if the cycle itself overflowed."""
+    host.fk_reset(1)
+    c = Ctx(host, mg)
+    host.pmg_ctx_set_graphs(c.h, 0)
+    host.fk_set(1, np.nan, zero, 0, 0)
+    h = (ctypes.c_void_p * 1)(c.h)
+    assert (host.pmg_ctx_solve_group(h, 1, 1) if group else host.pmg_ctx_solve(c.h, 1)) == OK
+    it, rel = ctypes.c_int(), ctypes.c_double()
+    host.pmg_ctx_stats(c.h, ctypes.byref(it), None, ctypes.byref(rel), None, None)
+    host.pmg_ctx_history.argtypes = [ctypes.c_void_p, _D, ctypes.c_int]
+    assert it.value == iters and np.isnan(rel.value)
+    assert host.pmg_ctx_history(c.h, None, 0) == iters
+    c.close()
