@@ -2060,7 +2060,11 @@ __device__ inline void cg_load_row(const double *__restrict__ ac, size_t n,
 // coarsest levels of the benchmark workloads (condition 6 to 20), 45 with
 // the unit diagonal of k_cg_rows.  A level that converges too slowly for
 // this (a condition beyond about 100) takes all 100 as before.
+// An r0.r0 that overflows settles nothing: the iterations show it as NaN.
 constexpr double CG_SETTLED = 1e-40;
+__device__ __forceinline__ double cg_settled(double rho0) {
+  return rho0 < HUGE_VAL ? CG_SETTLED * rho0 : -1.0;
+}
 
 template <class T, int NPT, int ND>
 __global__ __launch_bounds__(CG_NT) void k_cg_single(
@@ -2108,7 +2112,7 @@ __global__ __launch_bounds__(CG_NT) void k_cg_single(
   double rhok2 = cg_allsum<CG_NT / 64>(s, rbuf[0]);
   int b = 1;
   const double denom = sqrt(rhok2);
-  const double settled = CG_SETTLED * rhok2;
+  const double settled = cg_settled(rhok2);
   int iters = 0;
   double rhok1 = 0.0;
   if (denom != 0.0) {
@@ -2451,7 +2455,7 @@ __device__ __forceinline__ void cg_rows_body(
     cg_sum4(s4, slots, t4);
     rhok2 = t4[3];
   }
-  const double denom = sqrt(rhok2), settled = CG_SETTLED * rhok2;
+  const double denom = sqrt(rhok2), settled = cg_settled(rhok2);
   int iters = 0;
 #pragma unroll
   for (int r = 0; r < R; r++) pp[r] = rr[r];

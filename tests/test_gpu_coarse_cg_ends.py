@@ -42,3 +42,18 @@ def test_almost_an_eigenvector(mg, orc, dims):
     for e in np.geomspace(3e-8, 3e-10, 24):
         got, want = _cycle(mg, orc, dims, f + e * odd)
         assert np.max(np.abs(got - want)) <= 1e-10 * np.max(np.abs(want)), e
+
+
+# coarse levels of 3^3 and 5^3 unknowns
+@pytest.mark.parametrize("dims", [(9, 9, 9), (13, 13, 13)])
+@pytest.mark.parametrize("scale", [1e120, 1e200])
+def test_overflow(mg, orc, dims, scale):
+    """A right-hand side whose square overflows shows as it does in the
+    oracle; one whose square does not is solved."""
+    print(f"coarse cg overflow dims={dims} scale={scale}", flush=True)
+    nx, ny, nz = dims
+    f = np.random.default_rng(3).standard_normal((nz, ny, nx)) * scale
+    got, want = _cycle(mg, orc, dims, f)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    ok = ~np.isnan(want)
+    assert np.max(np.abs(got - want)[ok]) <= 1e-10 * np.max(np.abs(want[ok]))
