@@ -101,11 +101,10 @@ void nmresid(const Dim &d, int numdia, const double *ac, const double *cc,
              const double *fc, const double *x, double *r, const Red *red,
              hipStream_t s);
 
-// ---- y = A x; with red, red->out[0] = (x.w0) / (x.y), the Hackbusch-
-// Reusken damping of the coarse correction (pmgc/mgcsd.cc:429-452) ----
+// ---- y = A x (pmgc/matvecd.cc:61-261) ----
 template <class T>
-void matvec_dots(const Dim &d, int numdia, const T *ac, const T *cc,
-                 const T *x, const T *w0, T *y, const Red *red, hipStream_t s);
+void matvec(const Dim &d, int numdia, const T *ac, const T *cc, const T *x,
+            T *y, hipStream_t s);
 
 // y = A x and the per-block partials of (x.w0, x.y) into part (2 per
 // block), for interp_damped; returns the number of blocks.
@@ -175,12 +174,13 @@ void cg_class(const Dim &d, int numdia, const double *ac, const double *cc,
 // red.out[0] = x.y over the interior (deterministic order)
 void dot_interior(const Dim &d, const double *x, const double *y,
                   const Red &red, hipStream_t s);
-// x += (rs/pap) p, r -= (rs/pap) q; p = s + (rsn/rs) p (interior; device
-// scalars, a zero denominator gives a zero coefficient)
 // y = A x of the fine level and x . y; dg: oC + cc when precomputed.
 void matvec7_dot(const Dim &d, const double *ac, const double *cc,
                  const double *dg, const double *x, double *y, const Red &red,
                  hipStream_t s);
+// x += (rs/pap) p, r -= (rs/pap) q; p = s + (rsn/rs) p (interior; device
+// scalars, a zero denominator gives a zero coefficient); red: the L1 norm of
+// the new r
 void pcg_xr(const Dim &d, double *x, double *r, const double *p,
             const double *q, const double *rs, const double *pap,
             const Red *red, hipStream_t s);

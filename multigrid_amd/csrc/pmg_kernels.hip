@@ -100,25 +100,18 @@ __device__ inline void red_store(const Red &r, double v0, double v1) {
                    v0, v1);
 }
 
-// out[0] = sum0 (MODE 0), sum0 / sum1 (MODE 1; 0 when sum1 == 0, a zero
-// coarse correction) or sum1 (MODE 2).  Fixed order: thread t sums blocks
-// t, t+1024, ...
-template <int NV, int MODE>
+// out[0] = the sum of the blocks' last values (NV per block).  Fixed order:
+// thread t sums blocks t, t+1024, ...
+template <int NV>
 __device__ __forceinline__ void red_final_body(const double *part,
                                                unsigned nblk, double *out,
                                                double *host) {
   __shared__ double lds[16];
-  double a = 0.0, c = 0.0;
-  for (unsigned q = threadIdx.x; q < nblk; q += 1024) {
-    a += part[(size_t)q * NV];
-    if (NV == 2) c += part[(size_t)q * NV + 1];
-  }
-  const double sa = block_sum<1024>(a, lds);
-  const double sc = NV == 2 ? block_sum<1024>(c, lds) : 0.0;
+  double a = 0.0;
+  for (unsigned q = threadIdx.x; q < nblk; q += 1024)
+    a += part[(size_t)q * NV + NV - 1];
+  const double v = block_sum<1024>(a, lds);
   if (threadIdx.x == 0) {
-    const double v = MODE == 1   ? (sc != 0.0 ? sa / sc : 0.0)
-                     : MODE == 2 ? sc
-                                 : sa;
     out[0] = v;
     // the host waits for this one store, not for the kernel: nothing else
     // it reads depends on it, so no fence
@@ -126,17 +119,16 @@ __device__ __forceinline__ void red_final_body(const double *part,
       __hip_atomic_store(host, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
-template <int NV, int MODE>
+template <int NV>
 __global__ __launch_bounds__(1024) void k_red_final(const double *part,
                                                     unsigned nblk, double *out,
                                                     double *host) {
-  red_final_body<NV, MODE>(part, nblk, out, host);
+  red_final_body<NV>(part, nblk, out, host);
 }
 
-template <int NV, int MODE>
+template <int NV>
 static void red_final(const Red &r, const dim3 &g, hipStream_t s) {
-  k_red_final<NV, MODE><<<1, 1024, 0, s>>>(r.part, g.x * g.y * g.z, r.out,
-                                          r.host);
+  k_red_final<NV><<<1, 1024, 0, s>>>(r.part, g.x * g.y * g.z, r.out, r.host);
 }
 
 // ---------------------------------------------------------------------------
@@ -1232,7 +1224,7 @@ void resid(const Dim &d, int numdia, const T *ac, const T *cc, const T *fc,
       k_resid7m<T, TO, false, false><<<nb, dim3(RM_TX, RM_TY), 0, s>>>(
           d.nx, d.ny, d.nz, ac, cc, fc, x, r, dg, rdm, red ? 1 : 0, kcm, gx,
           gy, gz);
-    if (red) red_final<1, 0>(rdm, dim3(nb), s);
+    if (red) red_final<1>(rdm, dim3(nb), s);
     check_launch("resid");
     return;
   }
@@ -1242,7 +1234,7 @@ void resid(const Dim &d, int numdia, const T *ac, const T *cc, const T *fc,
     const P27 sh = p27_shape(d);
     k_resid27<T, TO><<<sh.nblk, dim3(BX, sh.rows), 0, s>>>(d.nx, d.ny, d.nz, ac, cc, fc, x, r,
                                            rd, red ? 1 : 0, sh);
-    if (red) red_final<1, 0>(rd, dim3(sh.nblk), s);
+    if (red) red_final<1>(rd, dim3(sh.nblk), s);
     check_launch("resid");
     return;
   }
@@ -1254,7 +1246,7 @@ void resid(const Dim &d, int numdia, const T *ac, const T *cc, const T *fc,
   else
     k_resid<T, TO, false><<<xcd_blocks(g), b, 0, s>>>(
         d.nx, d.ny, d.nz, ac, cc, fc, x, r, dg, rd, red ? 1 : 0, kc, xg_of(g));
-  if (red) red_final<1, 0>(rd, dim3(xcd_blocks(g)), s);
+  if (red) red_final<1>(rd, dim3(xcd_blocks(g)), s);
   check_launch("resid");
 }
 
@@ -1370,7 +1362,7 @@ void nmresid(const Dim &d, int numdia, const double *ac, const double *cc,
   else
     k_nmresid<27><<<xcd_blocks(g), dim3(BX, BY), 0, s>>>(
         d.nx, d.ny, d.nz, ac, cc, fc, x, r, rd, red ? 1 : 0, xg_of(g));
-  if (red) red_final<1, 0>(rd, dim3(xcd_blocks(g)), s);
+  if (red) red_final<1>(rd, dim3(xcd_blocks(g)), s);
   check_launch("nmresid");
 }
 
@@ -1500,11 +1492,9 @@ static unsigned matvec_launch(const Dim &d, int numdia, const T *ac,
 }
 
 template <class T>
-void matvec_dots(const Dim &d, int numdia, const T *ac, const T *cc,
-                 const T *x, const T *w0, T *y, const Red *red,
-                 hipStream_t s) {
-  const unsigned nb = matvec_launch<T>(d, numdia, ac, cc, x, w0, y, red, s);
-  if (red) red_final<2, 1>(*red, dim3(nb), s);
+void matvec(const Dim &d, int numdia, const T *ac, const T *cc, const T *x,
+            T *y, hipStream_t s) {
+  matvec_launch<T>(d, numdia, ac, cc, x, nullptr, y, nullptr, s);
 }
 
 // y = A x of a 7-point level with x . y: the march where it serves the
@@ -1518,11 +1508,11 @@ void matvec7_dot(const Dim &d, const double *ac, const double *cc,
     k_resid7m<double, double, true><<<nb, dim3(RM_TX, RM_TY), 0, s>>>(
         d.nx, d.ny, d.nz, ac, nullptr, nullptr, x, y, dg, red, 1, kc, gx, gy,
         gz);
-    red_final<1, 0>(red, dim3(nb), s);
+    red_final<1>(red, dim3(nb), s);
   } else {
     const unsigned nb =
         matvec_launch<double>(d, 7, ac, cc, x, nullptr, y, &red, s);
-    red_final<2, 2>(red, dim3(nb), s);
+    red_final<2>(red, dim3(nb), s);
   }
   check_launch("matvec7_dot");
 }
@@ -1896,7 +1886,7 @@ template <class T>
 void nrm1(const Dim &d, const T *x, const Red &red, hipStream_t s) {
   dim3 g(cdiv(d.nx - 2, BX), cdiv(d.ny - 2, BY), cdiv(d.nz - 2, KCH));
   k_nrm1<T><<<g, dim3(BX, BY), 0, s>>>(d.nx, d.ny, d.nz, x, red);
-  red_final<1, 0>(red, g, s);
+  red_final<1>(red, g, s);
   check_launch("nrm1");
 }
 
@@ -1942,10 +1932,10 @@ void stop_diff(const Dim &d, int kind, double *tru, const double *u,
   dim3 b(BX, BY);
   if (kind == 2) {
     k_stopdiff<2><<<g, b, 0, s>>>(d.nx, d.ny, d.nz, tru, u, w, red);
-    red_final<1, 0>(red, g, s);
+    red_final<1>(red, g, s);
   } else if (kind == 3) {
     k_stopdiff<3><<<g, b, 0, s>>>(d.nx, d.ny, d.nz, tru, u, w, red);
-    red_final<1, 0>(red, g, s);
+    red_final<1>(red, g, s);
   } else {
     k_stopdiff<5><<<g, b, 0, s>>>(d.nx, d.ny, d.nz, tru, u, w, red);
   }
@@ -1956,7 +1946,7 @@ template <class T>
 void dot_energy(const Dim &d, int numdia, const T *ac, const T *cc,
                 const T *w, T *y, const Red &red, hipStream_t s) {
   const unsigned nb = matvec_launch<T>(d, numdia, ac, cc, w, w, y, &red, s);
-  red_final<2, 2>(red, dim3(nb), s);
+  red_final<2>(red, dim3(nb), s);
 }
 
 // Vextrac (matvecd.cc:997-1008): coarse interior by injection.
@@ -2717,7 +2707,7 @@ void start_mixed(const Dim &d, const double *f, float *r, double *u,
   const dim3 g(cdiv(d.nx * d.ny, ST_PTS), d.nz);
   k_start_mixed<<<g, 256, 0, s>>>(d.nx, d.ny, d.nz, f, r, u,
                                   red ? *red : Red{}, red ? 1 : 0);
-  if (red) red_final<1, 0>(*red, g, s);
+  if (red) red_final<1>(*red, g, s);
   check_launch("start_mixed");
 }
 
@@ -2750,7 +2740,7 @@ void dot_interior(const Dim &d, const double *x, const double *y,
                   const Red &red, hipStream_t s) {
   dim3 g(cdiv(d.nx - 2, BX), cdiv(d.ny - 2, BY), cdiv(d.nz - 2, KCH));
   k_dot<<<g, dim3(BX, BY), 0, s>>>(d.nx, d.ny, d.nz, x, y, red);
-  red_final<1, 0>(red, g, s);
+  red_final<1>(red, g, s);
   check_launch("dot_interior");
 }
 
@@ -2806,7 +2796,7 @@ void pcg_xr(const Dim &d, double *x, double *r, const double *p,
   dim3 g(cdiv(d.nx - 2, BX), cdiv(d.ny - 2, BY), cdiv(d.nz - 2, KCH));
   k_pcg_xr<<<g, dim3(BX, BY), 0, s>>>(d.nx, d.ny, d.nz, x, r, p, q, rs, pap,
                                       red ? *red : Red{}, red ? 1 : 0);
-  if (red) red_final<1, 0>(*red, g, s);
+  if (red) red_final<1>(*red, g, s);
   check_launch("pcg_xr");
 }
 
@@ -3638,10 +3628,10 @@ struct A_rf {
   unsigned nblk;
   double *out, *out2;
 };
-template <int NV, int MODE>
+template <int NV>
 __global__ __launch_bounds__(1024) void kb_red_final(const GTab<A_rf> t) {
   const A_rf &a = t.a[blockIdx.y];
-  red_final_body<NV, MODE>(a.part, a.nblk, a.out, nullptr);
+  red_final_body<NV>(a.part, a.nblk, a.out, nullptr);
   if (threadIdx.x == 0 && a.out2) a.out2[0] = a.out[0];
 }
 
@@ -3707,7 +3697,7 @@ void g_resid(const GResid<T, TO> *j, int n, hipStream_t s) {
         return A_rf{j[r].red->part, a[r].nblk, j[r].red->out, j[r].out2};
       },
       [&](const GTab<A_rf> &t, int m, int) {
-        kb_red_final<1, 0><<<dim3(1, m), 1024, 0, s>>>(t);
+        kb_red_final<1><<<dim3(1, m), 1024, 0, s>>>(t);
       });
   check_launch("g_resid");
 }
@@ -3969,9 +3959,8 @@ template void dot_energy<double>(const Dim &, int, const double *,
   template void diag_sum<T>(const T *, const T *, T *, size_t, hipStream_t);  \
   template void gs27<T>(const Dim &, const T *, const T *, const T *, T *,    \
                         int, int, hipStream_t, bool, T *);                    \
-  template void matvec_dots<T>(const Dim &, int, const T *, const T *,        \
-                               const T *, const T *, T *, const Red *,        \
-                               hipStream_t);                                  \
+  template void matvec<T>(const Dim &, int, const T *, const T *, const T *,   \
+                          T *, hipStream_t);                                  \
   template void restrict_<T>(const Dim &, const Dim &, const T *, T *,        \
                              const T *, hipStream_t, float *);                \
   template void interp<T>(const Dim &, const Dim &, const T *, const T *,     \

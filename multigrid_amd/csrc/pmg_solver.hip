@@ -754,8 +754,7 @@ void build_alg(pmg_ctx *c) {
       extrac(c->L[l - 1].d, L.d, t, L.r, c->s);
       t = L.r;
     }
-    matvec_dots<double>(L.d, L.numdia, L.ac, L.cc, t, nullptr, L.fc, nullptr,
-                        c->s);
+    matvec<double>(L.d, L.numdia, L.ac, L.cc, t, L.fc, c->s);
   }
 }
 
@@ -2051,7 +2050,7 @@ int interp_t(int nxc, int nyc, int nzc, int nxf, int nyf, int nzf,
 
 // xf(interior) += xdamp * (P xc), xdamp = (xc . w0c) / (xc . A_c xc): the
 // coarse-grid correction of the V-cycle's way up (mgcsd.cc:429-458), as
-// the cycle runs it: k_matvec_dots partials, then k_interp<T, true>.
+// the cycle runs it: the product's partials, then k_interp<T, true>.
 template <class T>
 int correct_t(int nxc, int nyc, int nzc, int nxf, int nyf, int nzf,
               int numdia, const T *acc, const T *ccc, const T *xc,
@@ -2327,7 +2326,7 @@ int pmg_matvec(int nx, int ny, int nz, int numdia, const double *ac,
   double *dac = S.put(ac, (numdia == 7 ? 4 : 14) * n), *dcc = S.put(cc, n),
          *dx = S.put(x, n), *dy = S.put(y, n);
   if (!S.ok) return PMG_ENOMEM;
-  matvec_dots<double>(d, numdia, dac, dcc, dx, nullptr, dy, nullptr, 0);
+  matvec<double>(d, numdia, dac, dcc, dx, dy, 0);
   return finish(S, y, dy, n);
 }
 
