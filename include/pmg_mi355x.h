@@ -64,7 +64,13 @@ int pmg_Vpackmg(int *iparm, double *rparm, size_t *nrwk, int *niwk, int *nx,
 int pmg_maxlev(int nx, int ny, int nz);
 
 /* Replaces pmgc::Vmgdriv (pmgc/mgdrvd.h:79-98, mgdrvd.cc:60-65): the linear
- * PMG solve, same pointer list minus the sycl::queue.  FP64 throughout.
+ * PMG solve, same pointer list minus the sycl::queue.  FP64 throughout;
+ * the coarsest CG, for which the reference takes 100 iterations, ends once
+ * its solution has settled, and where the coarse diagonal spans at most 96
+ * it runs on the operator scaled to a unit diagonal: the same solution to
+ * the last digits wherever 100 plain iterations settle, a more exact one
+ * where they do not (spans of 39 to 96 with a low-dielectric region of
+ * several coarse cells: the reference's is 1e-12 to 1e-7 short there).
  * On return u holds the solution with Dirichlet boundary values restored
  * (mgdrvd.cc:500-502); iwork holds iz/ipc and rwork holds rpc/cc/fc/pc/ac
  * as the reference leaves them (mgdrvd.cc:145-166).  Unlike the reference,
@@ -155,7 +161,8 @@ int pmg_ctx_create(pmg_ctx **out, const int *iparm, const double *rparm,
                    const double *a1cf, const double *a2cf, const double *a3cf,
                    const double *ccf, const double *fcf);
 /* Solve on the resident hierarchy (mode PMG_FP64 or PMG_MIXED).  The
- * solution stays in HBM until pmg_ctx_get_u. */
+ * solution stays in HBM until pmg_ctx_get_u.  The calling thread spins for
+ * up to 2 ms on each iteration's stopping scalar before it blocks. */
 int pmg_ctx_solve(pmg_ctx *ctx, int mode);
 /* Solve n (<= 64) distinct contexts together: their V-cycle iterations run
  * in lockstep with every kernel launched once for all of them (the
@@ -169,7 +176,11 @@ int pmg_ctx_solve_group(pmg_ctx *const *ctx, int n, int mode);
  * the V-cycle preconditioner in FP32 under the FP64 CG.  Statistics as
  * pmg_ctx_solve (iterations are CG iterations). */
 int pmg_ctx_pcg(pmg_ctx *ctx, int mode, int num_iters);
-/* Copy the solution (with Dirichlet boundary values) to host u (nx*ny*nz). */
+/* Copy the solution (with Dirichlet boundary values) to host u (nx*ny*nz).
+ * From 4 MB on to pageable memory the copy uses up to eight threads (this
+ * one and seven that live for the call) and a pinned ring of 32 MB, at most
+ * two of them, given back with the last context; the calling thread's
+ * current device may be any. */
 int pmg_ctx_get_u(pmg_ctx *ctx, double *u);
 /* Stats of the last solve on ctx: iterations, ierror, relative residual,
  * device milliseconds of setup and of the solve. */

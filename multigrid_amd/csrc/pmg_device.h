@@ -141,8 +141,9 @@ __device__ __forceinline__ const T *lane_at(const T *base, int di,
 // FP32 56 -> 44 us, 81^3 FP32 11.2 -> 8.4, FP64 16.5 -> 12.2, 33^3 and 17^3
 // FP64 8.2 -> 5.8 us; the same sums in the same order).  The four-element
 // loads of the last pair of the grid's last row reach one element past the
-// end of x, whose value no sum uses: every x array has that element
-// (allocations are padded).
+// end of x, whose value no sum uses; interp_body's reach two past the end of
+// xc, and its pair loads one past the end of pc.  Every array these kernels
+// are given has room for that (allocations are padded).
 template <class T>
 struct G27C {          // couplings, the right-hand side, the diagonal's parts
   T cN[2], cS[2];      // oN(p), oN(p - sy)

@@ -217,9 +217,10 @@ bool smooth(pmg_ctx *c, const LV<T> &l, const T *f, T *x, int nu, int iadj,
   return added;
 }
 
-// Coarsest-level solve: Vcghs with 100 iterations and errtol = epsiln = 0
-// (mgsolv 0; epsiln 0 gives exactly 100 iterations), or the factored band (mgsolv 1, mgcsd.cc:391-407, which
-// ignores cc as the reference's band does).  FP64 inside either way.
+// Coarsest-level solve: Vcghs with errtol = epsiln = 0 (mgsolv 0; the
+// reference then takes 100 iterations, here they end once the solution has
+// settled), or the factored band (mgsolv 1, mgcsd.cc:391-407, which ignores
+// cc as the reference's band does).  FP64 inside either way.
 // errtol > 0: Vcghs's relative stopping test sqrt(r.r)/sqrt(r0.r0) <= errtol
 // with that tolerance instead of epsiln (at most 100 iterations).
 // damp (may be null): the device scalar for the Hackbusch-Reusken factor of
@@ -676,8 +677,8 @@ int ctx_create_pbe(pmg_ctx **out, const Params &p, double h, double ionic,
 // One step enqueues one iteration of Vmvcs's loop (mgcsd.cc:299-527): the
 // V-cycle and the FP64 L1 stopping norm (for PMG_MIXED: the FP32 V-cycle on
 // the FP64 residual, the FP64 update, the new FP64 residual and its norm),
-// then an 8-byte copy of the norm to pinned host memory and an event.  The
-// host decides whether to continue when the event has completed.  The step
+// which its reduction stores to pinned host memory.  The host decides
+// whether to continue when that store has landed.  The step
 // body is captured once per mode as a HIP graph and replayed.
 
 void views(pmg_ctx *c, LV<double> *L64, LV<float> *L32, int mode) {
